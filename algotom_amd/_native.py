@@ -50,6 +50,9 @@ SIGNATURES = (
                              _I, _P]),
     ("ath_back_projection", _I, [_P, _I, _I, _I, _I, _P, _F, _I, _I, _D, _I,
                                  _P, _P]),
+    ("ath_back_projection_matrix_workspace_bytes", _S, [_I, _I, _I, _I]),
+    ("ath_back_projection_matrix", _I, [_P, _I, _I, _I, _I, _P, _F, _I, _I,
+                                        _D, _I, _P, _P, _S, _P]),
     ("ath_back_projection_with_derivative", _I, [_P, _I, _I, _I, _P, _F,
                                                  _I, _D, _I, _P, _P, _P]),
     ("ath_back_projection_tiled", _I, [_P, _I, _I, _I, _I, _P, _F, _I, _I,

@@ -103,12 +103,23 @@ struct BpArgs {
     int mask_c;            // ncol // 2
     int apply_scale;
     float pi32, denom;     // float32(pi), float32(nrow - 1)
+    // null, or one word per slice: only slices whose word exceeds `above`
+    // are computed and written
+    const unsigned* only_above;
+    unsigned above;
 };
 
 // sb / py <= 0 select the default tile configuration
 int back_projection(const BpArgs& a, int sino_dtype, int acc, int sb, int py,
                     hipStream_t stream);
 int back_projection_naive(const BpArgs& a, int acc, hipStream_t stream);
+// stacks on the matrix cores (bp_matrix.hip); acc: the vector kernel's
+// accumulation for slices it has to redo
+constexpr int kMaxMatrixCols = 32768;
+size_t back_projection_matrix_workspace(int dtype, int nrow, int nslice,
+                                        int ncol);
+int back_projection_matrix(const BpArgs& a, int dtype, int acc, void* work,
+                           hipStream_t stream);
 
 // ---- forward projection = adjoint of the back-projection ------------------
 // largest FFT length of the 1D ramp filter and of its adjoint

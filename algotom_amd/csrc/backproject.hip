@@ -685,6 +685,8 @@ __device__ __forceinline__ void bp_tile(
 #pragma unroll
             for (int js = 0; js < SB; ++js) {
                 if (js < nsb) {
+                    if (a.only_above && a.only_above[j0 + js] <= a.above)
+                        continue;
                     const size_t o = ((size_t)y * S + j0 + js) * C + x;
                     a.recon[o] = finalize(a, M::result(acc[k][js]), x, y);
                     if constexpr (M::kTwoOut)
@@ -707,6 +709,12 @@ __global__ __launch_bounds__(kThreads) void bp_tiled_kernel(
     bid /= tiles_x;
     const int ty = bid % tiles_y;
     const int grp = bid / tiles_y;
+    if (a.only_above) {
+        bool any = false;
+        for (int j = grp * SB; j < min(a.nslice, grp * SB + SB); ++j)
+            any = any || a.only_above[j] > a.above;
+        if (!any) return;
+    }
     bp_tile<MODE, SB, PY, A, Tin>(a, tx, ty, grp, sh);
 }
 
@@ -758,6 +766,7 @@ __global__ __launch_bounds__(kThreads) void bp_batched_kernel(
         a.apply_scale = jb.apply_scale;
         a.pi32 = (float)M_PI;
         a.denom = (float)(jb.nrow - 1);
+        a.only_above = nullptr;
         const int tiles_x = (jb.ncol + kTileX - 1) / kTileX;
         const int tiles_y = (jb.ncol + TY - 1) / TY;
         long long local = item - jb.tile_begin;

@@ -1,0 +1,808 @@
+// Back-projection of slice stacks on the matrix cores.
+//
+// One pixel's interpolation at one angle is a product of two weights with two
+// neighbouring detector samples, and the weights are the same for every
+// slice.  A 4 x 4 pixel block spans at most 3 (|cos| + |sin|) <= 4.25
+// detector columns, so its samples of one angle always lie in 8 columns that
+// start at an even column.  Four angles of one block are therefore one
+//     (16 pixels) x (4 angles x 8 columns) . (4 angles x 8 columns) x 16 slices
+// product: v_mfma_f32_16x16x32_f16 with a weight operand that holds two
+// non-zero entries per pixel and angle.  Building it costs about 30 VALU
+// instructions per block and four angles, shared by every slice of the
+// workgroup; the vector kernel (bp_tiled_kernel) pays 3.4 (16-bit) to 8.9
+// (reference typing) per pixel, angle and slice.
+//
+// Precision.  Nothing is reduced to 16 bits; 16-bit factors appear as exact
+// splits:
+//   * a float32 sample s, scaled by a power of two per slice so that
+//     max|s| <= 2^15, is h + l with h = f16(s), l = f16(s - h): 22-23 bits
+//     and an absolute floor of 2^-40 of the slice's maximum; 16-bit storage
+//     is one f16 value (bfloat16 after the same scaling, exact);
+//   * the fraction of the detector position, rounded to nearest on 22 bits,
+//     is 2^-11 a + 2^-22 b, and so is its complement; a, b <= 2^11 are
+//     integers, and an integer n <= 2048 read as a float16 bit pattern is
+//     exactly n 2^-24 (subnormals and the first two binades share one step),
+//     so a and b need no conversion;
+//   * every product (h + l)(a + b) is exact in float32, the sums are float32.
+// Sums over four angles at a time round fewer times than a float32 sum after
+// every angle does: from about 100 angles on the error against float64 is
+// below that of ATH_ACC_F32SEQ (181 angles of noise 1.9e-7 against 2.4e-7,
+// 1801 angles 4.2e-7 against 7.4e-7).
+//
+// A slice with a non-finite (or > 2^100) sample would spread it over the 8
+// columns of a window; such slices, found by the maximum that also gives the
+// scale, are redone by the vector kernel in the caller's accumulation.
+//
+// Measured (64 x 1801 x 2560, with the mask): float32 42 ms against 181 ms
+// for ATH_ACC_F32SEQ (17.9 against 4.2 updates per ps), float16 31
+// against 75 ms; 16 slices 15.8 against 46 ms.  What bounds it is VALU issue,
+// 41 instructions per block and four angles of 32 slices (76 % busy with the
+// matrix unit 41 %; simple 32-bit instructions take 1.2 ns per wave here,
+// permutes, shift-adds and float64 2.0, a matrix instruction 7.4 of which it
+// holds up the VALU for about 4).  Tried and left out: 8 waves per CU instead
+// of 16 (45 ms), four slice groups (48), records of four pairs for float32
+// (one product less, but twice the LDS stores: 17.4 against 15.8 ms for 16
+// slices), 2:4 sparse products (the weights would have to change lanes).
+//
+// Layout.  split_kernel writes the stack as (group of 16 slices, angle,
+// column pair, slice) entries: the f16 pair of two columns, high parts then
+// low parts.  A workgroup's strip of one angle is contiguous there.  It is
+// staged in LDS as one 16-byte record per (column pair i, slice): the pairs
+// i and i + 1 (high and low part each), or i .. i + 3 for 16-bit storage, so an
+// operand is read with aligned ds_read_b128 at any even column: a 4-byte
+// aligned 16-byte LDS read runs at 16 B per clock and CU here, an aligned
+// one at 208.  Records are double buffered: the next four angles are loaded
+// into registers before a step's arithmetic and stored after it.
+#include <cmath>
+#include <type_traits>
+
+#include "ath_internal.h"
+
+namespace ath {
+namespace {
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
+typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
+typedef unsigned short ushort2_t __attribute__((ext_vector_type(2)));
+
+// LDS by its 32-bit offset
+typedef __attribute__((address_space(3))) uint4_t* LdsQuad;
+typedef __attribute__((address_space(3))) uint2_t* LdsPair;
+typedef __attribute__((address_space(3))) half8_t* LdsHalf8;
+
+constexpr int kThreads = 1024;
+constexpr int kWaves = kThreads / 64;
+constexpr unsigned kPatchX = 8, kPatchY = 4;  // tiles
+constexpr int kGroup = 16;     // slices per matrix operand
+constexpr int kStep = 4;       // angles per matrix operand
+// |sample| above 2^100 (bit pattern) goes to the vector kernel
+constexpr unsigned kMaxBits = 0x71800000u;
+
+// SG slice groups per workgroup share the weights of its pixels; every tile
+// keeps 64 accumulator registers per lane.
+//   rows: records per angle.  A window starts at record e, 2 e < b <= 2 e + 2,
+//   b the block's lowest position less L (and a slack of 2^-20), L the tile's
+//   lowest position (less 2^-19) rounded down to even: 0 < b < 2 + 2^-19 +
+//   diag - 3, diag = sqrt((X-1)^2 + (Y-1)^2); the last record read is e + 2.
+//   wx: waves side by side (the others are below each other).
+// Tile corners lie on one 64-column grid, and a position is built from its
+// column's grid point, so that a slice's bits do not depend on the tile.
+template <int SG> struct Tile;
+template <> struct Tile<2> {
+    static constexpr int X = 32, Y = 32, rows = 24, wx = 2;
+};
+template <> struct Tile<1> {
+    static constexpr int X = 64, Y = 32, rows = 40, wx = 2;
+};
+template <int SG> constexpr bool rows_cover() {
+    // e <= ceil(b / 2) - 1 and e + 2 <= rows - 1, i.e. b <= 2 (rows - 2)
+    constexpr int X = Tile<SG>::X - 1, Y = Tile<SG>::Y - 1;
+    constexpr int m = 2 * (Tile<SG>::rows - 2);  // diag - 0.99 <= m
+    return 100 * 100 * (X * X + Y * Y) <= (100 * m + 99) * (100 * m + 99);
+}
+static_assert(rows_cover<2>() && rows_cover<1>(), "rows");
+
+// zero pairs past the last row, which a tile at its end may stage
+constexpr int kTailPairs = 64;
+static_assert(kTailPairs >= Tile<1>::rows + 16, "tail");
+
+struct MatArgs {
+    const unsigned* op;     // split samples
+    const unsigned* smax;   // per slice: bits of max|s|
+    const double2* trig;    // per angle: cos, sin
+    int scaled;             // samples carry the power of two of smax
+    int npair;              // column pairs per row
+    int group0, group_end;  // slice groups of the launch
+    int group_have;         // slice groups of the stack
+    unsigned patches_x, patches_y;
+};
+
+__device__ __forceinline__ double det_pos(double xc_c, double yc, double s,
+                                          double cen) {
+    return fma(yc, s, xc_c) + cen;  // as bp_tiled_kernel
+}
+
+// power of two that takes max|s| (its bits) into [2^14, 2^15); 0 where the
+// samples are all zero or the vector kernel takes the slice
+__device__ __forceinline__ int scale_exp(unsigned bits) {
+    if (bits == 0u || bits > kMaxBits) return 0;
+    return 14 - ilogbf(__uint_as_float(bits));
+}
+
+template <typename T> __device__ __forceinline__ float widen(T v);
+template <> __device__ __forceinline__ float widen<float>(float v) { return v; }
+template <> __device__ __forceinline__ float widen<__half>(__half v) {
+    return __half2float(v);
+}
+template <>
+__device__ __forceinline__ float widen<__hip_bfloat16>(__hip_bfloat16 v) {
+    return __bfloat162float(v);
+}
+
+__global__ void trig_kernel(const float* __restrict__ angles, int nrow,
+                            double2* __restrict__ trig,
+                            unsigned* __restrict__ smax, int nmax,
+                            unsigned* __restrict__ tail, int ntail) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nrow) {
+        const float th = -angles[i];
+        trig[i] = make_double2((double)(float)cos((double)th),
+                               (double)(float)sin((double)th));
+    }
+    if (i < nmax) smax[i] = 0u;
+    if (i < ntail) tail[i] = 0u;
+}
+
+// max|s| per slice: grid (row chunks, slices).  Integer order of the bit
+// patterns is the order of the magnitudes, with infinities and NaN on top.
+template <typename T>
+__global__ __launch_bounds__(256) void slice_max_kernel(
+    const T* __restrict__ sino, int nrow, int nslice, int ncol,
+    unsigned* __restrict__ smax) {
+    const int j = blockIdx.y;
+    unsigned m = 0u;
+    for (int r = blockIdx.x; r < nrow; r += gridDim.x) {
+        const T* row = sino + ((size_t)r * nslice + j) * ncol;
+        for (int c = threadIdx.x; c < ncol; c += 256)
+            m = max(m, __float_as_uint(fabsf(widen(row[c]))));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+    __shared__ unsigned part[4];
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = max(max(part[0], part[1]), max(part[2], part[3]));
+        if (m) atomicMax(&smax[j], m);
+    }
+}
+
+// (row, slice, column) samples -> (group, angle, pair, slice) entries.  A
+// block handles 128 columns of one angle's 16 slices through LDS, so both
+// the reads (columns) and the writes (slices) are contiguous.
+template <typename T, int PL>
+__global__ __launch_bounds__(256) void split_kernel(
+    const T* __restrict__ sino, int nrow, int nslice, int ncol, int npair,
+    const unsigned* __restrict__ smax, int scaled,
+    unsigned* __restrict__ op) {
+    constexpr int COLS = 128;
+    __shared__ float tile[kGroup][COLS + 1];
+    const int c0 = blockIdx.x * COLS, row = blockIdx.y, g = blockIdx.z;
+    const int tid = threadIdx.x;
+    for (int e = tid; e < kGroup * COLS; e += 256) {
+        const int n = e / COLS, c = c0 + e % COLS, j = g * kGroup + n;
+        float v = 0.0f;
+        if (j < nslice && c < ncol)
+            v = widen(sino[((size_t)row * nslice + j) * ncol + c]);
+        tile[n][e % COLS] = v;
+    }
+    __syncthreads();
+    const int n = tid & 15, j = g * kGroup + n;
+    const unsigned bits = j < nslice ? smax[j] : 0u;
+    const bool bad = bits > kMaxBits;  // redone by the vector kernel
+    const int ex = scaled ? scale_exp(bits) : 0;
+    unsigned* base = op + (((size_t)g * nrow + row) * npair) * (kGroup * PL);
+    for (int i = tid >> 4; i < COLS / 2; i += 16) {
+        const int p = c0 / 2 + i;
+        if (p >= npair) break;
+        float s0 = tile[n][2 * i], s1 = tile[n][2 * i + 1];
+        if (bad) s0 = s1 = 0.0f;
+        s0 = ldexpf(s0, ex);
+        s1 = ldexpf(s1, ex);
+        const half2_t h = {(_Float16)s0, (_Float16)s1};
+        unsigned* dst = base + ((size_t)p * kGroup + n) * PL;
+        if constexpr (PL == 2) {
+            const half2_t l = {(_Float16)(s0 - (float)h[0]),
+                               (_Float16)(s1 - (float)h[1])};
+            *reinterpret_cast<uint2_t*>(dst) =
+                uint2_t{__builtin_bit_cast(unsigned, h),
+                        __builtin_bit_cast(unsigned, l)};
+        } else {
+            *dst = __builtin_bit_cast(unsigned, h);
+        }
+    }
+}
+
+__device__ __forceinline__ double clamp_pos(double f, double w1) {
+    return fmin(fmax(f, 0.0), w1);
+}
+
+// a wave-uniform value in scalar registers
+__device__ __forceinline__ double to_scalar(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+// Geometry of one angle for a tile.  Positions are fixed point in the low
+// word of a double: 1.5 * 2^25 puts 27 fraction bits there (5 integer bits:
+// enough for the offset within a window; the 2 folds in the 1 of
+// -e = (127 - e) + 1 mod 16), 2^-23 rounds to the 22 bits that are kept;
+// 1.5 * 2^28 puts 24 fraction bits (8 integer bits: enough for a tile).
+constexpr double kPosMagic = 50331648.0 + 2.0 + 1.0 / 8388608.0;
+constexpr double kWinMagic = 402653184.0;
+constexpr double kSlack = 1.0 / 1048576.0;
+struct alignas(16) Angle {
+    double c, s;       // cos, sin
+    double pos;        // position = c x + s y + pos, less L, plus kPosMagic
+    double win;        // win - (c x + s y): kWinMagic less the lowest
+                       // position of the block centred at (x, y), less L,
+                       // plus the slack
+    int L;             // tile's first column (even)
+    int inner;         // every pixel of the tile is in range
+    int valid;         // the angle exists
+    int pad;
+};
+
+template <int PL, int SG>
+__global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
+                                                             MatArgs ma,
+                                                             int tiles_x,
+                                                             int tiles_y) {
+    using TL = Tile<SG>;
+    constexpr int S = SG * kGroup;
+    constexpr int ROWS = TL::rows;
+    constexpr int BX = TL::X / 4 / TL::wx;   // blocks per wave, side by side
+    static_assert(TL::Y / 4 * TL::wx == kWaves, "one row of blocks per wave");
+    // staging: a strip is the records of one (angle, slice group); a wave
+    // loads a SHARE-th of one, a 16-lane group RUN consecutive records
+    constexpr int SHARE = kWaves / (kStep * SG);
+    constexpr int WROWS = ROWS / SHARE;
+    constexpr int RUN = (WROWS + 3) / 4;
+    // a record: two pairs' high and low parts, or four pairs (WIDE)
+    constexpr bool WIDE = PL == 1;
+    constexpr int EXTRA = WIDE ? 3 : 1;               // pairs past a record
+    constexpr int kTerms = 2 * PL;                    // products per group
+    constexpr unsigned kRow = S * 16;
+    constexpr unsigned kBuf = kStep * ROWS * kRow;    // one step's records
+    static_assert(WROWS * SHARE == ROWS && SHARE * kStep * SG == kWaves,
+                  "rows split evenly");
+    using Raw = typename std::conditional<PL == 2, uint2_t, unsigned>::type;
+    constexpr int kPairBytes = kGroup * sizeof(Raw);  // one pair, 16 slices
+
+    // [8] selectors, three steps' angles [3][kStep], then records
+    // [2][kStep][ROWS][S], an angle's rows in descending order (the window
+    // counts down, see place)
+    extern __shared__ uint4_t lds[];
+    const unsigned sh = (unsigned)(size_t)(LdsQuad)lds;
+    constexpr unsigned kAngAt = 8 * 16;
+    Angle* const angles = reinterpret_cast<Angle*>(lds + 8);
+    constexpr unsigned kRecAt = kAngAt + 3 * kStep * sizeof(Angle);
+
+    // Workgroups go to the 8 XCDs in turn.  An XCD's consecutive ones take a
+    // kPatchX x kPatchY patch of tiles, whose strips of an angle overlap: one
+    // L2 then holds them for as many angles as the workgroups drift apart.
+    // Grid: groups x patches (a multiple of 8) x tiles of a patch.
+    const unsigned xcd = blockIdx.x & 7u, seq = blockIdx.x >> 3;
+    const unsigned patch = (seq / (kPatchX * kPatchY)) * 8u + xcd;
+    const unsigned in = seq % (kPatchX * kPatchY);
+    const unsigned px = patch % ma.patches_x, pr = patch / ma.patches_x;
+    const int tx = px * kPatchX + in % kPatchX;
+    const int ty = (pr % ma.patches_y) * kPatchY + in / kPatchX;
+    const int grp = ma.group0 + (pr / ma.patches_y) * SG;
+    if (tx >= tiles_x || ty >= tiles_y || grp >= ma.group_end) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n16 = lane & 15, k4 = lane >> 4;
+    const int x0 = tx * TL::X, y0 = ty * TL::Y;
+    const int xw = x0 + 4 * BX * (wv % TL::wx);       // this wave's pixels
+    const int yw = y0 + 4 * (wv / TL::wx);
+    const int C = a.ncol, N = a.nrow;
+    const double ic = a.icenter, cen = a.center, w1 = (double)(C - 1);
+
+    float4_t acc[BX][SG];
+#pragma unroll
+    for (int i = 0; i < BX; ++i)
+#pragma unroll
+        for (int g = 0; g < SG; ++g) acc[i][g] = float4_t{0, 0, 0, 0};
+
+    // a tile whose every pixel the mask removes needs no sums
+    bool masked = false;
+    if (a.use_mask) {
+        const int xl = x0 - a.mask_c, xh = x0 + TL::X - 1 - a.mask_c;
+        const int yl = y0 - a.mask_c, yh = y0 + TL::Y - 1 - a.mask_c;
+        const long long dx = xl > 0 ? xl : (xh < 0 ? xh : 0);
+        const long long dy = yl > 0 ? yl : (yh < 0 ? yh : 0);
+        masked = !((double)(dx * dx + dy * dy) <= a.mask_r2);
+    }
+
+    if (!masked) {
+        // selectors of the byte permutation that places (1 - w, w) at columns
+        // d, d + 1 of the window's 8: entry d <= 6, one word per column
+        // pair; entry 7 places nothing (pixels out of range)
+        if (tid < 32) {
+            const int d = tid >> 2, p = tid & 3;
+            unsigned sel = 0;
+            for (int h = 0; h < 2; ++h) {
+                const int col = 2 * p + h;
+                const unsigned v = d == 7 ? 0x0c0cu
+                                   : col == d ? 0x0100u
+                                   : col == d + 1 ? 0x0302u : 0x0c0cu;
+                sel |= v << (16 * h);
+            }
+            reinterpret_cast<unsigned*>(lds)[tid] = sel;
+        }
+
+        // the lane's pixel and, for the windows, the block's centre, both in
+        // the grid column of 64 that holds the tile
+        const int xg = x0 & ~63;
+        const double xl = (double)(xg + (n16 & 3)) - ic;
+        const double yl = (double)(yw + (n16 >> 2)) - ic;
+        const double xb = to_scalar((double)xg + 1.5 - ic);
+        const double yb = to_scalar((double)yw + 1.5 - ic);
+
+        auto trig = [&](int a0) { return ma.trig[min(a0 + k4, N - 1)]; };
+        // lanes 0, 16, 32, 48 of one wave: the angles of the step at a0
+        auto geometry = [&](int a0, double2 t, unsigned slot) {
+            const double xm = (double)x0 + 0.5 * (TL::X - 1) - ic;
+            const double ym = (double)y0 + 0.5 * (TL::Y - 1) - ic;
+            const double fm = det_pos(xm * t.x, ym, t.y, cen);
+            const double ext = fma(0.5 * (TL::Y - 1), fabs(t.y),
+                                   0.5 * (TL::X - 1) * fabs(t.x));
+            const double lo = fm - ext - 2.0 * kSlack;
+            const double hi = fm + ext + 2.0 * kSlack;
+            Angle g;
+            g.c = t.x;
+            g.s = t.y;
+            g.L = (int)clamp_pos(lo, w1) & ~1;
+            g.valid = a0 + k4 < N;
+            g.inner = g.valid && lo >= 0.0 && hi <= w1;
+            g.pad = 0;
+            const double off = cen - (double)g.L;
+            g.pos = off + kPosMagic;
+            g.win = kWinMagic -
+                    (off - fma(1.5, fabs(t.x) + fabs(t.y), kSlack));
+            if (n16 == 0) angles[slot * kStep + k4] = g;
+        };
+
+        // this wave's share of a strip
+        const int sk = wv / SHARE / SG, sg = wv / SHARE % SG;
+        const int row0 = wv % SHARE * WROWS + k4 * RUN;
+        const int row_end = wv % SHARE * WROWS + WROWS;
+        const unsigned lane_at = (unsigned)(row0 * kGroup + n16) * sizeof(Raw);
+        // (an idle last group repeats the one before it)
+        const int gr = min(grp + sg, ma.group_have - 1);
+        Raw raw[RUN + EXTRA];
+        // (pairs past the row's end are the next row's, or the buffer's zero
+        // tail: finite, and their weights are zero)
+        auto load = [&](int a0, unsigned slot) {
+            const int ai = min(a0 + sk, N - 1);
+            const int L =
+                __builtin_amdgcn_readfirstlane(angles[slot * kStep + sk].L);
+            const char* src =
+                reinterpret_cast<const char*>(ma.op) +
+                (((size_t)gr * N + ai) * ma.npair + (L >> 1)) * kPairBytes;
+#pragma unroll
+            for (int u = 0; u < RUN + EXTRA; ++u)
+                raw[u] = *reinterpret_cast<const Raw*>(
+                    src + (lane_at + u * kPairBytes));
+        };
+        auto store = [&](unsigned buf) {
+            // row RUN - 1 of the run lies lowest
+            const unsigned dst =
+                sh + kRecAt + buf * kBuf +
+                (sk * ROWS + ROWS - RUN - row0) * kRow +
+                (sg * kGroup + n16) * 16;
+#pragma unroll
+            for (int u = 0; u < RUN; ++u) {
+                const Raw* r = raw + u;
+                if (RUN * 4 != WROWS && row0 + u >= row_end) continue;
+                const unsigned at = dst + (RUN - 1 - u) * kRow;
+                if constexpr (PL == 2) {
+                    // two 8-byte stores: one instruction, no copies of the
+                    // entry that two records share
+                    *(LdsPair)(at) = r[0];
+                    *(LdsPair)(at + 8) = r[1];
+                } else {
+                    *(LdsQuad)(at) = uint4_t{r[0], r[1], r[2], r[3]};
+                }
+            }
+        };
+
+        // One block of pixels goes through four stages, a stage per turn of
+        // the block loop, so that LDS latencies and the matrix unit's own lie
+        // behind other blocks' work: its weights' halves and selectors
+        // (place), the weight operands and the records they meet (operands),
+        // the products, and the sum into the total.
+        struct Place {
+            unsigned pa, pb, at;
+            uint4_t sel;
+        };
+        struct Operands {
+            half8_t w[kTerms];
+            half8_t r[SG][PL == 2 ? 2 : 1];
+        };
+        struct Sums {
+            float4_t t[SG];
+        };
+        // p: the lane's position; e: 127 - the window's record (its sign
+        // takes one shift-add off the offset in the window)
+        auto place = [&](unsigned p, unsigned e, unsigned lbase) {
+            Place k;
+            const unsigned rel = (e << 28) + p;
+            k.sel = *(LdsQuad)(((rel >> 23) & 0x70u) | sh);
+            k.at = e * kRow + lbase;
+            const unsigned T = p & 0x07ffffe0u;        // w, 22 bits
+            const unsigned Q = 0x08000000u - T;        // 1 - w
+            k.pa = __builtin_amdgcn_perm(T, Q, 0x07060302u);
+            k.pb = __builtin_amdgcn_perm(T, Q, 0x05040100u);
+            k.pb = __builtin_bit_cast(
+                unsigned,
+                (ushort2_t)(__builtin_bit_cast(ushort2_t, k.pb) >> 5));
+            // 2^-24 a -> 2^-13 a, so that a and b share the scale 2^-2
+            const half2_t up = {(_Float16)2048.0f, (_Float16)2048.0f};
+            k.pa = __builtin_bit_cast(unsigned,
+                                      __builtin_bit_cast(half2_t, k.pa) * up);
+            return k;
+        };
+        auto operands = [&](const Place& k) {
+            Operands o;
+#pragma unroll
+            for (int g = 0; g < SG; ++g) {
+                if constexpr (PL == 2) {
+                    // the record and the second one after it
+                    o.r[g][0] = *(LdsHalf8)(k.at + 2 * kRow + g * kGroup * 16);
+                    o.r[g][1] = *(LdsHalf8)(k.at + g * kGroup * 16);
+                } else {
+                    o.r[g][0] = *(LdsHalf8)(k.at + g * kGroup * 16);
+                }
+            }
+            unsigned wa[4], wb[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                wa[q] = __builtin_amdgcn_perm(0u, k.pa, k.sel[q]);
+                wb[q] = __builtin_amdgcn_perm(0u, k.pb, k.sel[q]);
+            }
+            if constexpr (!WIDE) {
+                // records hold a pair's high and low parts side by side
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    o.w[h] = __builtin_bit_cast(
+                        half8_t, (uint4_t{wb[2 * h], wb[2 * h], wb[2 * h + 1],
+                                          wb[2 * h + 1]}));
+                    o.w[2 + h] = __builtin_bit_cast(
+                        half8_t, (uint4_t{wa[2 * h], wa[2 * h], wa[2 * h + 1],
+                                          wa[2 * h + 1]}));
+                }
+            } else {
+                o.w[0] = __builtin_bit_cast(
+                    half8_t, (uint4_t{wb[0], wb[1], wb[2], wb[3]}));
+                o.w[1] = __builtin_bit_cast(
+                    half8_t, (uint4_t{wa[0], wa[1], wa[2], wa[3]}));
+            }
+            return o;
+        };
+        // A step's sum starts from zero and is added to the total in the
+        // vector unit: the matrix unit truncates, and into the total that
+        // would be a bias (1801 angles of positive samples: -7e-7).
+        auto products = [&](const Operands& o) {
+            Sums u;
+#pragma unroll
+            for (int g = 0; g < SG; ++g) u.t[g] = float4_t{0, 0, 0, 0};
+            // (small terms first: they are truncated at their own size)
+#pragma unroll
+            for (int q = 0; q < kTerms; ++q)
+#pragma unroll
+                for (int g = 0; g < SG; ++g)
+                    u.t[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        o.w[q], o.r[g][PL == 2 ? q & 1 : 0], u.t[g], 0, 0, 0);
+            return u;
+        };
+        auto total = [&](const Sums& u, float4_t (&ac)[SG]) {
+#pragma unroll
+            for (int g = 0; g < SG; ++g)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) ac[g][q] += u.t[g][q];
+        };
+        // the other stages' instructions between the matrix instructions
+        auto interleave = [&]() {
+            constexpr int M = kTerms * SG;
+            constexpr int V = (PL == 1 ? 22 : 30) + 4 * SG;
+#pragma unroll
+            for (int q = 0; q < M; ++q) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (V + M - 1) / M,
+                                                     0);
+            }
+        };
+
+        if (wv == 0) {
+            geometry(0, trig(0), 0);
+            geometry(kStep, trig(kStep), 1);
+        }
+        __syncthreads();
+        load(0, 0);
+        store(0);
+        __syncthreads();
+        // step t: its angles are in slot t % 3; the samples of step t + 1 are
+        // loaded and stored, and one wave works out the angles of step t + 2
+        unsigned cur = 0, buf = 0, turn = 0;
+        double2 tr = trig(2 * kStep);
+        for (int a0 = 0; a0 < N; a0 += kStep) {
+            const unsigned next = cur == 2 ? 0 : cur + 1;
+            const unsigned after = next == 2 ? 0 : next + 1;
+            if (wv == (int)turn) geometry(a0 + 2 * kStep, tr, after);
+            turn = turn + 1 == kWaves ? 0 : turn + 1;
+            // (past the last angle these repeat it)
+            load(a0 + kStep, next);
+            const Angle* g = angles + cur * kStep + k4;
+            const double c = g->c, s = g->s;
+            // record 127 - e of the lane's angle and the second one after it
+            // (lower) start e rows past here
+            const unsigned lbase =
+                sh + kRecAt + buf * kBuf +
+                (unsigned)(k4 * ROWS + ROWS - 1 - 127 - (WIDE ? 0 : 2)) * kRow +
+                n16 * 16;
+            const double fr = fma(yl, s, fma(xl, c, g->pos));
+            unsigned p[BX], e[BX];
+            if (__all(g->inner)) {
+                const double bn = fma(-yb, s, fma(-xb, c, g->win));
+#pragma unroll
+                for (int i = 0; i < BX; ++i) {
+                    const double m = (double)(xw - xg + 4 * i);
+                    p[i] = (unsigned)__double2loint(fma(m, c, fr));
+                    e[i] = (unsigned)__double2loint(fma(-m, c, bn)) >> 25;
+                }
+            } else {
+                // some pixel or angle is out of range: the vector kernel's
+                // exact position decides which, window positions are clamped
+                // to the row, and in-range pixels keep the weights above
+                // (opaque, so that the columns' coordinates are not kept in
+                // registers across the angle loop)
+                double xo = xl, yo = yl;
+                asm volatile("" : "+v"(xo), "+v"(yo));
+                const double l = (double)g->L;
+                const double br = det_pos(xb * c, yb, s, cen) -
+                                  fma(1.5, fabs(c) + fabs(s), kSlack);
+                const bool valid = g->valid;
+#pragma unroll
+                for (int i = 0; i < BX; ++i) {
+                    const double m = (double)(xw - xg + 4 * i);
+                    const double f = det_pos((xo + m) * c, yo, s, cen);
+                    const bool in = f >= 0.0 && f <= w1;
+                    const double edge = clamp_pos(f, w1) - l + kPosMagic;
+                    const double b =
+                        clamp_pos(fma(m, c, br), w1) - l + 0.5 * kSlack;
+                    e[i] = (unsigned)__double2loint(kWinMagic - b) >> 25;
+                    p[i] = (unsigned)__double2loint(in ? fma(m, c, fr) : edge);
+                    // selector 7: no weights
+                    unsigned none = e[i];
+                    asm volatile("" : "+v"(none));
+                    if (!valid || (!in && !a.edge_pad))
+                        p[i] = 0x38000000u - (none << 28);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            Place pl = place(p[0], e[0], lbase);
+            Operands op = operands(pl);
+            if (BX > 1) pl = place(p[1], e[1], lbase);
+            Sums su;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < BX; ++i) {
+                const Sums next_su = products(op);
+                if (i > 0) total(su, acc[i - 1]);
+                if (i + 1 < BX) op = operands(pl);
+                if (i + 2 < BX) pl = place(p[i + 2], e[i + 2], lbase);
+                su = next_su;
+                interleave();
+                __builtin_amdgcn_sched_barrier(0);
+                // the samples have arrived: their stores go beside the
+                // other waves' products
+                if (i == BX * 3 / 4 - 1) store(buf ^ 1);
+            }
+            total(su, acc[BX - 1]);
+            tr = trig(a0 + 3 * kStep);
+            cur = next;
+            buf ^= 1;
+            __syncthreads();
+        }
+    }
+
+    // lane: slice n16 of each group; rows 4 g + r of the product are the
+    // pixels (x + r, y + g), g = lane >> 4
+    const bool vec = (C & 3) == 0 && (reinterpret_cast<size_t>(a.recon) & 15) == 0;
+#pragma unroll
+    for (int g = 0; g < SG; ++g) {
+        const int j = (grp + g) * kGroup + n16;
+        if (j >= a.nslice) continue;
+        const unsigned bits = ma.smax[j];
+        if (bits > kMaxBits) continue;  // the vector kernel's
+        const int ex = 2 - (ma.scaled ? scale_exp(bits) : 0);
+        const int y = yw + k4;
+        if (y >= C) continue;
+        float* row = a.recon + ((size_t)y * a.nslice + j) * C;
+        const long long dy = y - a.mask_c;
+#pragma unroll
+        for (int i = 0; i < BX; ++i) {
+            const int x = xw + 4 * i;
+            __builtin_amdgcn_sched_barrier(0);
+            float4_t v;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float t = ldexpf(acc[i][g][q], ex);
+                if (a.use_mask) {
+                    const long long dx = x + q - a.mask_c;
+                    t *= (double)(dx * dx + dy * dy) <= a.mask_r2 ? 1.0f
+                                                                  : 0.0f;
+                }
+                if (a.apply_scale) {
+                    t = t * a.pi32;
+                    t = t / a.denom;
+                }
+                v[q] = t;
+            }
+            if (vec && x + 3 < C) {
+                *reinterpret_cast<float4_t*>(row + x) = v;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (x + q < C) row[x + q] = v[q];
+            }
+        }
+    }
+}
+
+template <int PL, int SG>
+int launch_matrix(const BpArgs& a, MatArgs ma, int groups,
+                  hipStream_t stream) {
+    using TL = Tile<SG>;
+    const int tiles_x = (a.ncol + TL::X - 1) / TL::X;
+    const int tiles_y = (a.ncol + TL::Y - 1) / TL::Y;
+    ma.group_end = ma.group0 + groups;
+    ma.patches_x = (tiles_x + kPatchX - 1) / kPatchX;
+    ma.patches_y = (tiles_y + kPatchY - 1) / kPatchY;
+    const long long patches =
+        (long long)ma.patches_x * ma.patches_y * (groups / SG);
+    const long long blocks = (patches + 7) / 8 * 8 * (kPatchX * kPatchY);
+    if (blocks > 0x7fffffffLL)
+        return set_error(ATH_ERR_UNSUPPORTED, "back-projection grid too large");
+    auto kern = bp_matrix_kernel<PL, SG>;
+    const size_t lds =
+        (size_t)(2 * kStep * TL::rows * SG * kGroup + 8) * sizeof(uint4_t) +
+        3 * kStep * sizeof(Angle);
+    const int st = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
+    if (st != ATH_OK) return st;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), lds,
+                       stream, a, ma, tiles_x, tiles_y);
+    return check_hip(hipGetLastError(), "bp_matrix_kernel launch");
+}
+
+// rounds of 256 workgroups that `units` slice groups (or pairs) take
+template <int SG> double rounds_of(int ncol, int units) {
+    const double tiles = (double)((ncol + Tile<SG>::X - 1) / Tile<SG>::X) *
+                         ((ncol + Tile<SG>::Y - 1) / Tile<SG>::Y);
+    return std::ceil(tiles * units / 256.0);
+}
+
+size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+int groups_of(int nslice) { return (nslice + kGroup - 1) / kGroup; }
+int planes_of(int dtype) { return dtype == ATH_F32 ? 2 : 1; }
+
+template <typename T, int PL>
+int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
+               hipStream_t s) {
+    const int groups = groups_of(a.nslice), npair = (a.ncol + 1) / 2;
+    MatArgs ma;
+    unsigned* smax = reinterpret_cast<unsigned*>(work);
+    work += align256((size_t)groups * kGroup * sizeof(unsigned));
+    double2* trig = reinterpret_cast<double2*>(work);
+    work += align256((size_t)a.nrow * sizeof(double2));
+    unsigned* op = reinterpret_cast<unsigned*>(work);
+    ma.op = op;
+    ma.smax = smax;
+    ma.trig = trig;
+    ma.scaled = dtype != ATH_F16;
+    ma.npair = npair;
+    const int nmax = groups * kGroup;
+    const size_t nop = (size_t)groups * kGroup * a.nrow * npair * PL;
+    const int ntail = kTailPairs * kGroup * PL;
+    const T* sino = static_cast<const T*>(a.sino);
+    hipLaunchKernelGGL(trig_kernel,
+                       dim3((std::max({a.nrow, nmax, ntail}) + 255) / 256),
+                       dim3(256), 0, s, a.angles, a.nrow, trig, smax, nmax,
+                       op + nop, ntail);
+    int st = check_hip(hipGetLastError(), "trig_kernel launch");
+    if (st != ATH_OK) return st;
+    hipLaunchKernelGGL((slice_max_kernel<T>),
+                       dim3((unsigned)std::min(a.nrow, 128),
+                            (unsigned)a.nslice),
+                       dim3(256), 0, s, sino, a.nrow, a.nslice, a.ncol, smax);
+    st = check_hip(hipGetLastError(), "slice_max_kernel launch");
+    if (st != ATH_OK) return st;
+    hipLaunchKernelGGL((split_kernel<T, PL>),
+                       dim3((unsigned)((a.ncol + 127) / 128),
+                            (unsigned)a.nrow, (unsigned)groups),
+                       dim3(256), 0, s, sino, a.nrow, a.nslice, a.ncol, npair,
+                       smax, ma.scaled, op);
+    st = check_hip(hipGetLastError(), "split_kernel launch");
+    if (st != ATH_OK) return st;
+    ma.group0 = 0;
+    ma.group_have = groups;
+    // Pairs of groups; a last odd group by itself unless an idle one beside
+    // it is cheaper, which it is where the launch does not fill the chip
+    // twice (rounds of 256 workgroups, at the measured 0.69 against 0.88 us
+    // per angle)
+    int pairs = groups / 2;
+    if (groups & 1) {
+        const double with = rounds_of<2>(a.ncol, pairs + 1) * 0.69;
+        const double apart = rounds_of<2>(a.ncol, pairs) * 0.69 +
+                             rounds_of<1>(a.ncol, 1) * 0.88;
+        if (with < apart) ++pairs;
+    }
+    if (pairs) {
+        st = launch_matrix<PL, 2>(a, ma, 2 * pairs, s);
+        if (st != ATH_OK) return st;
+        ma.group0 = 2 * pairs;
+    }
+    if (groups > 2 * pairs) {
+        st = launch_matrix<PL, 1>(a, ma, 1, s);
+        if (st != ATH_OK) return st;
+    }
+    // slices with non-finite or huge samples (workgroups of others leave at
+    // once)
+    BpArgs rest = a;
+    rest.only_above = smax;
+    rest.above = kMaxBits;
+    return back_projection(rest, dtype, acc, 0, 0, s);
+}
+
+}  // namespace
+
+size_t back_projection_matrix_workspace(int dtype, int nrow, int nslice,
+                                        int ncol) {
+    const size_t groups = groups_of(nslice);
+    return align256(groups * kGroup * sizeof(unsigned)) +
+           align256((size_t)nrow * sizeof(double2)) +
+           (groups * nrow * (size_t)((ncol + 1) / 2) + kTailPairs) * kGroup *
+               4 * planes_of(dtype);
+}
+
+int back_projection_matrix(const BpArgs& a, int dtype, int acc, void* work,
+                           hipStream_t s) {
+    if (a.ncol > kMaxMatrixCols || a.nrow > 65535 || a.nslice > 65535)
+        return set_error(ATH_ERR_UNSUPPORTED,
+                         "matrix back-projection: at most 32768 columns, "
+                         "65535 angles and 65535 slices");
+    char* w = static_cast<char*>(work);
+    if (dtype == ATH_F32) {
+        if (acc != ATH_ACC_F32SEQ && acc != ATH_ACC_F32)
+            return set_error(ATH_ERR_INVALID_ARG,
+                             "matrix back-projection: acc must be "
+                             "ATH_ACC_F32SEQ or ATH_ACC_F32");
+        return run_matrix<float, 2>(a, dtype, acc, w, s);
+    }
+    if (acc != ATH_ACC_F32)
+        return set_error(ATH_ERR_UNSUPPORTED,
+                         "back-projection: float16/bfloat16 sinograms need "
+                         "acc = ATH_ACC_F32");
+    if (dtype == ATH_F16) return run_matrix<__half, 1>(a, dtype, acc, w, s);
+    if (dtype == ATH_BF16)
+        return run_matrix<__hip_bfloat16, 1>(a, dtype, acc, w, s);
+    return set_error(ATH_ERR_INVALID_ARG, "back-projection: bad sinogram dtype");
+}
+
+}  // namespace ath

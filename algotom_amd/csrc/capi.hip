@@ -143,6 +143,8 @@ int fill_bp_args(BpArgs& a, const void* sino, int nrow, int nslice, int ncol,
     a.apply_scale = apply_scale ? 1 : 0;
     a.pi32 = (float)M_PI;
     a.denom = (float)(nrow - 1);
+    a.only_above = nullptr;
+    a.above = 0u;
     return ATH_OK;
 }
 
@@ -356,6 +358,44 @@ int ath_back_projection(const void* sino, int sino_dtype, int nrow,
     if (st != ATH_OK) return st;
     return back_projection(a, sino_dtype, acc, 0, 0,
                            static_cast<hipStream_t>(stream));
+}
+
+size_t ath_back_projection_matrix_workspace_bytes(int sino_dtype, int nrow,
+                                                  int nslice, int ncol) {
+    if (nrow < 1 || nslice < 1 || ncol < 1 || ncol > kMaxMatrixCols ||
+        (sino_dtype != ATH_F32 && sino_dtype != ATH_F16 &&
+         sino_dtype != ATH_BF16))
+        return 0;
+    return back_projection_matrix_workspace(sino_dtype, nrow, nslice, ncol);
+}
+
+int ath_back_projection_matrix(const void* sino, int sino_dtype, int nrow,
+                               int nslice, int ncol, const float* angles,
+                               float center, int edge_pad, int acc,
+                               double mask_radius, int apply_scale,
+                               float* recon, void* workspace,
+                               size_t workspace_bytes, void* stream) {
+    clear_error();
+    BpArgs a;
+    int st = fill_bp_args(a, sino, nrow, nslice, ncol, angles, center,
+                          edge_pad, mask_radius, apply_scale, recon);
+    if (st != ATH_OK) return st;
+    if (!workspace)
+        return set_error(ATH_ERR_INVALID_ARG, "null device pointer");
+    if (reinterpret_cast<size_t>(workspace) & 15)
+        return set_error(ATH_ERR_INVALID_ARG,
+                         "the workspace must be 16-byte aligned");
+    const size_t need = ath_back_projection_matrix_workspace_bytes(
+        sino_dtype, nrow, nslice, ncol);
+    if (need == 0)
+        return set_error(ATH_ERR_UNSUPPORTED,
+                         "matrix back-projection: float32, float16 or "
+                         "bfloat16 sinograms of at most 32768 columns");
+    if (workspace_bytes < need)
+        return set_error(ATH_ERR_WORKSPACE,
+                         "matrix back-projection workspace too small");
+    return back_projection_matrix(a, sino_dtype, acc, workspace,
+                                  static_cast<hipStream_t>(stream));
 }
 
 int ath_back_projection_with_derivative(const float* sino, int nrow,

@@ -48,7 +48,8 @@ class BatchFBP:
     it: with ``precision=None`` a single sinogram with ``gpu=True`` is
     back-projected with float64 sums and the rest with float32 storage
     after every angle, so the batch runs one persistent back-projection
-    launch per arithmetic it contains.
+    launch per arithmetic it contains, and one launch per stack that
+    fbp_reconstruction sums on the matrix cores.
     """
 
     def __init__(self, shapes, centers, angles=None, filter_name="hann",
@@ -139,29 +140,50 @@ class BatchFBP:
             self.filter_groups.append((L, code, len(members), row,
                                        self._to_device(jobs)))
 
+        def mask_radius(i):
+            c, ncol = centers[i], self.shapes3[i][2]
+            if c < 0 or c >= ncol:
+                raise ValueError("Center is out of the range [0, {}]"
+                                 .format(ncol - 1))
+            if ratio is None:
+                return -1.0
+            r = ratio
+            if r == 0.0:
+                r = min(c, ncol - c) / (0.5 * ncol)
+            return float(r * (ncol // 2))
+
+        # ---- stacks that fbp_reconstruction sums on the matrix cores: a
+        # launch each, sharing one workspace
+        self.matrix_jobs = []
+        matrix = [rec._matrix_stack(*s, accs[i], store)
+                  for i, s in enumerate(self.shapes3)]
+        for i in range(n):
+            if matrix[i]:
+                self.matrix_jobs.append(
+                    (i, accs[i], float(np.float32(centers[i])),
+                     mask_radius(i)))
+        self.matrix_work = None
+        if self.matrix_jobs:
+            self.matrix_work = max(
+                (rec._matrix_workspace(*self.shapes3[job[0]], store, self.dev)
+                 for job in self.matrix_jobs), key=lambda w: w.numel())
+
         # ---- back-projection work lists, one per arithmetic: heaviest
         # per-tile cost (most angles) first
         self.bp_groups = []
         for acc in sorted(set(accs)):
-            members = [i for i in range(n) if accs[i] == acc]
+            members = [i for i in range(n) if accs[i] == acc
+                       and not matrix[i]]
+            if not members:
+                continue
             order = sorted(members, key=lambda i: -self.shapes3[i][0])
             jobs = (nat.BpJob * len(order))()
             for k, i in enumerate(order):
                 nrow, nslice, ncol = self.shapes3[i]
-                c = centers[i]
-                if c < 0 or c >= ncol:
-                    raise ValueError("Center is out of the range [0, {}]"
-                                     .format(ncol - 1))
-                radius = -1.0
-                if ratio is not None:
-                    r = ratio
-                    if r == 0.0:
-                        r = min(c, ncol - c) / (0.5 * ncol)
-                    radius = float(r * (ncol // 2))
                 jobs[k] = nat.BpJob(
                     self.filtered[i].data_ptr(), self.outputs[i].data_ptr(),
                     self._angles[i].data_ptr(), nrow, nslice, ncol,
-                    float(np.float32(c)), radius, 1, 0, 0)
+                    float(np.float32(centers[i])), mask_radius(i), 1, 0, 0)
             sb = 1 if all(self.shapes3[i][1] == 1 for i in members) else 4
             self.bp_groups.append({
                 "acc": acc, "slice_batch": sb, "jobs": jobs,
@@ -214,6 +236,14 @@ class BatchFBP:
                 self.store_code, g["acc"], g["slice_batch"], self.tile_rows,
                 self.nblocks, nat.ptr(g["counter"]), stream),
                 "ath_back_projection_batched")
+        for i, acc, center, radius in self.matrix_jobs:
+            nrow, nslice, ncol = self.shapes3[i]
+            nat.check(self.lib.ath_back_projection_matrix(
+                nat.ptr(self.filtered[i]), self.store_code, nrow, nslice,
+                ncol, nat.ptr(self._angles[i]), center, 0, acc, radius, 1,
+                nat.ptr(self.outputs[i]), nat.ptr(self.matrix_work),
+                self.matrix_work.numel(), stream),
+                "ath_back_projection_matrix")
 
     def capture(self):
         """Record launch() in a HIP graph; run() then replays it."""

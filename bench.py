@@ -855,6 +855,9 @@ def main():
     acc = nat.ACC_F32SEQ if args.precision is None else nat.ACC_F32
     store = rec._storage_dtype(args.precision)
     mask_radius = float(1.0 * (NCOL // 2))
+    project = (rec._backproject_matrix
+               if rec._matrix_stack(NROW, NSLICE, NCOL, acc, store)
+               else rec._backproject_stack)
 
     def step(events=None):
         # exactly fbp_reconstruction's device path, split so the
@@ -863,9 +866,8 @@ def main():
         filt = rec._filter_stack(sino, pad, "edge", True, taps, store)
         if events:
             events[0].record()
-        out = rec._backproject_stack(filt, angles, CENTER, acc,
-                                     mask_radius=mask_radius,
-                                     apply_scale=True)
+        out = project(filt, angles, CENTER, acc, mask_radius=mask_radius,
+                      apply_scale=True)
         if events:
             events[1].record()
         return out

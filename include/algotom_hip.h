@@ -173,6 +173,26 @@ int ath_back_projection(const void* sino, int sino_dtype, int nrow,
                         double mask_radius, int apply_scale, float* recon,
                         void* stream);
 
+/* The back-projection of a stack on the matrix cores (the fast path of
+ * fbp_reconstruction and bpf_reconstruction for stacks): samples and
+ * interpolation weights as exact two-term float16 splits (22 bits), float32
+ * sums.  Not bit-identical to ath_back_projection; from about 100 angles on
+ * its error against float64 is below that of ATH_ACC_F32SEQ.  A slice's result does not
+ * depend on the other slices of the stack.  sino_dtype: ATH_F32 (acc
+ * ATH_ACC_F32SEQ or ATH_ACC_F32), ATH_F16 or ATH_BF16 (acc ATH_ACC_F32).
+ * Slices with a non-finite or > 2^100 sample are computed with acc exactly
+ * as ath_back_projection does.  workspace: device memory of at least
+ * ath_back_projection_matrix_workspace_bytes(...) (0: unsupported), 16-byte
+ * aligned; ATH_ERR_WORKSPACE when too small. */
+size_t ath_back_projection_matrix_workspace_bytes(int sino_dtype, int nrow,
+                                                  int nslice, int ncol);
+int ath_back_projection_matrix(const void* sino, int sino_dtype, int nrow,
+                               int nslice, int ncol, const float* angles,
+                               float center, int edge_pad, int acc,
+                               double mask_radius, int apply_scale,
+                               float* recon, void* workspace,
+                               size_t workspace_bytes, void* stream);
+
 /* The back-projection of ath_back_projection with acc ATH_ACC_F64 into
  * recon and, in the same pass over the same positions and staged samples,
  * its derivative with respect to the rotation centre (acc ATH_ACC_DERIV)

@@ -1,0 +1,133 @@
+"""Matrix-core back-projection of stacks (ath_back_projection_matrix).
+
+Bar, against the float64-sum kernel on the same (16-bit: widened) samples:
+relative 2-norm error at most max(error of ATH_ACC_F32SEQ, 3e-7).  3e-7 is
+the sum of what the design allows at few angles, where a float32 sum after
+every angle rounds less often: samples and weights of 22 bits (2^-23 each),
+a truncated float32 sum over four angles (3 products at 2^-24 of it, at most
+doubled by the difference between a partial sum and the total).
+"""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# ncol, nrow, nslice, centre, angle span, edge_pad.  Tiles are 32 x 32 (pairs
+# of 16 slices) and 64 x 32 (a last group), steps 4 angles, staged strips end
+# at the row's last column pair.
+CASES = [
+    (65, 37, 5, 32.0, np.pi, False),         # one padded group, odd width
+    (64, 4, 16, 31.5, np.pi, True),          # one step
+    (97, 5, 17, 96.0, np.pi, True),          # one angle past a step; a pair
+    (257, 61, 33, 128.0 - 7.25, 2 * np.pi, True),  # pair + one group
+    (130, 181, 48, 3.0, np.pi, False),       # centre at the edge
+    (512, 181, 16, 255.1, np.pi, False),     # whole tiles
+    (1025, 130, 9, 512.37, np.pi, False),    # one column past 16 tiles
+    (7192, 9, 6, 3595.5, 2 * np.pi, False),  # 64-bit offsets, widest windows
+]
+
+
+def _case(ncol, nrow, nslice, span, seed):
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn((nrow, nslice, ncol), generator=gen, device="cuda")
+    ang = np.linspace(0.0, span, nrow, endpoint=False) + 1e-3 * seed
+    return x, ang
+
+
+def _rel(got, ref):
+    return ((got.double() - ref.double()).norm() / ref.double().norm()).item()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_error_against_float64_sums(case, dtype):
+    import torch
+    from algotom_amd.rec import reconstruction as rec
+    ncol, nrow, nslice, center, span, edge = CASES[case]
+    print("case", CASES[case], dtype, flush=True)
+    x, ang = _case(ncol, nrow, nslice, span, case)
+    x = x.to(getattr(torch, dtype))
+    ref = rec._backproject_stack(x.float(), ang, center, 0, edge)
+    seq = rec._backproject_stack(x.float(), ang, center, 1, edge)
+    got = rec._backproject_matrix(x, ang, center,
+                                  1 if dtype == "float32" else 2, edge)
+    err, bound = _rel(got, ref), max(_rel(seq, ref), 3e-7)
+    print("error %.3g, bound %.3g" % (err, bound))
+    assert err <= bound
+
+
+def test_slice_bits_do_not_depend_on_the_stack():
+    """A slice in a pair of groups, alone in a group, or beside other slices
+    keeps its bits, and so do mask and scale (zero outside the circle)."""
+    import torch
+    from algotom_amd.rec import reconstruction as rec
+    x, ang = _case(200, 133, 37, np.pi, 3)
+    kw = dict(mask_radius=90.0, apply_scale=True)
+    full = rec._backproject_matrix(x, ang, 97.6, 1, **kw)
+    for j0, j1 in ((0, 5), (20, 36), (36, 37), (3, 33)):
+        part = rec._backproject_matrix(x[:, j0:j1].contiguous(), ang, 97.6,
+                                       1, **kw)
+        assert torch.equal(part, full[:, j0:j1])
+    again = rec._backproject_matrix(x, ang, 97.6, 1, **kw)
+    assert torch.equal(full, again)
+    yy, xx = np.mgrid[:200, :200] - 100
+    outside = torch.from_numpy(xx ** 2 + yy ** 2 > 90 ** 2).cuda()
+    assert not full.permute(1, 0, 2)[:, outside].any()
+
+
+def test_scales_and_special_samples():
+    """Slices of any magnitude keep their relative error; an all-zero slice
+    gives zeros; slices with inf, NaN or huge samples are exactly the vector
+    kernel's and leave their neighbours untouched."""
+    import torch
+    from algotom_amd.rec import reconstruction as rec
+    x, ang = _case(96, 140, 12, np.pi, 5)
+    x[:, 1] *= 1e-38
+    x[:, 2] *= 1e25
+    x[:, 3] = 0
+    x[:, 4, 1:] = 0          # one sample among zeros
+    clean = rec._backproject_matrix(x, ang, 47.2, 1)
+    ref = rec._backproject_stack(x, ang, 47.2, 0)
+    for j in (0, 1, 2, 4):
+        scale = ref[:, j].double().abs().max()
+        assert _rel(clean[:, j].double() / scale,
+                    ref[:, j].double() / scale) <= 5e-7, j
+    assert not clean[:, 3].any()
+    y = x.clone()
+    y[7, 6, 40] = float("inf")
+    y[9, 8, 11] = float("nan")
+    y[3, 9, 50] = 3e38
+    got = rec._backproject_matrix(y, ang, 47.2, 1)
+    vec = rec._backproject_stack(y, ang, 47.2, 1)
+    for j in range(12):
+        want = vec[:, j] if j in (6, 8, 9) else clean[:, j]
+        assert np.array_equal(got[:, j].cpu().numpy(), want.cpu().numpy(),
+                              equal_nan=True), j
+
+
+def test_fbp_dispatch_and_graph_replay():
+    """fbp_reconstruction takes the matrix path by its rule, a batch member
+    gets the single call's bits, also from a replayed graph."""
+    import torch
+    from algotom_amd.rec import batch, reconstruction as rec
+    rng = np.random.default_rng(2)
+    sinos = [rng.uniform(0.1, 1, (131, 6, 90)).astype(np.float32),
+             rng.uniform(0.1, 1, (60, 5, 64)).astype(np.float32),
+             rng.uniform(0.1, 1, (131, 90)).astype(np.float32)]
+    assert rec._matrix_stack(131, 6, 90, 1, torch.float32)
+    assert not rec._matrix_stack(60, 5, 64, 1, torch.float32)
+    plan = batch.BatchFBP([s.shape for s in sinos], [44.2, 31.0, 45.0],
+                          apply_log=True)
+    plan.load(sinos)
+    plan.capture()
+    for _ in range(3):
+        torch.randn(1 << 18, device="cuda").sum().item()
+        for o in plan.outputs:
+            o.fill_(7.0)
+        plan.run()
+        torch.cuda.synchronize()
+        for s, c, g in zip(sinos, [44.2, 31.0, 45.0], plan.results()):
+            ref = rec.fbp_reconstruction(s.copy(), c, apply_log=True)
+            assert np.array_equal(g, ref), s.shape
