@@ -47,34 +47,58 @@ struct StitchImages {
 
 // factors[2*j] = mean of the first image's overlap, factors[2*j+1] = mean of
 // the second image's overlap (slice j), float64 sums rounded to float32.
-__global__ __launch_bounds__(kThreads) void stitch_means_kernel(
+// One workgroup per slice: a wave sums every 16th row, lanes along the
+// overlap, so no lane divides an element index; a wave keeps 8 independent
+// loads in flight (the 16 x 901 x 3596 volume call 21.6 -> 20.5 ms, its means
+// 0.97 ms before with 256 threads and a 64-bit division per element).
+constexpr int kMeanThreads = 1024;
+__global__ __launch_bounds__(kMeanThreads) void stitch_means_kernel(
     StitchImages im, int nslice, int ncol, int nrow_180, int overlap,
     int side, float* __restrict__ factors) {
-    __shared__ double red[2][kThreads];
+    constexpr int kWaves = kMeanThreads / 64, kRows = 4;
+    __shared__ double red[2][kWaves];
     const int j = blockIdx.x;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     // side 1: mean(img1[:, -ov:]), mean(img2[:, :ov]); side 0:
     // mean(img1[:, :ov]), mean(img2[:, -ov:]) (image coordinates)
     const int c1 = side == 1 ? ncol - overlap : 0;
     const int c2 = side == 1 ? 0 : ncol - overlap;
     const long long n = (long long)nrow_180 * overlap;
-    double s1 = 0.0, s2 = 0.0;
-    for (long long e = tid; e < n; e += kThreads) {
-        const int r = (int)(e / overlap), k = (int)(e % overlap);
-        const size_t row = (size_t)r * nslice + j;
-        s1 += (double)im.at1(row, c1 + k, ncol);
-        s2 += (double)im.at2(row, c2 + k, ncol);
-    }
-    red[0][tid] = s1;
-    red[1][tid] = s2;
-    __syncthreads();
-    for (int w = kThreads / 2; w > 0; w >>= 1) {
-        if (tid < w) {
-            red[0][tid] += red[0][tid + w];
-            red[1][tid] += red[1][tid + w];
+    double s1[kRows] = {}, s2[kRows] = {};
+    for (int r0 = wv; r0 < nrow_180; r0 += kWaves * kRows)
+        for (int k = lane; k < overlap; k += 64) {
+            float v1[kRows], v2[kRows];
+#pragma unroll
+            for (int u = 0; u < kRows; ++u) {
+                const int r = r0 + u * kWaves;
+                const size_t row = (size_t)min(r, nrow_180 - 1) * nslice + j;
+                v1[u] = im.at1(row, c1 + k, ncol);
+                v2[u] = im.at2(row, c2 + k, ncol);
+            }
+#pragma unroll
+            for (int u = 0; u < kRows; ++u) {
+                const bool on = r0 + u * kWaves < nrow_180;
+                s1[u] += on ? (double)v1[u] : 0.0;
+                s2[u] += on ? (double)v2[u] : 0.0;
+            }
         }
-        __syncthreads();
+    double t1 = (s1[0] + s1[1]) + (s1[2] + s1[3]);
+    double t2 = (s2[0] + s2[1]) + (s2[2] + s2[3]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        t1 += __shfl_xor(t1, o);
+        t2 += __shfl_xor(t2, o);
     }
+    if (lane == 0) {
+        red[0][wv] = t1;
+        red[1][wv] = t2;
+    }
+    __syncthreads();
+    if (tid == 0)
+        for (int w = 1; w < kWaves; ++w) {
+            red[0][0] += red[0][w];
+            red[1][0] += red[1][w];
+        }
     if (tid == 0) {
         factors[2 * j] = (float)(red[0][0] / (double)n);
         factors[2 * j + 1] = (float)(red[1][0] / (double)n);
@@ -365,7 +389,7 @@ int stitch_images(const float* img1, const float* img2, int flip2,
                   int wdtype, float* factors, float* out, hipStream_t s) {
     const StitchImages im{img1, img2, flip2};
     if (norm) {
-        hipLaunchKernelGGL(stitch_means_kernel, dim3(nslice), dim3(kThreads),
+        hipLaunchKernelGGL(stitch_means_kernel, dim3(nslice), dim3(kMeanThreads),
                            0, s, im, nslice, ncol, nrow_180, overlap, side,
                            factors);
         const int st = check_hip(hipGetLastError(), "stitch_means_kernel");
