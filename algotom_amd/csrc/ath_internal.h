@@ -109,6 +109,17 @@ struct BpArgs {
     unsigned above;
 };
 
+// Whether the mask removes every pixel of the TX x TY tile at (x0, y0).
+template <int TX, int TY>
+__device__ __forceinline__ bool tile_masked(const BpArgs& a, int x0, int y0) {
+    if (!a.use_mask) return false;
+    const int xl = x0 - a.mask_c, xh = xl + TX - 1;
+    const int yl = y0 - a.mask_c, yh = yl + TY - 1;
+    const long long dx = xl > 0 ? xl : (xh < 0 ? xh : 0);
+    const long long dy = yl > 0 ? yl : (yh < 0 ? yh : 0);
+    return !((double)(dx * dx + dy * dy) <= a.mask_r2);
+}
+
 // sb / py <= 0 select the default tile configuration
 int back_projection(const BpArgs& a, int sino_dtype, int acc, int sb, int py,
                     hipStream_t stream);

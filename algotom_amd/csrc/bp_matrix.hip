@@ -319,16 +319,7 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
         for (int g = 0; g < SG; ++g) acc[i][g] = float4_t{0, 0, 0, 0};
 
     // a tile whose every pixel the mask removes needs no sums
-    bool masked = false;
-    if (a.use_mask) {
-        const int xl = x0 - a.mask_c, xh = x0 + TL::X - 1 - a.mask_c;
-        const int yl = y0 - a.mask_c, yh = y0 + TL::Y - 1 - a.mask_c;
-        const long long dx = xl > 0 ? xl : (xh < 0 ? xh : 0);
-        const long long dy = yl > 0 ? yl : (yh < 0 ? yh : 0);
-        masked = !((double)(dx * dx + dy * dy) <= a.mask_r2);
-    }
-
-    if (!masked) {
+    if (!tile_masked<TL::X, TL::Y>(a, x0, y0)) {
         // selectors of the byte permutation that places (1 - w, w) at columns
         // d, d + 1 of the window's 8: entry d <= 6, one word per column
         // pair; entry 7 places nothing (pixels out of range)
