@@ -495,6 +495,256 @@ __device__ void fft_big_forward(double2* buf, double2* scratch, int N,
     __syncthreads();
 }
 
+// ---- transforms held in registers, 16 points per thread ------------------
+// M = 16 * 16 * R points (R = 4, 8, 16), NT = M / 16 threads.  Forward,
+// decimation in frequency: three register passes (16, 16, R points) with one
+// LDS exchange between two of them; the bins end up in digit-reversed places,
+// which the inverse (the same steps backwards) takes as they are.  With
+//   n = j + r NT,  j = j2 + r2 R   and   k = k1 + 16 k2 + 256 k3
+// thread t holds x[t + r NT] on entry, then (k1, j2) = (t / R, t % R) with
+// all r2, then the items k1 + 16 k2 = t + u NT, u < U = 16 / R, with all j2,
+// i.e. the bins k = t + u NT + 256 k3: tables and partners M - k are read in
+// order.
+//
+// Real and imaginary parts are exchanged one after the other through the same
+// doubles: half the LDS of whole values lets three waves instead of two share
+// a SIMD, which gains more than the further barriers cost (a filtered row of
+// 2560 columns per CU: 8.1 us with whole values, 7.5 us so).  Layouts in
+// doubles (32 lanes cover the 64 banks): [k1][j], then [k1][k2][j2 ^ (k1 /
+// U)], both with R doubles of padding per k1; at R = 16 no access has a bank
+// conflict, at R = 4 and 8 some reads of the second take a second cycle (5%
+// of the LDS cycles).
+constexpr int pos16(int k) { return 4 * (k & 3) + (k >> 2); }
+
+// 16-point DFT, natural order in, value k out at pos16(k)
+template <int DIR>
+__device__ __forceinline__ void dft16(double2 (&v)[16]) {
+    constexpr double c1 = 0.92387953251128675613, s1 = 0.38268343236508977173;
+    constexpr double h = 0.70710678118654752440;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        dft4<DIR>(v[q], v[q + 4], v[q + 8], v[q + 12]);
+    // v[q + 4 p] *= W16^(q p); W16 = exp(-i pi / 8) forward
+    const auto tw = [](double2 a, double c, double s) {
+        return cmul(a, make_double2(c, DIR < 0 ? -s : s));
+    };
+    v[5] = tw(v[5], c1, s1);
+    v[9] = tw(v[9], h, h);
+    v[13] = tw(v[13], s1, c1);
+    v[6] = tw(v[6], h, h);
+    v[10] = rot<DIR>(v[10]);
+    v[14] = tw(v[14], -h, h);
+    v[7] = tw(v[7], s1, c1);
+    v[11] = tw(v[11], -h, h);
+    v[15] = tw(v[15], -c1, -s1);
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+        dft4<DIR>(v[4 * p], v[4 * p + 1], v[4 * p + 2], v[4 * p + 3]);
+}
+
+// v[at(k)] *= w^k (conjugated for the inverse), k = 1 .. 15
+template <int DIR, typename At>
+__device__ __forceinline__ void twiddle16(double2 (&v)[16], double2 w, At at) {
+    if (DIR > 0) w = conjg(w);
+    const double2 w2 = cmul(w, w), w3 = cmul(w2, w), w4 = cmul(w2, w2);
+    v[at(1)] = cmul(v[at(1)], w);
+    v[at(2)] = cmul(v[at(2)], w2);
+    v[at(3)] = cmul(v[at(3)], w3);
+    double2 b = w4;
+#pragma unroll
+    for (int q = 4; q < 16; q += 4) {
+        v[at(q)] = cmul(v[at(q)], b);
+        v[at(q + 1)] = cmul(v[at(q + 1)], cmul(b, w));
+        v[at(q + 2)] = cmul(v[at(q + 2)], cmul(b, w2));
+        v[at(q + 3)] = cmul(v[at(q + 3)], cmul(b, w3));
+        b = cmul(b, w4);
+    }
+}
+
+// exp(-i pi n / 16), 0 <= n < 16
+constexpr double2 unit32(int n) {
+    constexpr double c[9] = {1.0, 0.98078528040323044913,
+                             0.92387953251128675613, 0.83146961230254523708,
+                             0.70710678118654752440, 0.55557023301960222474,
+                             0.38268343236508977173, 0.19509032201612826785,
+                             0.0};
+    return n <= 8 ? double2{c[n], -c[8 - n]} : double2{-c[16 - n], -c[n - 8]};
+}
+
+template <int R>
+struct RegFft {
+    static constexpr int M = 256 * R, NT = M / 16, U = 16 / R;
+    static constexpr int kS = 16 * R + R;     // entries per k1, both layouts
+    static constexpr int kEntries = 16 * kS;
+    static_assert(kEntries >= M);
+    static constexpr size_t kLds = kEntries * sizeof(double);
+
+    static __device__ __forceinline__ int at1(int k1, int j) {
+        return k1 * kS + j;
+    }
+    static __device__ __forceinline__ int at2(int k1, int k2, int j2) {
+        return k1 * kS + k2 * R + (j2 ^ ((k1 / U) & (R - 1)));
+    }
+
+    // what thread t takes from the length-2M table
+    struct Bases {
+        double2 first, second, w[U];
+    };
+    static __device__ __forceinline__ Bases bases(
+        const double2* __restrict__ tw) {
+        const int t = threadIdx.x;
+        Bases b{tw[2 * t], tw[32 * (t % R)], {}};
+#pragma unroll
+        for (int u = 0; u < U; ++u) b.w[u] = tw[t + u * NT];
+        return b;
+    }
+
+    // register of bin k3 of item u
+    static constexpr int slot(int u, int k3) {
+        return u * R + (R == 16 ? pos16(k3) : k3);
+    }
+
+    // v[from(i)] to place to(i) of the buffer, then place at(i) to v[i].
+    // The buffer is free on entry and on return.
+    template <typename From, typename To, typename At>
+    static __device__ __forceinline__ void exchange(double2 (&v)[16],
+                                                    double* d, From from,
+                                                    To to, At at) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) d[to(i)] = v[from(i)].x;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i].x = d[at(i)];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) d[to(i)] = v[from(i)].y;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i].y = d[at(i)];
+        __syncthreads();
+    }
+
+    // t: the thread.  v: x[t + r NT] in; item u's bin k3 out at slot(u, k3).
+    static __device__ __forceinline__ void forward(int t, double2 (&v)[16],
+                                                   double* d,
+                                                   const Bases& tb) {
+        const int k1 = t / R, j2 = t % R;
+        const auto pos = [](int k) { return pos16(k); };
+        dft16<-1>(v);
+        twiddle16<-1>(v, tb.first, pos);
+        exchange(v, d, pos, [&](int k) { return at1(k, t); },
+                 [&](int r) { return at1(k1, j2 + r * R); });
+        dft16<-1>(v);
+        twiddle16<-1>(v, tb.second, pos);
+        exchange(v, d, pos, [&](int k) { return at2(k1, k, j2); },
+                 [&](int i) {
+                     const int l = t + (i / R) * NT;
+                     return at2(l & 15, l >> 4, i % R);
+                 });
+        last<-1>(v);
+    }
+
+    // the R-point transforms of the U items
+    template <int DIR>
+    static __device__ __forceinline__ void last(double2 (&v)[16]) {
+        if constexpr (R == 16) {
+            dft16<DIR>(v);
+        } else if constexpr (R == 8) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                double2 a[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) a[q] = v[8 * u + q];
+                dft8<DIR>(a);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[8 * u + q] = a[q];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                dft4<DIR>(v[4 * u], v[4 * u + 1], v[4 * u + 2], v[4 * u + 3]);
+        }
+    }
+
+    // forward backwards: item u's bin k3 in at u R + k3, x[t + r NT] out at
+    // pos16(r)
+    static __device__ __forceinline__ void inverse(int t, double2 (&v)[16],
+                                                   double* d,
+                                                   const Bases& tb) {
+        const int k1 = t / R, j2 = t % R;
+        const auto same = [](int i) { return i; };
+        last<1>(v);
+        exchange(v, d, [](int i) { return slot(i / R, i % R); },
+                 [&](int i) {
+                     const int l = t + (i / R) * NT;
+                     return at2(l & 15, l >> 4, i % R);
+                 },
+                 [&](int k) { return at2(k1, k, j2); });
+        twiddle16<1>(v, tb.second, same);
+        dft16<1>(v);
+        exchange(v, d, [](int r) { return pos16(r); },
+                 [&](int r) { return at1(k1, j2 + r * R); },
+                 [&](int k) { return at1(k, t); });
+        twiddle16<1>(v, tb.first, same);
+        dft16<1>(v);
+    }
+
+    // The kernel product of the packed real row between the two transforms.
+    // A thread's bins k with k3 < R/2 and their partners M - k, which another
+    // thread holds at k3 >= R/2, are one piece of work: the upper halves go
+    // over to the threads of the lower ones and come back through the
+    // buffer.  k = 0 is its own partner, and so is k = M/2, which is sent to
+    // it in its place.
+    // v: slot(u, k3) in, u R + k3 out.  G: the kernel's half spectrum (M + 1
+    // values).
+    static __device__ __forceinline__ void product(
+        int t, double2 (&v)[16], double* d, const Bases& tb,
+        const double2* __restrict__ G) {
+        constexpr int H = R / 2;
+        double2* buf = reinterpret_cast<double2*>(d);  // k - M/2
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k3 = H; k3 < R; ++k3)
+                buf[t + u * NT + 256 * (k3 - H)] = v[slot(u, k3)];
+        __syncthreads();
+        double2 o[8];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int k3 = 0; k3 < H; ++k3) {
+                const int k = t + u * NT + 256 * k3;
+                const int p = u == 0 && k3 == 0 && t == 0 ? M / 2 : M - k;
+                const double2 zk = v[slot(u, k3)];
+                const double2 zp = buf[p - M / 2];
+                double2 zm = u == 0 && k3 == 0 && t == 0 ? zk : zp;
+                zm = conjg(zm);
+                // W_2M^k = W_2M^(t + u NT) exp(-i pi k3 / R)
+                const double2 w = cmul(tb.w[u], unit32(k3 * (16 / R)));
+                // 2 X[k] = e + w o, 2 conj X[M-k] = e - w o
+                const double2 e = cadd(zk, zm);
+                const double2 wo = cmul(w, rot<-1>(csub(zk, zm)));
+                const double2 a = cmul(cadd(e, wo), G[k]);
+                const double2 b = cmul(csub(e, wo), conjg(G[M - k]));
+                const double2 f = rot<1>(cmul(conjg(w), csub(a, b)));
+                const double2 g = cadd(a, b);
+                o[u * H + k3] = cscale(cadd(g, f), 0.25);
+                double2 q = conjg(cscale(csub(g, f), 0.25));
+                if (u == 0 && k3 == 0 && t == 0) q = cmul(zp, conjg(G[M / 2]));
+                buf[p - M / 2] = q;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k3 = 0; k3 < R; ++k3)
+                v[u * R + k3] = k3 < H ? o[u * H + k3]
+                                       : buf[t + u * NT + 256 * (k3 - H)];
+        __syncthreads();
+    }
+};
+
 // Z = FFT_M(x[2n] + i x[2n+1]) -> X[k] = rfft_L(x)[k] for k and M-k.
 __device__ __forceinline__ void split_real(double2 zk, double2 zm, double2 wk,
                                            double2& xk, double2& xm) {

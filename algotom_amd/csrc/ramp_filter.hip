@@ -23,29 +23,46 @@ constexpr int kThreads = 256;
 
 // Row kernels by size class CLS = maxb_for(M) (the butterflies a 256-thread
 // workgroup would give each thread): the workgroup's thread count and the
-// butterflies per thread actually used.  Larger transforms get more threads
-// (more waves per SIMD to hide LDS latency) at two butterflies each:
-// M = 4096 as 512 threads (two workgroups of 80 KB per CU), M = 8192 as 1024
-// threads (one workgroup of 128 KB per CU).
+// butterflies per thread actually used: M = 8192 as 1024 threads at two
+// butterflies each (one workgroup of 128 KB per CU).
 template <int CLS> struct RowCfg { static constexpr int maxb = CLS, nt = 256; };
-template <> struct RowCfg<4> { static constexpr int maxb = 2, nt = 512; };
 template <> struct RowCfg<8> { static constexpr int maxb = 2, nt = 1024; };
+// M = 1024, 2048 and 4096 (rows of about 400 to 3900 columns) stay in
+// registers (RegFft, classes kRegs1024, 2 and 4): 4 exchanges through LDS for
+// the two transforms of a row instead of 16 passes of a row through LDS and
+// back, and half of the product's reads of the kernel's spectrum.  What
+// bounds it is float64 arithmetic (2170 vector instructions per wave and row,
+// issued in 58% of the cycles at M = 4096).  115264 float32 rows: of 2560
+// columns 5.56 -> 3.24 ms (with the logarithm 6.15 -> 4.1 ms), of 1200
+// columns 2.58 -> 1.35 ms, of 600 columns 1.42 -> 0.97 ms.  Below M = 1024 a row is
+// less than a wave of 16 points per thread; M = 8192 would be 32 points per
+// thread.
+constexpr int kRegs1024 = 3;
+template <> struct RowCfg<kRegs1024> : RegFft<4> {
+    static constexpr int nt = NT;
+};
+template <> struct RowCfg<2> : RegFft<8> { static constexpr int nt = NT; };
+template <> struct RowCfg<4> : RegFft<16> { static constexpr int nt = NT; };
+template <int CLS>
+constexpr bool kInRegs = CLS == kRegs1024 || CLS == 2 || CLS == 4;
+// waves per SIMD that the registers are divided for
+template <int CLS> constexpr int kRowWaves = kInRegs<CLS> ? 3 : 1;
+
+// -log of a sample of type Tin: -np.log of a float32 array is float32
+// (reconstruction.py:436)
+template <typename Tin>
+__device__ __forceinline__ double neg_log(double x) {
+    if constexpr (std::is_same_v<Tin, float>)
+        return (double)neg_log_f32((float)x);
+    else
+        return -log(x);
+}
 
 template <typename Tin>
 __device__ __forceinline__ double load_sample(const Tin* row, int src,
-                                              int apply_log);
-template <>
-__device__ __forceinline__ double load_sample<float>(const float* row, int src,
-                                                     int apply_log) {
-    const float x = row[src];
-    // -np.log of a float32 array is float32 (reconstruction.py:436)
-    return apply_log ? (double)neg_log_f32(x) : (double)x;
-}
-template <>
-__device__ __forceinline__ double load_sample<double>(const double* row,
-                                                      int src, int apply_log) {
-    const double x = row[src];
-    return apply_log ? -log(x) : x;
+                                              int apply_log) {
+    const double x = (double)row[src];
+    return apply_log ? neg_log<Tin>(x) : x;
 }
 
 // ---- numpy.pad's value modes (ATH_PAD_LINEAR_RAMP .. ATH_PAD_MINIMUM) ----
@@ -210,6 +227,73 @@ __device__ __forceinline__ void spectral_pair(double2& zk, double2& zm, int k,
     merge_pair(cmul(xk, G[k]), cmul(xm, G[M - k]), k, M, tw, zk, zm);
 }
 
+// Transpose of the padding: z[n], n in [0, W) in LDS; out[c] = sum of z[n]
+// over the n whose pad source is c (the interior n = pad + c, plus folded
+// pad samples).
+template <int NT, typename Tout>
+__device__ __forceinline__ void fold_row(const double* z, Tout* dst, int ncol,
+                                         int pad, int pad_mode) {
+    const int width = ncol + 2 * pad;
+    for (int c = threadIdx.x; c < ncol; c += NT) {
+        double v = z[pad + c];
+        if (pad_mode == ATH_PAD_EDGE) {
+            if (c == 0)
+                for (int n = 0; n < pad; ++n) v += z[n];
+            if (c == ncol - 1)
+                for (int n = pad + ncol; n < width; ++n) v += z[n];
+        } else if (pad_mode != ATH_PAD_CONSTANT) {
+            for (int n = 0; n < pad; ++n)
+                if (pad_source(n - pad, ncol, pad_mode) == c) v += z[n];
+            for (int n = pad + ncol; n < width; ++n)
+                if (pad_source(n - pad, ncol, pad_mode) == c) v += z[n];
+        }
+        store_elem(dst + c, v);
+    }
+}
+
+// A row of ncol elements behind a buffer descriptor: loads outside it are 0
+// and stores outside it are dropped, without a branch.  The offset is
+// clamped first, so that no address wraps.
+template <typename T>
+struct RowBuffer {
+    __amdgpu_buffer_rsrc_t rsrc;
+    unsigned bytes;
+    __device__ __forceinline__ RowBuffer(T* row, int ncol)
+        : bytes((unsigned)ncol * (unsigned)sizeof(T)) {
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<std::remove_const_t<T>*>(row), 0, bytes, 0x00020000);
+    }
+    __device__ __forceinline__ unsigned offset(int c) const {
+        return min((unsigned)c, bytes / (unsigned)sizeof(T)) *
+               (unsigned)sizeof(T);
+    }
+    __device__ __forceinline__ std::remove_const_t<T> load(int c) const {
+        if constexpr (sizeof(T) == 8)
+            return __builtin_bit_cast(
+                double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, offset(c),
+                                                             0, 0));
+        else
+            return __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, offset(c),
+                                                            0, 0));
+    }
+    __device__ __forceinline__ void store(int c, double x) const {
+        T e;
+        store_elem(&e, x);
+        if constexpr (sizeof(T) == 8) {
+            typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, e),
+                                                  rsrc, offset(c), 0, 0);
+        } else if constexpr (sizeof(T) == 4) {
+            __builtin_amdgcn_raw_buffer_store_b32(
+                __builtin_bit_cast(unsigned, e), rsrc, offset(c), 0, 0);
+        } else {
+            __builtin_amdgcn_raw_buffer_store_b16(
+                __builtin_bit_cast(unsigned short, e), rsrc, offset(c), 0, 0);
+        }
+    }
+};
+
 // Filters one row in LDS buffer `buf` (M double2): pad, rfft, multiply by
 // the kernel half spectrum G, irfft, crop into dst.  All 256 threads.
 // ADJ: the transpose of the filter -- the row is embedded with zeros
@@ -221,10 +305,10 @@ template <int MAXB, typename Tin, typename Tout, bool ADJ = false>
 __device__ __forceinline__ void filter_row(
     double2* buf, const double2* tq, const Tin* __restrict__ src_row,
     Tout* __restrict__ dst, int ncol, int pad, int pad_mode, int apply_log,
-    const double2* __restrict__ tw, const double2* __restrict__ G, int M) {
-    constexpr bool QT = MAXB <= 4;  // quarter table in LDS (M <= 4096)
-    constexpr int B = RowCfg<MAXB>::maxb, NT = RowCfg<MAXB>::nt;
-    const int tid = threadIdx.x;
+    const double2* __restrict__ tw, const double2* __restrict__ G, int M,
+    const Log32Table* tab = nullptr) {
+    constexpr int NT = RowCfg<MAXB>::nt;
+    int tid = threadIdx.x;
     const int width = ncol + 2 * pad;
     PadVals pv{0.0, 0.0};
     bool value_mode = false;
@@ -234,6 +318,110 @@ __device__ __forceinline__ void filter_row(
             pv = row_pad_values<NT, Tin>(buf, src_row, ncol, pad, pad_mode,
                                          apply_log);
     }
+    if constexpr (kInRegs<MAXB>) {
+        using F = RowCfg<MAXB>;
+        // tables, addresses and bounds are formed again for every row: held
+        // over the loop they would take more registers than there are
+        asm volatile("" : "+s"(G), "+v"(tid));
+        const typename F::Bases tb = F::bases(tw);
+        // packed, padded, zero-extended row: v[r] = (p[2n], p[2n+1]),
+        // n = tid + r NT; all loads of the row itself in flight at once, a
+        // column outside the row read as 0 by the buffer's bounds
+        double* y = reinterpret_cast<double*>(buf);
+        Tin* z = reinterpret_cast<Tin*>(buf);
+        const RowBuffer<const Tin> in(src_row, ncol);
+        const auto inside = [&](int c) {
+            return (unsigned)c < (unsigned)ncol;
+        };
+        Tin x[32];
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+            x[i] = in.load(2 * (tid + (i >> 1) * NT) + (i & 1) - pad);
+        if (!ADJ && apply_log) {
+            // a rolled loop over the row (ncol <= M samples) in LDS
+            asm volatile("" : "+v"(tid));
+#pragma unroll
+            for (int i = 0; i < 32; ++i) {
+                const int c = 2 * (tid + (i >> 1) * NT) + (i & 1) - pad;
+                if (2 * (i >> 1) * NT < pad + ncol)
+                    if (inside(c)) z[c] = x[i];
+            }
+            __syncthreads();
+            for (int c = tid; c < ncol; c += NT) {
+                if constexpr (std::is_same_v<Tin, float>)
+                    z[c] = neg_log_f32(z[c], *tab);
+                else
+                    z[c] = -log(z[c]);
+            }
+            __syncthreads();
+            asm volatile("" : "+v"(tid));
+#pragma unroll
+            for (int i = 0; i < 32; ++i) {
+                const int c = 2 * (tid + (i >> 1) * NT) + (i & 1) - pad;
+                const Tin l = z[min((unsigned)c, (unsigned)ncol - 1)];
+                x[i] = inside(c) ? l : (Tin)0;
+            }
+            __syncthreads();
+        }
+        if (!ADJ && pad_mode != ATH_PAD_CONSTANT) {
+            // the samples of the two sides go through the pad map one by one
+            asm volatile("" : "+v"(tid));
+            for (int i = tid; i < 2 * pad; i += NT)
+                z[i] = (Tin)padded_sample<Tin, ADJ>(
+                    src_row, i < pad ? i : ncol + i, width, ncol, pad,
+                    pad_mode, apply_log, value_mode, pv);
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int lo = 2 * r * NT, hi = lo + 2 * NT;
+                if (lo < pad || (lo < width && hi > pad + ncol)) {
+#pragma unroll
+                    for (int i = 2 * r; i < 2 * r + 2; ++i) {
+                        const int k = 2 * (tid + r * NT) + (i & 1);
+                        if (k < width && !inside(k - pad))
+                            x[i] = z[k < pad ? k : k - ncol];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        asm volatile("" : "+v"(tid));
+        double2 v[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            v[r] = make_double2((double)x[2 * r], (double)x[2 * r + 1]);
+        F::forward(tid, v, y, tb);
+        F::product(tid, v, y, tb, G);
+        F::inverse(tid, v, y, tb);
+        if constexpr (!ADJ) {
+            const RowBuffer<Tout> to(dst, ncol);
+            const int off = width + pad;
+            asm volatile("" : "+v"(tid));
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int c = 2 * (tid + r * NT) - off;
+                if (2 * (r + 1) * NT <= off || 2 * r * NT >= off + ncol)
+                    continue;
+                to.store(c, v[pos16(r)].x);
+                to.store(c + 1, v[pos16(r)].y);
+            }
+            return;
+        } else {
+            // the W outputs that fold back, z[n] = y[W + n]
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int n = 2 * (tid + r * NT) - width;
+                if (n >= 0 && n < width) y[n] = v[pos16(r)].x;
+                if (n + 1 >= 0 && n + 1 < width) y[n + 1] = v[pos16(r)].y;
+            }
+            __syncthreads();
+            fold_row<NT>(y, dst, ncol, pad, pad_mode);
+            __syncthreads();  // buf free for the caller's next row
+            return;
+        }
+    } else {
+    constexpr bool QT = MAXB == 1;  // quarter table in LDS (M <= 512)
+    constexpr int B = RowCfg<MAXB>::maxb;
     // packed, padded, zero-extended row: buf[n] = (p[2n], p[2n+1])
     for (int n = tid; n < M; n += NT)
         buf[n] = make_double2(
@@ -254,6 +442,7 @@ __device__ __forceinline__ void filter_row(
     }
     __syncthreads();
     lds_fft<1, B, QT, NT, 1, true>(buf, M, tw, tq);
+    }
 
     const double* y = reinterpret_cast<const double*>(buf);
     if (!ADJ) {
@@ -261,66 +450,77 @@ __device__ __forceinline__ void filter_row(
         for (int c = tid; c < ncol; c += NT)
             store_elem(dst + c, y[off + c]);
     } else {
-        // z[n] = y[W + n], n in [0, W); out[c] = sum of z[n] over the n whose
-        // pad source is c (the interior n = pad + c, plus folded pad samples)
-        const double* z = y + width;
-        for (int c = tid; c < ncol; c += NT) {
-            double v = z[pad + c];
-            if (pad_mode == ATH_PAD_EDGE) {
-                if (c == 0)
-                    for (int n = 0; n < pad; ++n) v += z[n];
-                if (c == ncol - 1)
-                    for (int n = pad + ncol; n < width; ++n) v += z[n];
-            } else if (pad_mode != ATH_PAD_CONSTANT) {
-                for (int n = 0; n < pad; ++n)
-                    if (pad_source(n - pad, ncol, pad_mode) == c) v += z[n];
-                for (int n = pad + ncol; n < width; ++n)
-                    if (pad_source(n - pad, ncol, pad_mode) == c) v += z[n];
-            }
-            store_elem(dst + c, v);
-        }
+        fold_row<NT>(y + width, dst, ncol, pad, pad_mode);
     }
     __syncthreads();  // buf free for the caller's next row
 }
 
-// LDS of the row kernels: the row (M complex) then, for M <= 4096, the
-// quarter twiddle table (M/4 complex).
+// The buffer in front of the log table (M = 1024 .. 4096): the exchange's
+// doubles, and room for the 2 pad samples of the row's two sides: 2 ncol +
+// 3 pad <= 2M leaves up to 4M / 3 of them.
+template <int MAXB>
+constexpr size_t row_buffer_bytes() {
+    constexpr size_t sides = (RowCfg<MAXB>::M * 4 / 3 + 8) & ~size_t{7};
+    return std::max(RowCfg<MAXB>::kLds, sides * sizeof(double));
+}
+
+// LDS of the row kernels: buffer and log table (M = 1024 .. 4096), or the row
+// (M complex) and, for M <= 512, the quarter twiddle table (M/4 complex).
 template <int MAXB>
 constexpr size_t row_lds_bytes(int M) {
-    return (size_t)(M + (MAXB <= 4 ? M / 4 : 0)) * sizeof(double2);
+    if constexpr (kInRegs<MAXB>) {
+        return row_buffer_bytes<MAXB>() + sizeof(Log32Table);
+    } else {
+        return (size_t)(M + (MAXB == 1 ? M / 4 : 0)) * sizeof(double2);
+    }
+}
+
+// the log table behind the exchange buffer (M = 1024 .. 4096)
+template <int MAXB>
+__device__ __forceinline__ Log32Table* row_log_table(double2* buf) {
+    if constexpr (kInRegs<MAXB>)
+        return reinterpret_cast<Log32Table*>(reinterpret_cast<char*>(buf) +
+                                             row_buffer_bytes<MAXB>());
+    else
+        return nullptr;
 }
 
 // Persistent: each workgroup stages the twiddles once, then filters rows
 // blockIdx.x, blockIdx.x + gridDim.x, ... of the (nrow, nslice, ncol) stack.
 template <int MAXB, typename Tin, typename Tout>
-__global__ __launch_bounds__(RowCfg<MAXB>::nt) void ramp_filter_kernel(
+__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>) void ramp_filter_kernel(
     const Tin* __restrict__ sino, Tout* __restrict__ out, size_t rows,
     int nslice, int ncol, int pad, int pad_mode, int apply_log,
     const double2* __restrict__ tw, const double2* __restrict__ spec,
     int nwin, int M) {
     extern __shared__ double2 buf[];
     double2* tq = buf + M;
-    if (MAXB <= 4)  // read after the row's barrier
+    Log32Table* tab = row_log_table<MAXB>(buf);
+    if constexpr (kInRegs<MAXB>) {
+        if (apply_log && std::is_same_v<Tin, float>)
+            stage_log32_table<RowCfg<MAXB>::nt>(tab);
+    } else if (MAXB == 1)  // read after the row's barrier
         stage_quarter<RowCfg<MAXB>::nt>(tq, tw, M);
     for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
         const double2* G =
             spec + (nwin > 1 ? (row / nslice) : 0) * (size_t)(M + 1);
         filter_row<MAXB, Tin, Tout>(buf, tq, sino + row * (size_t)ncol,
                                     out + row * (size_t)ncol, ncol, pad,
-                                    pad_mode, apply_log, tw, G, M);
+                                    pad_mode, apply_log, tw, G, M, tab);
     }
 }
 
 // Transpose of ramp_filter_kernel (float32 in and out), persistent.
 template <int MAXB>
-__global__ __launch_bounds__(RowCfg<MAXB>::nt) void ramp_filter_adjoint_kernel(
+__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>) void ramp_filter_adjoint_kernel(
     const float* __restrict__ in, float* __restrict__ out, size_t rows,
     int nslice, int ncol, int pad, int pad_mode,
     const double2* __restrict__ tw, const double2* __restrict__ spec,
     int nwin, int M) {
     extern __shared__ double2 buf[];
     double2* tq = buf + M;
-    if (MAXB <= 4) stage_quarter<RowCfg<MAXB>::nt>(tq, tw, M);
+    if (MAXB == 1)
+        stage_quarter<RowCfg<MAXB>::nt>(tq, tw, M);
     for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
         const double2* G =
             spec + (nwin > 1 ? (row / nslice) : 0) * (size_t)(M + 1);
@@ -333,12 +533,16 @@ __global__ __launch_bounds__(RowCfg<MAXB>::nt) void ramp_filter_adjoint_kernel(
 // Rows of many stacks sharing the FFT length L = 2M (hence the twiddles),
 // persistent; a row's stack is found by binary search over row_begin.
 template <int MAXB, typename Tin, typename Tout>
-__global__ __launch_bounds__(RowCfg<MAXB>::nt) void ramp_filter_batched_kernel(
+__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>) void ramp_filter_batched_kernel(
     const ath_filter_job* __restrict__ jobs, int njobs, long long total_rows,
     int pad_mode, int apply_log, int M) {
     extern __shared__ double2 buf[];
     double2* tq = buf + M;
-    if (MAXB <= 4)
+    Log32Table* tab = row_log_table<MAXB>(buf);
+    if constexpr (kInRegs<MAXB>) {
+        if (apply_log && std::is_same_v<Tin, float>)
+            stage_log32_table<RowCfg<MAXB>::nt>(tab);
+    } else if (MAXB == 1)
         stage_quarter<RowCfg<MAXB>::nt>(
             tq, static_cast<const double2*>(jobs[0].plan), M);
     for (long long grow = blockIdx.x; grow < total_rows; grow += gridDim.x) {
@@ -357,7 +561,7 @@ __global__ __launch_bounds__(RowCfg<MAXB>::nt) void ramp_filter_batched_kernel(
         filter_row<MAXB, Tin, Tout>(
             buf, tq, static_cast<const Tin*>(jb.sino) + row * (size_t)jb.ncol,
             static_cast<Tout*>(jb.out) + row * (size_t)jb.ncol, jb.ncol,
-            jb.pad, pad_mode, apply_log, tw, G, M);
+            jb.pad, pad_mode, apply_log, tw, G, M, tab);
     }
 }
 
@@ -625,6 +829,7 @@ __global__ __launch_bounds__(kBigRowNT) void kernel_spectrum_big_kernel(
 constexpr int kBigClass = 16;
 inline int filter_class(int M) {
     if (M == 2 * kBigH) return kBigClass;
+    if (M == 1024) return kRegs1024;
     return maxb_for(M);
 }
 
@@ -817,6 +1022,7 @@ int plan_build(const double* taps, int nwin, int width, int fft_len,
     int st = check_hip(hipGetLastError(), "twiddle_kernel launch");
     if (st != ATH_OK) return st;
     switch (filter_class(M)) {
+    case kRegs1024:
     case 1: return launch_spectrum<1>(taps, nwin, width, tw, spec, M, stream);
     case 2: return launch_spectrum<2>(taps, nwin, width, tw, spec, M, stream);
     case 4: return launch_spectrum<4>(taps, nwin, width, tw, spec, M, stream);
@@ -840,6 +1046,9 @@ int ramp_filter_batched(const ath_filter_job* jobs, int njobs,
                         hipStream_t s) {
     switch (filter_class(fft_len / 2)) {
     case 1: return batched_in<1>(in_dtype, out_dtype, jobs, njobs, total_rows,
+                                 fft_len, pad_mode, apply_log, s);
+    case kRegs1024:
+        return batched_in<kRegs1024>(in_dtype, out_dtype, jobs, njobs, total_rows,
                                  fft_len, pad_mode, apply_log, s);
     case 2: return batched_in<2>(in_dtype, out_dtype, jobs, njobs, total_rows,
                                  fft_len, pad_mode, apply_log, s);
@@ -903,6 +1112,9 @@ int ramp_filter_adjoint(const float* in, int nrow, int nslice, int ncol,
     switch (maxb_for(fft_len / 2)) {
     case 1: return launch_adjoint<1>(in, nrow, nslice, ncol, pad, pad_mode,
                                      plan, fft_len, nwin, out, s);
+    case kRegs1024:
+        return launch_adjoint<kRegs1024>(in, nrow, nslice, ncol, pad, pad_mode,
+                                     plan, fft_len, nwin, out, s);
     case 2: return launch_adjoint<2>(in, nrow, nslice, ncol, pad, pad_mode,
                                      plan, fft_len, nwin, out, s);
     case 4: return launch_adjoint<4>(in, nrow, nslice, ncol, pad, pad_mode,
@@ -926,6 +1138,10 @@ int ramp_filter(const void* sino, int in_dtype, int nrow, int nslice,
                                       nslice, ncol, pad, pad_mode, apply_log,
                                       plan, fft_len, nwin, s);
     case 1: return dispatch_in<1>(in_dtype, out_dtype, sino, out, nrow, nslice,
+                                  ncol, pad, pad_mode, apply_log, plan,
+                                  fft_len, nwin, s);
+    case kRegs1024:
+        return dispatch_in<kRegs1024>(in_dtype, out_dtype, sino, out, nrow, nslice,
                                   ncol, pad, pad_mode, apply_log, plan,
                                   fft_len, nwin, s);
     case 2: return dispatch_in<2>(in_dtype, out_dtype, sino, out, nrow, nslice,

@@ -244,3 +244,63 @@ def test_filter_fft_32768_per_row_windows_and_f32():
         ulps = np.abs(got32[i].view(np.int32).astype(np.int64)
                       - r32.view(np.int32).astype(np.int64))
         assert ulps.max() <= 1
+
+
+# the rows held in registers (M = 1024, 2048, 4096): the shortest and longest
+# row of each length (2 ncol + 3 pad just above and at a power of two), no
+# padding, and one column with the most padding
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("ncol,pad", [
+    (400, 75), (799, 150), (1024, 0), (800, 150), (1823, 150), (1, 1364),
+    (1824, 150), (3871, 150), (2501, 3)])
+def test_filter_rows_in_registers(ncol, pad, dtype):
+    """Bar: 1e-12 * max|ref|; a float32 mean may sit one float32 ulp off."""
+    import torch
+    from oracle import fbp_np
+    sino = _rows(3, 2, ncol, ncol + pad).astype(dtype)
+    rng = np.random.default_rng(pad)
+    taps = rng.uniform(-1.0, 1.0, (1, ncol + 2 * pad))
+    spec = np.fft.fftshift(np.fft.fft(taps[0]))
+    for log in (False, True):
+        for mode in ("edge", "reflect", "symmetric", "wrap", "constant",
+                     "linear_ramp", "maximum", "mean", "median", "minimum"):
+            got = _gpu_filter(sino, pad, mode, log, taps, torch.float64)
+            x = sino
+            if log:
+                x = (-np.log(x.astype(np.float64))).astype(dtype)
+            p = np.pad(x, ((0, 0), (0, 0), (pad, pad)), mode=mode)
+            ref = np.fft.ifft(np.fft.fft(p.astype(np.float64))
+                              * np.fft.ifftshift(spec)).real
+            ref = ref[..., pad:pad + ncol]
+            bound = 1e-6 if (mode == "mean" and dtype == "float32") else 1e-12
+            scale = np.linalg.norm(taps) * np.abs(p).max()
+            err = np.abs(got - ref).max()
+            assert err <= bound * scale, (mode, log, err / scale)
+
+
+@pytest.mark.parametrize("ncol", [600, 1200, 2560])
+def test_filter_rows_in_registers_many(ncol):
+    """More rows than workgroups: each workgroup's later rows are the first
+    ones' bits, forwards and in the transpose, one NaN row apart."""
+    import torch
+    from algotom_amd import _native as nat
+    from algotom_amd.rec import autograd
+    dev, pad, rep = nat.device(), 150, 1500
+    few = torch.from_numpy(_rows(5, 1, ncol, 7)).to(dev)
+    few[3, 0, ncol // 2] = float("nan")
+    many = few.repeat(rep, 1, 1)
+    geom = autograd.FBPGeometry(many.shape[0], ncol,
+                                np.linspace(0.0, np.pi, many.shape[0]))
+    from algotom_amd.rec import reconstruction as rec
+    for log in (False, True):
+        for mode in ("edge", "median"):
+            out = rec._filter_stack(many, pad, mode, log, geom.taps,
+                                    torch.float32)
+            assert torch.isnan(out[3::5]).all()
+            out = out.view(rep, 5, ncol)[:, [0, 1, 2, 4]]
+            assert torch.isfinite(out).all()
+            assert torch.equal(out, out[:1].expand_as(out))
+    adj = geom.filter_adjoint(many)
+    adj = adj.view(rep, 5, ncol)[:, [0, 1, 2, 4]]
+    assert torch.isfinite(adj).all()
+    assert torch.equal(adj, adj[:1].expand_as(adj))
