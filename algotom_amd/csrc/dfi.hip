@@ -456,10 +456,10 @@ __global__ __launch_bounds__(NT) void dfi_rows_fwd_kernel(
                     d = d < 0 ? -d : d;
                     if (d <= kK5) {
                         const double h = h5[d];
-                        a1[r].x += h * v1.x;
-                        a1[r].y += h * v1.y;
-                        a2[r].x += h * v2.x;
-                        a2[r].y += h * v2.y;
+                        a1[r].x = fma(h, v1.x, a1[r].x);
+                        a1[r].y = fma(h, v1.y, a1[r].y);
+                        a2[r].x = fma(h, v2.x, a2[r].x);
+                        a2[r].y = fma(h, v2.y, a2[r].y);
                     }
                 }
             }
@@ -478,34 +478,60 @@ __global__ __launch_bounds__(NT) void dfi_rows_fwd_kernel(
 // ---- 4. column prefilter ----------------------------------------------------
 // out[r][c] = sum_t h5[|t|] X[fold_half(r + t)][c]: one column per lane,
 // kColRun consecutive rows per thread (each loaded row feeds every output
-// within kK5 of it).
-constexpr int kColRun = 16;
+// within kK5 of it).  kColStep rows are loaded together; row i of output q
+// takes tap i - kK5 - q, so one step needs kColRun + kColStep - 1 taps, read
+// once from a table in LDS that holds zeros past the half lengths.  What
+// bounds it is the float64 multiply-add, 105 of them (and a few zero taps)
+// per component; with a tap read from LDS for each of them, and a multiply
+// and an add, a 1801 x 2861 slice took 260 us instead of 131 us.  Each XCD
+// (workgroup index mod 8) walks down its own columns, so that the halo rows
+// of one workgroup are in its L2 for the next: 142 us without.
+constexpr int kColRun = 16, kColStep = 8;
+constexpr int kColLoop = (kColRun + 2 * kK5 + kColStep - 1) / kColStep;
 
 __global__ __launch_bounds__(kThreads) void dfi_cols_kernel(
     const double2* __restrict__ X, int rows, int N,
     const double* __restrict__ h5, double2* __restrict__ out) {
-    __shared__ double hs[kK5 + 1];
-    if (threadIdx.x <= kK5) hs[threadIdx.x] = h5[threadIdx.x];
+    // hs[kColRun - 1 + i] = tap i - kK5
+    constexpr int kTaps = kColLoop * kColStep + kColRun;
+    __shared__ double2 hs2[(kTaps + 1) / 2];
+    double* hs = reinterpret_cast<double*>(hs2);
+    for (int k = threadIdx.x; k < kTaps; k += kThreads) {
+        int d = k - (kColRun - 1) - kK5;
+        d = d < 0 ? -d : d;
+        hs[k] = d <= kK5 ? h5[d] : 0.0;
+    }
     __syncthreads();
-    const int c = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int r0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * kColRun;
+    const int ny = (rows + 4 * kColRun - 1) / (4 * kColRun);
+    const int j = blockIdx.x >> 3;
+    const int c = ((j / ny * 8 + (blockIdx.x & 7)) * 64) + (threadIdx.x & 63);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = (j % ny * 4 + wave) * kColRun;
     if (c >= N || r0 >= rows) return;
     double2 acc[kColRun];
 #pragma unroll
     for (int q = 0; q < kColRun; ++q) acc[q] = make_double2(0.0, 0.0);
-    for (int i = 0; i < kColRun + 2 * kK5; ++i) {
-        const int r = fold_half(r0 - kK5 + i, rows);
-        const double2 v = X[(size_t)r * N + c];
+#pragma unroll 1
+    for (int b = 0; b < kColLoop; ++b) {
+        double2 v[kColStep];
 #pragma unroll
-        for (int q = 0; q < kColRun; ++q) {
-            int d = i - kK5 - q;
-            d = d < 0 ? -d : d;
-            if (d <= kK5) {
-                const double h = hs[d];
-                acc[q].x += h * v.x;
-                acc[q].y += h * v.y;
-            }
+        for (int i = 0; i < kColStep; ++i)
+            v[i] = X[(size_t)fold_half(r0 - kK5 + b * kColStep + i, rows) * N +
+                     c];
+        double h[kColRun + kColStep];
+#pragma unroll
+        for (int k = 0; k < kColRun + kColStep; k += 2) {
+            const double2 p = hs2[(b * kColStep + k) / 2];
+            h[k] = p.x;
+            h[k + 1] = p.y;
         }
+#pragma unroll
+        for (int i = 0; i < kColStep; ++i)
+#pragma unroll
+            for (int q = 0; q < kColRun; ++q) {
+                acc[q].x = fma(h[kColRun - 1 + i - q], v[i].x, acc[q].x);
+                acc[q].y = fma(h[kColRun - 1 + i - q], v[i].y, acc[q].y);
+            }
     }
 #pragma unroll
     for (int q = 0; q < kColRun; ++q)
@@ -551,11 +577,11 @@ __device__ __forceinline__ double2 grid_eval(const double2* __restrict__ coef,
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
             const double2 c = crow[cx[j]];
-            rs.x += wx[j] * c.x;
-            rs.y += wx[j] * c.y;
+            rs.x = fma(wx[j], c.x, rs.x);
+            rs.y = fma(wx[j], c.y, rs.y);
         }
-        val.x += wy * rs.x;
-        val.y += wy * rs.y;
+        val.x = fma(wy, rs.x, val.x);
+        val.y = fma(wy, rs.y, val.y);
     }
     return val;
 }
@@ -573,69 +599,77 @@ __device__ __forceinline__ double2 grid_eval(const double2* __restrict__ coef,
 // rounded theta is the same and its knot window the mirror image, conj of
 // its value reuses the first point's 36 coefficients in reversed column
 // order; otherwise it is gathered on its own.
+//
+// A workgroup takes 16 x 16 frequencies, a wave 8 x 8 of them: what bounds it
+// are the cache lines that the 36 gathers touch, and a patch shares them (a
+// line holds 8 coefficients of one angle) where a run of one column of
+// frequencies crosses an angle per lane.  N = 2861, 1801
+// angles: 567 -> 236 us a slice; the tiles of one XCD next to each other gave
+// nothing more.
 __global__ __launch_bounds__(kThreads) void dfi_grid_kernel(
     const double2* __restrict__ coef, int rows, int N,
     double2* __restrict__ T) {
     const int m = (N - 1) / 2;
-    for (int v = blockIdx.y; v <= m; v += gridDim.y) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int tu = (N + 15) / 16, tv = (m + 16) / 16;
+    for (int t = blockIdx.x; t < tu * tv; t += gridDim.x) {
+        const int u = t % tu * 16 + (wave & 1) * 8 + (lane & 7);
+        const int v = t / tu * 16 + (wave >> 1) * 8 + (lane >> 3);
+        if (u >= N || v > m) continue;
         int x = v + m;
         if (x >= N) x -= N;
         const int X = m - x;
-        double2* dst = T + (size_t)v * N;
-        for (int u = blockIdx.x * kThreads + threadIdx.x; u < N;
-             u += gridDim.x * kThreads) {
-            int y = u + m;
-            if (y >= N) y -= N;
-            const int Y = y - m;
-            double2 h = make_double2(0.0, 0.0);
-            if (X * X + Y * Y <= m * m) {
-                double tta, rra, ttb, rrb;
-                grid_coords(rows, N, m, X, Y, tta, rra);
-                grid_coords(rows, N, m, -X, -Y, ttb, rrb);
-                const int s1 = (int)floor(rra) - 2;
-                const int s1b = (int)floor(rrb) - 2;
-                if (tta == ttb && s1b == 2 * m - s1 - 5) {
-                    const int s0 = (int)floor(tta) - 2;
-                    double wa[6], wb[6];
-                    int cx[6];
+        int y = u + m;
+        if (y >= N) y -= N;
+        const int Y = y - m;
+        double2 h = make_double2(0.0, 0.0);
+        if (X * X + Y * Y <= m * m) {
+            double tta, rra, ttb, rrb;
+            grid_coords(rows, N, m, X, Y, tta, rra);
+            grid_coords(rows, N, m, -X, -Y, ttb, rrb);
+            const int s1 = (int)floor(rra) - 2;
+            const int s1b = (int)floor(rrb) - 2;
+            if (tta == ttb && s1b == 2 * m - s1 - 5) {
+                const int s0 = (int)floor(tta) - 2;
+                double wa[6], wb[6];
+                int cx[6];
+#pragma unroll
+                for (int j = 0; j < 6; ++j) {
+                    wa[j] = beta5(rra - (double)(s1 + j));
+                    wb[j] = beta5(rrb - (double)(s1b + 5 - j));
+                    cx[j] = fold_half(s1 + j, N);
+                }
+                double2 sa = make_double2(0.0, 0.0);
+                double2 sb = make_double2(0.0, 0.0);
+#pragma unroll 1
+                for (int i = 0; i < 6; ++i) {
+                    const double wy = beta5(tta - (double)(s0 + i));
+                    const double2* crow =
+                        coef + (size_t)fold_half(s0 + i, rows) * N;
+                    double2 ra = make_double2(0.0, 0.0);
+                    double2 rb = make_double2(0.0, 0.0);
 #pragma unroll
                     for (int j = 0; j < 6; ++j) {
-                        wa[j] = beta5(rra - (double)(s1 + j));
-                        wb[j] = beta5(rrb - (double)(s1b + 5 - j));
-                        cx[j] = fold_half(s1 + j, N);
+                        const double2 c = crow[cx[j]];
+                        ra.x = fma(wa[j], c.x, ra.x);
+                        ra.y = fma(wa[j], c.y, ra.y);
+                        rb.x = fma(wb[j], c.x, rb.x);
+                        rb.y = fma(wb[j], c.y, rb.y);
                     }
-                    double2 sa = make_double2(0.0, 0.0);
-                    double2 sb = make_double2(0.0, 0.0);
-#pragma unroll 1
-                    for (int i = 0; i < 6; ++i) {
-                        const double wy = beta5(tta - (double)(s0 + i));
-                        const double2* crow =
-                            coef + (size_t)fold_half(s0 + i, rows) * N;
-                        double2 ra = make_double2(0.0, 0.0);
-                        double2 rb = make_double2(0.0, 0.0);
-#pragma unroll
-                        for (int j = 0; j < 6; ++j) {
-                            const double2 c = crow[cx[j]];
-                            ra.x += wa[j] * c.x;
-                            ra.y += wa[j] * c.y;
-                            rb.x += wb[j] * c.x;
-                            rb.y += wb[j] * c.y;
-                        }
-                        sa.x += wy * ra.x;
-                        sa.y += wy * ra.y;
-                        sb.x += wy * rb.x;
-                        sb.y += wy * rb.y;
-                    }
-                    // sb = conj of the mirrored frequency's value
-                    h = make_double2(0.5 * (sa.x + sb.x), 0.5 * (sa.y + sb.y));
-                } else {
-                    const double2 a = grid_eval(coef, rows, N, tta, rra);
-                    const double2 b = grid_eval(coef, rows, N, ttb, rrb);
-                    h = make_double2(0.5 * (a.x + b.x), 0.5 * (a.y - b.y));
+                    sa.x = fma(wy, ra.x, sa.x);
+                    sa.y = fma(wy, ra.y, sa.y);
+                    sb.x = fma(wy, rb.x, sb.x);
+                    sb.y = fma(wy, rb.y, sb.y);
                 }
+                // sb = conj of the mirrored frequency's value
+                h = make_double2(0.5 * (sa.x + sb.x), 0.5 * (sa.y + sb.y));
+            } else {
+                const double2 a = grid_eval(coef, rows, N, tta, rra);
+                const double2 b = grid_eval(coef, rows, N, ttb, rrb);
+                h = make_double2(0.5 * (a.x + b.x), 0.5 * (a.y - b.y));
             }
-            dst[u] = h;
         }
+        T[(size_t)v * N + u] = h;
     }
 }
 
@@ -917,8 +951,8 @@ __global__ __launch_bounds__(kThreads) void dfi_rows_fir_kernel(
                     d = d < 0 ? -d : d;
                     if (d <= kK5) {
                         const double h = h5[d];
-                        a[r].x += h * v.x;
-                        a[r].y += h * v.y;
+                        a[r].x = fma(h, v.x, a[r].x);
+                        a[r].y = fma(h, v.y, a[r].y);
                     }
                 }
             }
@@ -1333,15 +1367,18 @@ int dfi_reconstruction(const void* sino, int dtype, int nrow_in, int nslice,
         }
         if (st != ATH_OK) return st;
         {
-            const dim3 grid((p.N + 63) / 64,
-                            (nrow + 4 * kColRun - 1) / (4 * kColRun));
+            const dim3 grid((p.N + 511) / 512 * 8 *
+                            ((nrow + 4 * kColRun - 1) / (4 * kColRun)));
             hipLaunchKernelGGL(dfi_cols_kernel, grid, dim3(kThreads), 0, s, R1,
                                nrow, p.N, h5, R2);
             st = check_hip(hipGetLastError(), "dfi_cols_kernel launch");
             if (st != ATH_OK) return st;
         }
         const int h = (p.N - 1) / 2 + 1;  // columns v <= m
-        hipLaunchKernelGGL(dfi_grid_kernel, row_grid(h, p.N, kThreads),
+        const long long gtiles =
+            (long long)((p.N + 15) / 16) * ((h + 15) / 16);
+        hipLaunchKernelGGL(dfi_grid_kernel,
+                           dim3((unsigned)std::min(gtiles, 1LL << 22)),
                            dim3(kThreads), 0, s, R2, nrow, p.N, R1);
         st = check_hip(hipGetLastError(), "dfi_grid_kernel launch");
         if (st != ATH_OK) return st;

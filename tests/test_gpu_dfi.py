@@ -107,6 +107,21 @@ def test_dfi_vs_oracle(nrow, ncol, center, dtype, pad_mode, filt, pad_rate,
     assert err <= 1e-12
 
 
+@pytest.mark.parametrize("nrow,ncol", [
+    (2, 9), (16, 15), (17, 17), (63, 31), (64, 33), (65, 47), (120, 341),
+    (129, 343)])
+def test_dfi_tile_edges_vs_oracle(nrow, ncol):
+    """Lines of 13 to 513 samples (one less, as many, one more than the
+    tiles of the column prefilter and the gridding) and rows around the
+    prefilter's 64."""
+    from oracle import dfi_np as D
+    from algotom_amd.rec import reconstruction as rec
+    sino = _sino(nrow, ncol, np.float64, 31 * nrow + ncol)
+    center = ncol / 2.0 - 0.3
+    got = rec.dfi_reconstruction(sino, center, apply_log=False)
+    assert _rel(got, D.dfi(sino, center, apply_log=False)) <= 1e-12
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_dfi_apply_log_vs_oracle(dtype):
     """-log after shift and padding (reconstruction.py:862-867): values
