@@ -24,7 +24,8 @@
 // The kernel spectrum Khat (L/2+1 columns of L complex values, 1/(M L)
 // folded in) is built once per (W, window) by the same two forward passes
 // over the 2W rows of K.  The column transform holds L complex doubles in
-// LDS, so L <= 8192 (ncol up to about 3800 with the default pad); L = 16384
+// LDS (registers for L = 1024, 2048 and 4096: cols_reg_kernel), so L <= 8192
+// (ncol up to about 3800 with the default pad); L = 16384
 // (ncol up to about 7960) runs the column pass as the two-level transform
 // of fft_lds.h (cols_big_kernel) with a per-workgroup global scratch.
 // Kernel samples at index >= L are dropped rather than wrapped: a kept
@@ -140,6 +141,64 @@ __global__ __launch_bounds__(F2Cfg<MAXB>::nt) void cols_kernel(
     double2* dst = U + (size_t)img * nout * (M + 1) + k;
     for (int y = tid; y < nout; y += NT_)
         dst[(size_t)y * (M + 1)] = buf[r0 + y];
+}
+
+// The column pass (not the spectrum) at L = 1024, 2048 and 4096: the column
+// in registers (RegFft), 16 rows per thread, instead of in LDS with a trip
+// per radix-8 pass.  A column is one complex double of every cache line that
+// it touches; the 8 columns of a line go to workgroups of one XCD (index mod
+// 8) that follow each other, so that its L2 serves 7 of them.  6 images of 1500
+// columns (L = 4096): 985 -> 536 us.
+template <int R>
+__global__ __launch_bounds__(RegFft<R>::NT, 3)
+void cols_reg_kernel(const double2* __restrict__ T, int nrows_in,
+                     const double2* __restrict__ tw2,
+                     const double2* __restrict__ khat,
+                     double2* __restrict__ U, int r0, int nout, int M) {
+    using F = RegFft<R>;
+    extern __shared__ double2 buf[];
+    double* d = reinterpret_cast<double*>(buf);
+    const int t = threadIdx.x;
+    const int b = blockIdx.x;
+    const int k = (b & ~63) + ((b & 7) << 3) + ((b >> 3) & 7);
+    if (k > M) return;
+    const int img = blockIdx.y;
+    const double2* col = T + (size_t)img * nrows_in * (M + 1) + k;
+    double2 v[16], w[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int i = t + r * F::NT;
+        const double2 x = col[(size_t)min(i, nrows_in - 1) * (M + 1)];
+        v[r] = i < nrows_in ? x : make_double2(0.0, 0.0);
+    }
+    const typename F::Bases tb = F::bases(tw2);
+    F::forward(t, v, d, tb);
+    const double2* kc = khat + (size_t)k * F::M + t;
+#pragma unroll
+    for (int u = 0; u < F::U; ++u)
+#pragma unroll
+        for (int k3 = 0; k3 < R; ++k3)
+            w[u * R + k3] =
+                cmul(v[F::slot(u, k3)], kc[u * F::NT + 256 * k3]);
+    F::inverse(t, w, d, tb);
+    double2* dst = U + (size_t)img * nout * (M + 1) + k;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int y = t + r * F::NT - r0;
+        if (y >= 0 && y < nout) dst[(size_t)y * (M + 1)] = w[pos16(r)];
+    }
+}
+
+template <int R>
+int launch_cols_reg(const double2* T, int nrows_in, const double2* tw2,
+                    const double2* khat, double2* U, int r0, int nout, int M,
+                    int nimg, hipStream_t s) {
+    auto ck = cols_reg_kernel<R>;
+    prepare_lds(ck, RegFft<R>::kLds);
+    hipLaunchKernelGGL(ck, dim3((M + 64) / 64 * 64, nimg),
+                       dim3(RegFft<R>::NT), RegFft<R>::kLds, s, T, nrows_in,
+                       tw2, khat, U, r0, nout, M);
+    return check_hip(hipGetLastError(), "cols_reg_kernel launch");
 }
 
 // Column pass at L = LV * H (16384: conv_big / fft_big_forward; 32768:
@@ -475,14 +534,21 @@ int run_filter(const float* images, int nimg, int ncol, long long row_stride,
                        width, p.tw, T, M);
     int st = check_hip(hipGetLastError(), "rows_fwd_kernel launch");
     if (st != ATH_OK) return st;
-    auto ck = cols_kernel<MAXB_C, false>;
-    const size_t lds_c = (size_t)L * sizeof(double2);
-    prepare_lds(ck, 1024 * (size_t)MAXB_C * sizeof(double2));
-    hipLaunchKernelGGL(ck, dim3(M + 1, nimg), dim3(F2Cfg<MAXB_C>::nt), lds_c, s,
-                       T,
-                       width, p.tw2, nullptr, p.khat, U, width + pad, ncol, M,
-                       1.0);
-    st = check_hip(hipGetLastError(), "cols_kernel launch");
+    if constexpr (MAXB_C == 2 || MAXB_C == 4) {
+        st = launch_cols_reg<4 * MAXB_C>(T, width, p.tw2, p.khat, U,
+                                         width + pad, ncol, M, nimg, s);
+    } else if (L == 1024) {
+        st = launch_cols_reg<4>(T, width, p.tw2, p.khat, U, width + pad, ncol,
+                                M, nimg, s);
+    } else {
+        auto ck = cols_kernel<MAXB_C, false>;
+        const size_t lds_c = (size_t)L * sizeof(double2);
+        prepare_lds(ck, 1024 * (size_t)MAXB_C * sizeof(double2));
+        hipLaunchKernelGGL(ck, dim3(M + 1, nimg), dim3(F2Cfg<MAXB_C>::nt),
+                           lds_c, s, T, width, p.tw2, nullptr, p.khat, U,
+                           width + pad, ncol, M, 1.0);
+        st = check_hip(hipGetLastError(), "cols_kernel launch");
+    }
     if (st != ATH_OK) return st;
     auto ik = rows_inv_kernel<MAXB_R, Tout>;
     prepare_lds(ik, 1024 * (size_t)MAXB_R * sizeof(double2));

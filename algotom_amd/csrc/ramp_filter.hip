@@ -34,9 +34,9 @@ template <> struct RowCfg<8> { static constexpr int maxb = 2, nt = 1024; };
 // bounds it is float64 arithmetic (2170 vector instructions per wave and row,
 // issued in 58% of the cycles at M = 4096).  115264 float32 rows: of 2560
 // columns 5.56 -> 3.24 ms (with the logarithm 6.15 -> 4.1 ms), of 1200
-// columns 2.58 -> 1.35 ms, of 600 columns 1.42 -> 0.97 ms.  Below M = 1024 a row is
-// less than a wave of 16 points per thread; M = 8192 would be 32 points per
-// thread.
+// columns 2.58 -> 1.35 ms, of 600 columns 1.42 -> 0.97 ms.  Below M = 1024 a
+// row is less than a wave of 16 points per thread; M = 8192 would be 32
+// points per thread.
 constexpr int kRegs1024 = 3;
 template <> struct RowCfg<kRegs1024> : RegFft<4> {
     static constexpr int nt = NT;
@@ -488,7 +488,8 @@ __device__ __forceinline__ Log32Table* row_log_table(double2* buf) {
 // Persistent: each workgroup stages the twiddles once, then filters rows
 // blockIdx.x, blockIdx.x + gridDim.x, ... of the (nrow, nslice, ncol) stack.
 template <int MAXB, typename Tin, typename Tout>
-__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>) void ramp_filter_kernel(
+__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>)
+void ramp_filter_kernel(
     const Tin* __restrict__ sino, Tout* __restrict__ out, size_t rows,
     int nslice, int ncol, int pad, int pad_mode, int apply_log,
     const double2* __restrict__ tw, const double2* __restrict__ spec,
@@ -512,15 +513,15 @@ __global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>) void ramp_filter
 
 // Transpose of ramp_filter_kernel (float32 in and out), persistent.
 template <int MAXB>
-__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>) void ramp_filter_adjoint_kernel(
+__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>)
+void ramp_filter_adjoint_kernel(
     const float* __restrict__ in, float* __restrict__ out, size_t rows,
     int nslice, int ncol, int pad, int pad_mode,
     const double2* __restrict__ tw, const double2* __restrict__ spec,
     int nwin, int M) {
     extern __shared__ double2 buf[];
     double2* tq = buf + M;
-    if (MAXB == 1)
-        stage_quarter<RowCfg<MAXB>::nt>(tq, tw, M);
+    if (MAXB == 1) stage_quarter<RowCfg<MAXB>::nt>(tq, tw, M);
     for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
         const double2* G =
             spec + (nwin > 1 ? (row / nslice) : 0) * (size_t)(M + 1);
@@ -533,7 +534,8 @@ __global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>) void ramp_filter
 // Rows of many stacks sharing the FFT length L = 2M (hence the twiddles),
 // persistent; a row's stack is found by binary search over row_begin.
 template <int MAXB, typename Tin, typename Tout>
-__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>) void ramp_filter_batched_kernel(
+__global__ __launch_bounds__(RowCfg<MAXB>::nt, kRowWaves<MAXB>)
+void ramp_filter_batched_kernel(
     const ath_filter_job* __restrict__ jobs, int njobs, long long total_rows,
     int pad_mode, int apply_log, int M) {
     extern __shared__ double2 buf[];
@@ -1048,8 +1050,9 @@ int ramp_filter_batched(const ath_filter_job* jobs, int njobs,
     case 1: return batched_in<1>(in_dtype, out_dtype, jobs, njobs, total_rows,
                                  fft_len, pad_mode, apply_log, s);
     case kRegs1024:
-        return batched_in<kRegs1024>(in_dtype, out_dtype, jobs, njobs, total_rows,
-                                 fft_len, pad_mode, apply_log, s);
+        return batched_in<kRegs1024>(in_dtype, out_dtype, jobs, njobs,
+                                     total_rows, fft_len, pad_mode, apply_log,
+                                     s);
     case 2: return batched_in<2>(in_dtype, out_dtype, jobs, njobs, total_rows,
                                  fft_len, pad_mode, apply_log, s);
     case 4: return batched_in<4>(in_dtype, out_dtype, jobs, njobs, total_rows,
@@ -1113,8 +1116,9 @@ int ramp_filter_adjoint(const float* in, int nrow, int nslice, int ncol,
     case 1: return launch_adjoint<1>(in, nrow, nslice, ncol, pad, pad_mode,
                                      plan, fft_len, nwin, out, s);
     case kRegs1024:
-        return launch_adjoint<kRegs1024>(in, nrow, nslice, ncol, pad, pad_mode,
-                                     plan, fft_len, nwin, out, s);
+        return launch_adjoint<kRegs1024>(in, nrow, nslice, ncol, pad,
+                                         pad_mode, plan, fft_len, nwin, out,
+                                         s);
     case 2: return launch_adjoint<2>(in, nrow, nslice, ncol, pad, pad_mode,
                                      plan, fft_len, nwin, out, s);
     case 4: return launch_adjoint<4>(in, nrow, nslice, ncol, pad, pad_mode,
@@ -1141,9 +1145,9 @@ int ramp_filter(const void* sino, int in_dtype, int nrow, int nslice,
                                   ncol, pad, pad_mode, apply_log, plan,
                                   fft_len, nwin, s);
     case kRegs1024:
-        return dispatch_in<kRegs1024>(in_dtype, out_dtype, sino, out, nrow, nslice,
-                                  ncol, pad, pad_mode, apply_log, plan,
-                                  fft_len, nwin, s);
+        return dispatch_in<kRegs1024>(in_dtype, out_dtype, sino, out, nrow,
+                                      nslice, ncol, pad, pad_mode, apply_log,
+                                      plan, fft_len, nwin, s);
     case 2: return dispatch_in<2>(in_dtype, out_dtype, sino, out, nrow, nslice,
                                   ncol, pad, pad_mode, apply_log, plan,
                                   fft_len, nwin, s);

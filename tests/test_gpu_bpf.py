@@ -38,6 +38,21 @@ def test_circular_filter_vs_oracle(ncol, pad, mode):
     assert err <= 1e-11
 
 
+# columns held in registers (FFT lengths 1024, 2048, 4096): 2 ncol + 3 pad at
+# a power of two, just above one, and without padding
+@pytest.mark.parametrize("ncol,pad", [
+    (287, 150), (512, 0), (513, 0), (799, 150), (1025, 0), (1823, 150)])
+def test_circular_filter_columns_in_registers(ncol, pad):
+    from oracle import bpf_np
+    from algotom_amd.rec import reconstruction as rec
+    rng = np.random.default_rng(ncol + pad)
+    img = rng.standard_normal((ncol, ncol)).astype(np.float32)
+    win = rec.make_circular_ramp_window(ncol + 2 * pad, "hann")
+    got = rec.apply_circular_ramp_filter(img, win, pad=pad, pad_mode="edge")
+    ref = bpf_np.circular_filter(img, win, pad, "edge")
+    assert np.abs(got - ref).max() <= 1e-11 * np.abs(ref).max()
+
+
 def _phantom_sino(nrow=181, ncol=96, center=47.5, nslice=1, seed=3):
     import torch
     from algotom_amd.util import phantom
