@@ -10,15 +10,19 @@ stack (log, pad, ramp filter, back-projection, mask, scale).
 value = pixel-angle updates per second (GUPS = 1e9 updates/s),
 U = 64 * 2560^2 * 1801 = 7.554e11 updates per step.
 
-roofline (back-projection kernel, the dominant one): it is a gather with no
-MFMA work and its HBM traffic is 8 % of peak, so the bound is VALU issue.
-achieved = the kernel's VALU instructions per launch (SQ_INSTS_VALU, from the
+roofline (bp_matrix_kernel, the dominant one): its products run on the matrix
+cores and their operands are built by the VALU, whose issue is the bound; its
+HBM traffic is 14 % of peak.
+achieved = the kernel's VALU instructions per launch (SQ_INSTS_VALU, which
+counts the matrix instructions too, from the
 committed rocprofv3 counters of this kernel and workload,
-profiles/bp_counters.json) x 64 lanes over the kernel's mean duration from
-HIP events on the launch stream; peak = 256 CU x 64 lanes x 2.4 GHz = 39.3 T
-lane-op/s; traffic = the same profile's calibrated FETCH_SIZE + WRITE_SIZE
-bytes per launch.  The gather-byte model (U x 8 B) and the compulsory-byte
-HBM fraction are reported in detail.
+profiles/bp_counters.json) x 64 lanes over the back-projection's mean time
+from HIP events on the launch stream (the split of the samples included);
+peak = 256 CU x 64 lanes x 2.4 GHz = 39.3 T lane-op/s; traffic = the same
+profile's calibrated FETCH_SIZE + WRITE_SIZE bytes per launch.  detail has
+the matrix instructions' rate (all operands, of which one weight in four is
+not zero) as a fraction of 2.5 PFLOP/s, the gather-byte model (U x 8 B) and
+the compulsory-byte HBM fraction.
 cpu_baseline: the oracle's OpenMP C port (numba-typed restatement of the
 reference's CPU path) on 4 of the 64 sinograms, on this host's cores
 (median of 5 after a warm-up).
@@ -96,6 +100,8 @@ NSLICE, NROW, NCOL, CENTER = 64, 1801, 2560, 1280.37
 PEAK_HBM_GBS = 8000.0
 # MI355X VALU issue peak: 256 CUs x 64 lanes per clock x 2.4 GHz
 PEAK_VALU_TLANE = 256 * 64 * 2.4e9 / 1e12
+# dense float16 matrix product
+PEAK_F16_FLOPS = 2.5e15
 METRIC = ("GUPS (pixel·angle updates/s) FBP 2560²×1801 ang; "
           "% HBM roofline; grad steps/s")
 
@@ -135,8 +141,8 @@ def copy_bandwidth(dev, nbytes=1 << 30, reps=5):
 
 
 def load_counters():
-    """rocprofv3 counters of the reference-arithmetic back-projection kernel
-    on this workload (profiles/bp_counters.json), or None."""
+    """rocprofv3 counters of the matrix back-projection kernel on this
+    workload (profiles/bp_counters.json), or None."""
     path = os.path.join(ROOT, "profiles", "bp_counters.json")
     if not os.path.exists(path):
         return None
@@ -925,6 +931,9 @@ def main():
                    "hbm_copy_GBs": copy_gbs,
                    "bp_valu_lane_ops_per_update":
                        cnt["valu_lane_ops_per_update"] if cnt else None,
+                   "bp_mfma_frac_of_peak":
+                       (cnt["mfma_flops_per_launch"] / (bp_ms * 1e-3)
+                        / PEAK_F16_FLOPS if cnt else None),
                    "bp_hbm_GBs": (cnt["traffic_bytes"] / (bp_ms * 1e-3) / 1e9
                                   if cnt else None),
                    "bp_hbm_frac_of_peak": (cnt["traffic_bytes"]
