@@ -109,11 +109,12 @@ def test_dfi_vs_oracle(nrow, ncol, center, dtype, pad_mode, filt, pad_rate,
 
 @pytest.mark.parametrize("nrow,ncol", [
     (2, 9), (16, 15), (17, 17), (63, 31), (64, 33), (65, 47), (120, 341),
-    (129, 343)])
+    (129, 343), (6, 1255), (6, 1257)])
 def test_dfi_tile_edges_vs_oracle(nrow, ncol):
     """Lines of 13 to 513 samples (one less, as many, one more than the
-    tiles of the column prefilter and the gridding) and rows around the
-    prefilter's 64."""
+    tiles of the column prefilter and the gridding), rows around the
+    prefilter's 64, and shifted lines of 1279 and 1281 samples (one workgroup
+    forms 1280 coefficients at a time)."""
     from oracle import dfi_np as D
     from algotom_amd.rec import reconstruction as rec
     sino = _sino(nrow, ncol, np.float64, 31 * nrow + ncol)
