@@ -361,10 +361,12 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
             g.valid = a0 + k4 < N;
             g.inner = g.valid && lo >= 0.0 && hi <= w1;
             g.pad = 0;
-            const double off = cen - (double)g.L;
-            g.pos = off + kPosMagic;
-            g.win = kWinMagic -
-                    (off - fma(1.5, fabs(t.x) + fabs(t.y), kSlack));
+            // rounded to fixed point before L is taken off, so that the bits
+            // of a block do not depend on the tile it lies in
+            g.pos = (cen + kPosMagic) - (double)g.L;
+            g.win = (kWinMagic -
+                     (cen - fma(1.5, fabs(t.x) + fabs(t.y), kSlack))) +
+                    (double)g.L;
             if (n16 == 0) angles[slot * kStep + k4] = g;
         };
 
@@ -548,9 +550,9 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
                 (unsigned)(k4 * ROWS + ROWS - 1 - 127 - (WIDE ? 0 : 2)) * kRow +
                 n16 * 16;
             const double fr = fma(yl, s, fma(xl, c, g->pos));
+            const double bn = fma(-yb, s, fma(-xb, c, g->win));
             unsigned p[BX], e[BX];
             if (__all(g->inner)) {
-                const double bn = fma(-yb, s, fma(-xb, c, g->win));
 #pragma unroll
                 for (int i = 0; i < BX; ++i) {
                     const double m = (double)(xw - xg + 4 * i);
@@ -559,8 +561,10 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
                 }
             } else {
                 // some pixel or angle is out of range: the vector kernel's
-                // exact position decides which, window positions are clamped
-                // to the row, and in-range pixels keep the weights above
+                // exact position decides which; windows that start in the
+                // row and in-range pixels' weights are those above (a tile of
+                // the other shape may take the same block there), other
+                // windows are clamped to the row
                 // (opaque, so that the columns' coordinates are not kept in
                 // registers across the angle loop)
                 double xo = xl, yo = yl;
@@ -575,9 +579,12 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
                     const double f = det_pos((xo + m) * c, yo, s, cen);
                     const bool in = f >= 0.0 && f <= w1;
                     const double edge = clamp_pos(f, w1) - l + kPosMagic;
-                    const double b =
-                        clamp_pos(fma(m, c, br), w1) - l + 0.5 * kSlack;
-                    e[i] = (unsigned)__double2loint(kWinMagic - b) >> 25;
+                    const double lo = fma(m, c, br);
+                    const double b = clamp_pos(lo, w1) - l + 0.5 * kSlack;
+                    // (lo >= kSlack - 2^-38 wherever the tile is in range)
+                    const bool whole = lo >= 0.5 * kSlack && lo <= w1;
+                    e[i] = (unsigned)__double2loint(
+                               whole ? fma(-m, c, bn) : kWinMagic - b) >> 25;
                     p[i] = (unsigned)__double2loint(in ? fma(m, c, fr) : edge);
                     // selector 7: no weights
                     unsigned none = e[i];

@@ -59,8 +59,9 @@ def test_error_against_float64_sums(case, dtype):
 
 
 def test_slice_bits_do_not_depend_on_the_stack():
-    """A slice in a pair of groups, alone in a group, or beside other slices
-    keeps its bits, and so do mask and scale (zero outside the circle)."""
+    """A slice in either group of a pair, in a padded group or beside other
+    slices keeps its bits, and so do mask and scale (zero outside the circle).
+    (At 200 columns every launch takes pairs of groups.)"""
     import torch
     from algotom_amd.rec import reconstruction as rec
     x, ang = _case(200, 133, 37, np.pi, 3)
@@ -75,6 +76,41 @@ def test_slice_bits_do_not_depend_on_the_stack():
     yy, xx = np.mgrid[:200, :200] - 100
     outside = torch.from_numpy(xx ** 2 + yy ** 2 > 90 ** 2).cuda()
     assert not full.permute(1, 0, 2)[:, outside].any()
+
+
+def _last_group_alone(ncol, nslice):
+    """run_matrix's choice for an odd number of groups: the last one by itself
+    (64 x 32 tiles) rather than in a pair (32 x 32) with an idle one."""
+    def rounds(tx, ty, units):
+        return -(-(-(-ncol // tx) * -(-ncol // ty) * units) // 256)
+    pairs, odd = divmod(-(-nslice // 16), 2)
+    return bool(odd) and not (
+        rounds(32, 32, pairs + 1) * 0.69
+        < rounds(32, 32, pairs) * 0.69 + rounds(64, 32, 1) * 0.88)
+
+
+@pytest.mark.parametrize("ncol,nrow,center,edge", [
+    (1025, 721, 512.37, False), (1025, 200, 1021.5, True),
+    # at angle 0 every block's lowest position is an even column and 3/4 of
+    # the slack 2^-20, and the columns out of range end in the left half of
+    # a 64-column tile
+    (1065, 160, 2.0 + 3 * 2.0 ** -22, False),
+    (1065, 160, 2.0 + 3 * 2.0 ** -22, True)])
+def test_slice_bits_do_not_depend_on_the_tile_shape(ncol, nrow, center, edge):
+    """Slices whose group is launched alone (64 x 32 tiles) have the bits that
+    they have in a pair (32 x 32 tiles), also in blocks whose tile of one
+    shape lies within the row and whose tile of the other does not."""
+    import torch
+    from algotom_amd.rec import reconstruction as rec
+    nslice = 48
+    assert _last_group_alone(ncol, nslice) and not _last_group_alone(ncol, 32)
+    x, ang = _case(ncol, nrow, nslice, np.pi, 1)
+    ang[::2] = 0.0
+    kw = dict(edge_pad=edge, mask_radius=ncol / 2)
+    full = rec._backproject_matrix(x, ang, center, 1, **kw)
+    pair = rec._backproject_matrix(x[:, 16:].contiguous(), ang, center, 1,
+                                   **kw)
+    assert torch.equal(full[:, 16:], pair)
 
 
 def test_scales_and_special_samples():
