@@ -112,12 +112,13 @@ static_assert(kTailPairs >= Tile<1>::rows + 16, "tail");
 struct MatArgs {
     const unsigned* op;     // split samples
     const unsigned* smax;   // per slice: bits of max|s|
-    const double2* trig;    // per angle: cos, sin
+    const float2* trig;     // per angle: cos, sin
     int scaled;             // samples carry the power of two of smax
     int npair;              // column pairs per row
     int group0, group_end;  // slice groups of the launch
     int group_have;         // slice groups of the stack
     unsigned patches_x, patches_y;
+    double pos0;            // centre + kPosMagic
 };
 
 __device__ __forceinline__ double det_pos(double xc_c, double yc, double s,
@@ -143,14 +144,13 @@ __device__ __forceinline__ float widen<__hip_bfloat16>(__hip_bfloat16 v) {
 }
 
 __global__ void trig_kernel(const float* __restrict__ angles, int nrow,
-                            double2* __restrict__ trig,
+                            float2* __restrict__ trig,
                             unsigned* __restrict__ smax, int nmax,
                             unsigned* __restrict__ tail, int ntail) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nrow) {
         const float th = -angles[i];
-        trig[i] = make_double2((double)(float)cos((double)th),
-                               (double)(float)sin((double)th));
+        trig[i] = make_float2((float)cos((double)th), (float)sin((double)th));
     }
     if (i < nmax) smax[i] = 0u;
     if (i < ntail) tail[i] = 0u;
@@ -345,10 +345,12 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
         const double yb = to_scalar((double)yw + 1.5 - ic);
 
         auto trig = [&](int a0) { return ma.trig[min(a0 + k4, N - 1)]; };
+        // the tile's centre
+        const double xm = to_scalar((double)x0 + 0.5 * (TL::X - 1) - ic);
+        const double ym = (double)y0 + 0.5 * (TL::Y - 1) - ic;
         // lanes 0, 16, 32, 48 of one wave: the angles of the step at a0
-        auto geometry = [&](int a0, double2 t, unsigned slot) {
-            const double xm = (double)x0 + 0.5 * (TL::X - 1) - ic;
-            const double ym = (double)y0 + 0.5 * (TL::Y - 1) - ic;
+        auto geometry = [&](int a0, float2 tf, unsigned slot) {
+            const double2 t = make_double2((double)tf.x, (double)tf.y);
             const double fm = det_pos(xm * t.x, ym, t.y, cen);
             const double ext = fma(0.5 * (TL::Y - 1), fabs(t.y),
                                    0.5 * (TL::X - 1) * fabs(t.x));
@@ -363,7 +365,7 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
             g.pad = 0;
             // rounded to fixed point before L is taken off, so that the bits
             // of a block do not depend on the tile it lies in
-            g.pos = (cen + kPosMagic) - (double)g.L;
+            g.pos = ma.pos0 - (double)g.L;
             g.win = (kWinMagic -
                      (cen - fma(1.5, fabs(t.x) + fabs(t.y), kSlack))) +
                     (double)g.L;
@@ -533,7 +535,7 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
         // step t: its angles are in slot t % 3; the samples of step t + 1 are
         // loaded and stored, and one wave works out the angles of step t + 2
         unsigned cur = 0, buf = 0, turn = 0;
-        double2 tr = trig(2 * kStep);
+        float2 tr = trig(2 * kStep);
         for (int a0 = 0; a0 < N; a0 += kStep) {
             const unsigned next = cur == 2 ? 0 : cur + 1;
             const unsigned after = next == 2 ? 0 : next + 1;
@@ -550,9 +552,9 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
                 (unsigned)(k4 * ROWS + ROWS - 1 - 127 - (WIDE ? 0 : 2)) * kRow +
                 n16 * 16;
             const double fr = fma(yl, s, fma(xl, c, g->pos));
-            const double bn = fma(-yb, s, fma(-xb, c, g->win));
             unsigned p[BX], e[BX];
             if (__all(g->inner)) {
+                const double bn = fma(-yb, s, fma(-xb, c, g->win));
 #pragma unroll
                 for (int i = 0; i < BX; ++i) {
                     const double m = (double)(xw - xg + 4 * i);
@@ -565,26 +567,21 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
                 // row and in-range pixels' weights are those above (a tile of
                 // the other shape may take the same block there), other
                 // windows are clamped to the row
-                // (opaque, so that the columns' coordinates are not kept in
-                // registers across the angle loop)
-                double xo = xl, yo = yl;
-                asm volatile("" : "+v"(xo), "+v"(yo));
                 const double l = (double)g->L;
-                const double br = det_pos(xb * c, yb, s, cen) -
-                                  fma(1.5, fabs(c) + fabs(s), kSlack);
+                const double bn = fma(-yb, s, fma(-xb, c, g->win));
+                // (where the tile is in range a window starts kSlack - 2^-23
+                // or more past L, so the clamps change none)
+                const double q_end = kWinMagic - (w1 - l + 0.5 * kSlack);
                 const bool valid = g->valid;
 #pragma unroll
                 for (int i = 0; i < BX; ++i) {
                     const double m = (double)(xw - xg + 4 * i);
-                    const double f = det_pos((xo + m) * c, yo, s, cen);
+                    const double q = fmin(fmax(fma(-m, c, bn), q_end),
+                                          kWinMagic - 0.5 * kSlack);
+                    e[i] = (unsigned)__double2loint(q) >> 25;
+                    const double f = det_pos((xl + m) * c, yl, s, cen);
                     const bool in = f >= 0.0 && f <= w1;
                     const double edge = clamp_pos(f, w1) - l + kPosMagic;
-                    const double lo = fma(m, c, br);
-                    const double b = clamp_pos(lo, w1) - l + 0.5 * kSlack;
-                    // (lo >= kSlack - 2^-38 wherever the tile is in range)
-                    const bool whole = lo >= 0.5 * kSlack && lo <= w1;
-                    e[i] = (unsigned)__double2loint(
-                               whole ? fma(-m, c, bn) : kWinMagic - b) >> 25;
                     p[i] = (unsigned)__double2loint(in ? fma(m, c, fr) : edge);
                     // selector 7: no weights
                     unsigned none = e[i];
@@ -707,14 +704,15 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
     MatArgs ma;
     unsigned* smax = reinterpret_cast<unsigned*>(work);
     work += align256((size_t)groups * kGroup * sizeof(unsigned));
-    double2* trig = reinterpret_cast<double2*>(work);
-    work += align256((size_t)a.nrow * sizeof(double2));
+    float2* trig = reinterpret_cast<float2*>(work);
+    work += align256((size_t)a.nrow * sizeof(float2));
     unsigned* op = reinterpret_cast<unsigned*>(work);
     ma.op = op;
     ma.smax = smax;
     ma.trig = trig;
     ma.scaled = dtype != ATH_F16;
     ma.npair = npair;
+    ma.pos0 = a.center + kPosMagic;
     const int nmax = groups * kGroup;
     const size_t nop = (size_t)groups * kGroup * a.nrow * npair * PL;
     const int ntail = kTailPairs * kGroup * PL;
@@ -774,7 +772,7 @@ size_t back_projection_matrix_workspace(int dtype, int nrow, int nslice,
                                         int ncol) {
     const size_t groups = groups_of(nslice);
     return align256(groups * kGroup * sizeof(unsigned)) +
-           align256((size_t)nrow * sizeof(double2)) +
+           align256((size_t)nrow * sizeof(float2)) +
            (groups * nrow * (size_t)((ncol + 1) / 2) + kTailPairs) * kGroup *
                4 * planes_of(dtype);
 }
