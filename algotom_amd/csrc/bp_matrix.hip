@@ -12,26 +12,33 @@
 // workgroup; the vector kernel (bp_tiled_kernel) pays 3.4 (16-bit) to 8.9
 // (reference typing) per pixel, angle and slice.
 //
-// Precision.  Nothing is reduced to 16 bits; 16-bit factors appear as exact
-// splits:
+// Precision.  16-bit factors appear as two-term splits:
 //   * a float32 sample s, scaled by a power of two per slice so that
-//     max|s| <= 2^15, is h + l with h = f16(s), l = f16(s - h): 22-23 bits
-//     and an absolute floor of 2^-40 of the slice's maximum; 16-bit storage
-//     is one f16 value (bfloat16 after the same scaling, exact);
+//     2^14 <= max|s| < 2^15, is h + l with h = f16(s), l = f16(s - h): 23 bits
+//     (22 where l rounds up), down to a last step of 2^-24 (2^-39 of the
+//     slice's maximum).  16-bit storage is one f16 value: float16 itself, a
+//     bfloat16 scaled in the same way, which is exact down to 2^-32 of the
+//     maximum;
 //   * the fraction of the detector position, rounded to nearest on 22 bits,
 //     is 2^-11 a + 2^-22 b, and so is its complement; a, b <= 2^11 are
 //     integers, and an integer n <= 2048 read as a float16 bit pattern is
 //     exactly n 2^-24 (subnormals and the first two binades share one step),
 //     so a and b need no conversion;
-//   * every product (h + l)(a + b) is exact in float32, the sums are float32.
-// Sums over four angles at a time round fewer times than a float32 sum after
-// every angle does: from about 100 angles on the error against float64 is
-// below that of ATH_ACC_F32SEQ (181 angles of noise 1.9e-7 against 2.4e-7,
-// 1801 angles 4.2e-7 against 7.4e-7).
+//   * every product (h + l)(a + b) is exact in float32; the matrix unit sums
+//     four angles in float32 and truncates, the total is rounded.
+// That is a bit less per sample than float32 and less per weight than the
+// float64 fraction of ATH_ACC_F32SEQ, against a quarter of its roundings of the
+// sum: from about 100 angles on the error against float64 is below
+// that of ATH_ACC_F32SEQ.  Relative 2-norm, 128 / 361 / 1801 / 3601 angles, the
+// largest of 131 to 2560 columns: white noise 1.8 / 2.3 / 4.3 / 5.8e-7 against
+// 2.0 / 3.3 / 7.4 / 10.5e-7, filtered projections 1.1 / 1.5 / 3.1 / 4.4e-7
+// against 1.8 / 2.8 / 6.2 / 8.8e-7, positive ones 0.9 / 1.5 / 3.2 / 4.5e-7
+// against 1.6 / 2.9 / 6.3 / 8.9e-7 (37 angles of noise: 1.6 against 1.1e-7).
 //
 // A slice with a non-finite (or > 2^100) sample would spread it over the 8
-// columns of a window; such slices, found by the maximum that also gives the
-// scale, are redone by the vector kernel in the caller's accumulation.
+// columns of a window, and one whose ordinary samples are small beside a few
+// huge ones would lose them (range_kernel); such slices are redone by the
+// vector kernel in the caller's accumulation.
 //
 // Measured (64 x 1801 x 2560, with the mask): float32 42 ms against 181 ms
 // for ATH_ACC_F32SEQ (17.9 against 4.2 updates per ps), float16 31
@@ -80,6 +87,8 @@ constexpr int kGroup = 16;     // slices per matrix operand
 constexpr int kStep = 4;       // angles per matrix operand
 // |sample| above 2^100 (bit pattern) goes to the vector kernel
 constexpr unsigned kMaxBits = 0x71800000u;
+constexpr unsigned kRedo = 0xffffffffu;  // in place of a slice's max|s|
+constexpr int kSpanCols = 32;            // columns of a span (range_kernel)
 
 // SG slice groups per workgroup share the weights of its pixels; every tile
 // keeps 64 accumulator registers per lane.
@@ -133,6 +142,12 @@ __device__ __forceinline__ int scale_exp(unsigned bits) {
     return 14 - ilogbf(__uint_as_float(bits));
 }
 
+// a scaled sample that is large for range_kernel
+constexpr float kLarge = 0.25f;
+__host__ __device__ inline int span_count(int ncol) {
+    return (ncol + kSpanCols - 1) / kSpanCols;
+}
+
 template <typename T> __device__ __forceinline__ float widen(T v);
 template <> __device__ __forceinline__ float widen<float>(float v) { return v; }
 template <> __device__ __forceinline__ float widen<__half>(__half v) {
@@ -145,14 +160,14 @@ __device__ __forceinline__ float widen<__hip_bfloat16>(__hip_bfloat16 v) {
 
 __global__ void trig_kernel(const float* __restrict__ angles, int nrow,
                             float2* __restrict__ trig,
-                            unsigned* __restrict__ smax, int nmax,
+                            unsigned* __restrict__ zero, int nzero,
                             unsigned* __restrict__ tail, int ntail) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nrow) {
         const float th = -angles[i];
         trig[i] = make_float2((float)cos((double)th), (float)sin((double)th));
     }
-    if (i < nmax) smax[i] = 0u;
+    if (i < nzero) zero[i] = 0u;
     if (i < ntail) tail[i] = 0u;
 }
 
@@ -182,14 +197,18 @@ __global__ __launch_bounds__(256) void slice_max_kernel(
 
 // (row, slice, column) samples -> (group, angle, pair, slice) entries.  A
 // block handles 128 columns of one angle's 16 slices through LDS, so both
-// the reads (columns) and the writes (slices) are contiguous.
+// the reads (columns) and the writes (slices) are contiguous.  Scaled samples
+// are counted on the way for range_kernel: spans[slice][span] = (angles in
+// which the span's samples are mostly small, angles in which they are all
+// zero); ordinary slices have few of either and add nothing.
 template <typename T, int PL>
 __global__ __launch_bounds__(256) void split_kernel(
     const T* __restrict__ sino, int nrow, int nslice, int ncol, int npair,
-    const unsigned* __restrict__ smax, int scaled,
+    const unsigned* __restrict__ smax, int scaled, uint2* __restrict__ spans,
     unsigned* __restrict__ op) {
-    constexpr int COLS = 128;
+    constexpr int COLS = 128, SPANS = COLS / kSpanCols;
     __shared__ float tile[kGroup][COLS + 1];
+    __shared__ unsigned count[SPANS][kGroup];  // not zero, large << 16
     const int c0 = blockIdx.x * COLS, row = blockIdx.y, g = blockIdx.z;
     const int tid = threadIdx.x;
     for (int e = tid; e < kGroup * COLS; e += 256) {
@@ -199,6 +218,7 @@ __global__ __launch_bounds__(256) void split_kernel(
             v = widen(sino[((size_t)row * nslice + j) * ncol + c]);
         tile[n][e % COLS] = v;
     }
+    if (tid < SPANS * kGroup) count[tid / kGroup][tid % kGroup] = 0u;
     __syncthreads();
     const int n = tid & 15, j = g * kGroup + n;
     const unsigned bits = j < nslice ? smax[j] : 0u;
@@ -212,6 +232,12 @@ __global__ __launch_bounds__(256) void split_kernel(
         if (bad) s0 = s1 = 0.0f;
         s0 = ldexpf(s0, ex);
         s1 = ldexpf(s1, ex);
+        if (scaled) {
+            const unsigned m = (s0 != 0.0f) + (s1 != 0.0f) +
+                               ((fabsf(s0) >= kLarge) << 16) +
+                               ((fabsf(s1) >= kLarge) << 16);
+            if (m) atomicAdd(&count[i / (kSpanCols / 2)][n], m);
+        }
         const half2_t h = {(_Float16)s0, (_Float16)s1};
         unsigned* dst = base + ((size_t)p * kGroup + n) * PL;
         if constexpr (PL == 2) {
@@ -224,6 +250,53 @@ __global__ __launch_bounds__(256) void split_kernel(
             *dst = __builtin_bit_cast(unsigned, h);
         }
     }
+    if (!scaled) return;
+    __syncthreads();
+    const int sp = tid / kGroup;
+    if (sp < SPANS && j < nslice && c0 + sp * kSpanCols < ncol) {
+        const unsigned m = count[sp][n], some = m & 0xffffu, large = m >> 16;
+        uint2* at = spans + (size_t)j * span_count(ncol) +
+                    c0 / kSpanCols + sp;
+        if (some == 0u)
+            atomicAdd(&at->y, 1u);
+        else if (8u * large < some)
+            atomicAdd(&at->x, 1u);
+    }
+}
+
+// Sends the slices whose samples the split does not hold well enough to the
+// vector kernel.  A term of the split ends 2^-40 below the slice's maximum: a
+// sample of less than 2^-16 of it has 24 bits no more.  That is nothing to a
+// pixel that also sees larger ones (the sum's own rounding is coarser), but a
+// pixel whose samples are all small, beside a few that are huge (a hot pixel
+// or column), would lose its value.  A pixel at a distance d from the axis sees
+// the columns within d of the centre, so a slice is redone if for any d, in
+// steps of a span of 32 columns, more than half of the (span, angle) pairs in
+// there that are not all zero have fewer than one sample in 8 of kLarge =
+// 2^-2 or more (the maximum is scaled to 2^14 .. 2^15).  With half of them
+// large the rms of a pixel's samples is 2^-4 or more, and the floor's error,
+// 2^-26 sqrt(2 n / 3) for n angles, below that of a float32 sum after every
+// angle, 2^-29 n / sqrt(2), from 128 angles on.
+__global__ __launch_bounds__(256) void range_kernel(
+    const uint2* __restrict__ spans, int nrow, int ncol, double center,
+    unsigned* __restrict__ smax) {
+    const int ns = span_count(ncol), j = blockIdx.x;
+    const uint2* sp = spans + (size_t)j * ns;
+    bool any = false;
+    for (int k = threadIdx.x; k < ns; k += 256) any |= sp[k].x != 0u;
+    if (!__syncthreads_or(any)) return;
+    const int mid = (int)fmin(fmax(center / kSpanCols, 0.0), ns - 1.0);
+    bool redo = false;
+    for (int d = threadIdx.x; d < ns; d += 256) {
+        unsigned long long low = 0, zero = 0, all = 0;
+        for (int k = max(mid - d, 0); k <= min(mid + d, ns - 1); ++k) {
+            low += sp[k].x;
+            zero += sp[k].y;
+            all += (unsigned)nrow;
+        }
+        redo |= 2 * low > all - zero;
+    }
+    if (__syncthreads_or(redo) && threadIdx.x == 0) smax[j] = kRedo;
 }
 
 __device__ __forceinline__ double clamp_pos(double f, double w1) {
@@ -702,8 +775,12 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
                hipStream_t s) {
     const int groups = groups_of(a.nslice), npair = (a.ncol + 1) / 2;
     MatArgs ma;
+    // maxima, then the spans' counts: cleared together
+    const size_t nmax = (size_t)groups * kGroup;
     unsigned* smax = reinterpret_cast<unsigned*>(work);
-    work += align256((size_t)groups * kGroup * sizeof(unsigned));
+    uint2* spans = reinterpret_cast<uint2*>(smax + nmax);
+    const size_t nzero = nmax * (1 + 2 * (size_t)span_count(a.ncol));
+    work += align256(nzero * sizeof(unsigned));
     float2* trig = reinterpret_cast<float2*>(work);
     work += align256((size_t)a.nrow * sizeof(float2));
     unsigned* op = reinterpret_cast<unsigned*>(work);
@@ -713,14 +790,16 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
     ma.scaled = dtype != ATH_F16;
     ma.npair = npair;
     ma.pos0 = a.center + kPosMagic;
-    const int nmax = groups * kGroup;
     const size_t nop = (size_t)groups * kGroup * a.nrow * npair * PL;
     const int ntail = kTailPairs * kGroup * PL;
     const T* sino = static_cast<const T*>(a.sino);
     hipLaunchKernelGGL(trig_kernel,
-                       dim3((std::max({a.nrow, nmax, ntail}) + 255) / 256),
-                       dim3(256), 0, s, a.angles, a.nrow, trig, smax, nmax,
-                       op + nop, ntail);
+                       dim3((unsigned)((std::max({(size_t)a.nrow, nzero,
+                                                  (size_t)ntail}) +
+                                        255) /
+                                       256)),
+                       dim3(256), 0, s, a.angles, a.nrow, trig, smax,
+                       (int)nzero, op + nop, ntail);
     int st = check_hip(hipGetLastError(), "trig_kernel launch");
     if (st != ATH_OK) return st;
     hipLaunchKernelGGL((slice_max_kernel<T>),
@@ -733,9 +812,15 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
                        dim3((unsigned)((a.ncol + 127) / 128),
                             (unsigned)a.nrow, (unsigned)groups),
                        dim3(256), 0, s, sino, a.nrow, a.nslice, a.ncol, npair,
-                       smax, ma.scaled, op);
+                       smax, ma.scaled, spans, op);
     st = check_hip(hipGetLastError(), "split_kernel launch");
     if (st != ATH_OK) return st;
+    if (ma.scaled) {
+        hipLaunchKernelGGL(range_kernel, dim3((unsigned)a.nslice), dim3(256),
+                           0, s, spans, a.nrow, a.ncol, a.center, smax);
+        st = check_hip(hipGetLastError(), "range_kernel launch");
+        if (st != ATH_OK) return st;
+    }
     ma.group0 = 0;
     ma.group_have = groups;
     // Pairs of groups; a last odd group by itself unless an idle one beside
@@ -771,7 +856,8 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
 size_t back_projection_matrix_workspace(int dtype, int nrow, int nslice,
                                         int ncol) {
     const size_t groups = groups_of(nslice);
-    return align256(groups * kGroup * sizeof(unsigned)) +
+    return align256(groups * kGroup * (1 + 2 * (size_t)span_count(ncol)) *
+                    sizeof(unsigned)) +
            align256((size_t)nrow * sizeof(float2)) +
            (groups * nrow * (size_t)((ncol + 1) / 2) + kTailPairs) * kGroup *
                4 * planes_of(dtype);

@@ -174,14 +174,18 @@ int ath_back_projection(const void* sino, int sino_dtype, int nrow,
                         void* stream);
 
 /* The back-projection of a stack on the matrix cores (the fast path of
- * fbp_reconstruction and bpf_reconstruction for stacks): samples and
- * interpolation weights as exact two-term float16 splits (22 bits), float32
- * sums.  Not bit-identical to ath_back_projection; from about 100 angles on
- * its error against float64 is below that of ATH_ACC_F32SEQ.  A slice's result does not
- * depend on the other slices of the stack.  sino_dtype: ATH_F32 (acc
- * ATH_ACC_F32SEQ or ATH_ACC_F32), ATH_F16 or ATH_BF16 (acc ATH_ACC_F32).
- * Slices with a non-finite or > 2^100 sample are computed with acc exactly
- * as ath_back_projection does.  workspace: device memory of at least
+ * fbp_reconstruction and bpf_reconstruction for stacks): samples as two
+ * float16 terms (22-23 bits, down to 2^-39 of the slice's largest; float16
+ * samples as they are, bfloat16 exactly down to 2^-32 of the largest),
+ * interpolation weights of 22 bits, float32 sums, four angles at a time
+ * truncated.  Not bit-identical to ath_back_projection; from about 100 angles
+ * on its error against float64 is below that of ATH_ACC_F32SEQ.  A slice's
+ * result does not depend on the other slices of the stack.  sino_dtype: ATH_F32
+ * (acc ATH_ACC_F32SEQ or ATH_ACC_F32), ATH_F16 or ATH_BF16 (acc ATH_ACC_F32).
+ * A slice with a non-finite or > 2^100 sample, or (not ATH_F16) one where the
+ * samples within some distance of the centre's column mostly lie below 2^-16
+ * of the slice's largest, is computed with acc exactly as ath_back_projection
+ * does.  workspace: device memory of at least
  * ath_back_projection_matrix_workspace_bytes(...) (0: unsupported), 16-byte
  * aligned; ATH_ERR_WORKSPACE when too small. */
 size_t ath_back_projection_matrix_workspace_bytes(int sino_dtype, int nrow,

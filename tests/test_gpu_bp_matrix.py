@@ -143,6 +143,74 @@ def test_scales_and_special_samples():
                               equal_nan=True), j
 
 
+def _outliers(x, kind):
+    """A stack whose slices 1 .. have huge samples among ordinary ones."""
+    nrow, _, ncol = x.shape
+    gen = np.random.default_rng(7)
+    if kind == "one sample":
+        for j, v in enumerate((1e20, -3e6, 2.0 ** 99, 7e30), 1):
+            x[37 + j, j, 11 * j] = v
+    elif kind == "hot column":      # beside, at and far from the centre
+        for j, c in enumerate((0, 70, 47, ncol - 1), 1):
+            x[:, j, c] *= 1e9
+    else:                           # a sample of every 3rd row
+        for j in range(1, 5):
+            rows = np.arange(0, nrow, 3)
+            x[rows, j, gen.integers(0, ncol, rows.size)] = 1e12
+    return x
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("kind", ["one sample", "hot column", "scattered"])
+def test_ordinary_samples_beside_huge_ones(kind, dtype):
+    """Finite outliers do not flush the other samples of their slice: such
+    slices are exactly the vector kernel's, the others' bits stay."""
+    import torch
+    from algotom_amd.rec import reconstruction as rec
+    x, ang = _case(150, 200, 9, np.pi, 6)
+    x = x.to(getattr(torch, dtype))
+    acc = 1 if dtype == "float32" else 2
+    clean = rec._backproject_matrix(x, ang, 77.3, acc, True)
+    y = _outliers(x.clone(), kind)
+    got = rec._backproject_matrix(y, ang, 77.3, acc, True)
+    vec = rec._backproject_stack(y, ang, 77.3, acc, True)
+    assert torch.equal(got[:, 1:5], vec[:, 1:5])
+    for j in (0, 5, 8):
+        assert torch.equal(got[:, j], clean[:, j])
+        assert not torch.equal(got[:, j], vec[:, j])   # not redone
+
+
+@pytest.mark.parametrize("nrow", [128, 400])
+@pytest.mark.parametrize("data", ["noise", "2 orders of columns", "tails"])
+def test_small_samples_that_are_kept(nrow, data):
+    """Slices with a large range that stay on the matrix cores: the error in
+    every ring of pixels is at most that of a float32 sum after every angle
+    (2-norm over the ring)."""
+    import torch
+    from algotom_amd.rec import reconstruction as rec
+    ncol, cen = 160, 79.6
+    x, ang = _case(ncol, nrow, 6, np.pi, 8)
+    col = torch.arange(ncol, device="cuda") - cen
+    if data == "noise":
+        x[5, :, 3] = 2.0 ** 13      # an outlier within the range
+    elif data == "2 orders of columns":
+        x = x * torch.where(col.abs() < 40, 1.0, 100.0)
+    else:                           # a narrow object's filtered tails
+        x = x * torch.exp2(-(col.abs() / 6))
+    x = x.contiguous()
+    ref = rec._backproject_stack(x, ang, cen, 0, True)
+    seq = rec._backproject_stack(x, ang, cen, 1, True)
+    got = rec._backproject_matrix(x, ang, cen, 1, True)
+    assert not torch.equal(got, seq)
+    r = torch.from_numpy(np.hypot(*(np.mgrid[:ncol, :ncol] - 79.5))).cuda()
+    for lo in range(0, 80, 16):
+        ring = ((r >= lo) & (r < lo + 16))[:, None, :].expand_as(ref)
+        err, bound = _rel(got[ring], ref[ring]), _rel(seq[ring], ref[ring])
+        print("%s %d angles, ring %d: %.3g, %.3g" % (data, nrow, lo, err,
+                                                     bound))
+        assert err <= bound
+
+
 def test_fbp_dispatch_and_graph_replay():
     """fbp_reconstruction takes the matrix path by its rule, a batch member
     gets the single call's bits, also from a replayed graph."""
