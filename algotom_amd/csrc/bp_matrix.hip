@@ -125,7 +125,7 @@ struct MatArgs {
     int scaled;             // samples carry the power of two of smax
     int npair;              // column pairs per row
     int group0, group_end;  // slice groups of the launch
-    int group_have;         // slice groups of the stack
+    int group_op, group_have;  // slice groups that op holds
     unsigned patches_x, patches_y;
     double pos0;            // centre + kPosMagic
 };
@@ -204,12 +204,13 @@ __global__ __launch_bounds__(256) void slice_max_kernel(
 template <typename T, int PL>
 __global__ __launch_bounds__(256) void split_kernel(
     const T* __restrict__ sino, int nrow, int nslice, int ncol, int npair,
-    const unsigned* __restrict__ smax, int scaled, uint2* __restrict__ spans,
+    int group_op, const unsigned* __restrict__ smax, int scaled, uint2* __restrict__ spans,
     unsigned* __restrict__ op) {
     constexpr int COLS = 128, SPANS = COLS / kSpanCols;
     __shared__ float tile[kGroup][COLS + 1];
     __shared__ unsigned count[SPANS][kGroup];  // not zero, large << 16
-    const int c0 = blockIdx.x * COLS, row = blockIdx.y, g = blockIdx.z;
+    const int c0 = blockIdx.x * COLS, row = blockIdx.y;
+    const int g = group_op + blockIdx.z;
     const int tid = threadIdx.x;
     for (int e = tid; e < kGroup * COLS; e += 256) {
         const int n = e / COLS, c = c0 + e % COLS, j = g * kGroup + n;
@@ -224,7 +225,8 @@ __global__ __launch_bounds__(256) void split_kernel(
     const unsigned bits = j < nslice ? smax[j] : 0u;
     const bool bad = bits > kMaxBits;  // redone by the vector kernel
     const int ex = scaled ? scale_exp(bits) : 0;
-    unsigned* base = op + (((size_t)g * nrow + row) * npair) * (kGroup * PL);
+    unsigned* base =
+        op + (((size_t)blockIdx.z * nrow + row) * npair) * (kGroup * PL);
     for (int i = tid >> 4; i < COLS / 2; i += 16) {
         const int p = c0 / 2 + i;
         if (p >= npair) break;
@@ -278,9 +280,9 @@ __global__ __launch_bounds__(256) void split_kernel(
 // 2^-26 sqrt(2 n / 3) for n angles, below that of a float32 sum after every
 // angle, 2^-29 n / sqrt(2), from 128 angles on.
 __global__ __launch_bounds__(256) void range_kernel(
-    const uint2* __restrict__ spans, int nrow, int ncol, double center,
-    unsigned* __restrict__ smax) {
-    const int ns = span_count(ncol), j = blockIdx.x;
+    const uint2* __restrict__ spans, int nrow, int ncol, int slice0,
+    double center, unsigned* __restrict__ smax) {
+    const int ns = span_count(ncol), j = slice0 + blockIdx.x;
     const uint2* sp = spans + (size_t)j * ns;
     bool any = false;
     for (int k = threadIdx.x; k < ns; k += 256) any |= sp[k].x != 0u;
@@ -451,7 +453,7 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
         const int row_end = wv % SHARE * WROWS + WROWS;
         const unsigned lane_at = (unsigned)(row0 * kGroup + n16) * sizeof(Raw);
         // (an idle last group repeats the one before it)
-        const int gr = min(grp + sg, ma.group_have - 1);
+        const int gr = min(grp + sg, ma.group_have - 1) - ma.group_op;
         Raw raw[RUN + EXTRA];
         // (pairs past the row's end are the next row's, or the buffer's zero
         // tail: finite, and their weights are zero)
@@ -770,6 +772,15 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 int groups_of(int nslice) { return (nslice + kGroup - 1) / kGroup; }
 int planes_of(int dtype) { return dtype == ATH_F32 ? 2 : 1; }
 
+// Slice groups split and summed at a time: as many pairs as 2 GiB of split
+// samples hold, so that the workspace stays small beside a large stack (64 x
+// 1801 x 2560 takes 1.2 GB).
+int part_groups(int planes, int nrow, int ncol, int groups) {
+    const size_t bytes = (size_t)nrow * ((ncol + 1) / 2) * kGroup * 4 * planes;
+    const size_t n = ((size_t)2 << 30) / bytes / 2 * 2;
+    return (int)std::min<size_t>(groups, std::max<size_t>(n, 2));
+}
+
 template <typename T, int PL>
 int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
                hipStream_t s) {
@@ -790,7 +801,8 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
     ma.scaled = dtype != ATH_F16;
     ma.npair = npair;
     ma.pos0 = a.center + kPosMagic;
-    const size_t nop = (size_t)groups * kGroup * a.nrow * npair * PL;
+    const int part = part_groups(PL, a.nrow, a.ncol, groups);
+    const size_t nop = (size_t)part * kGroup * a.nrow * npair * PL;
     const int ntail = kTailPairs * kGroup * PL;
     const T* sino = static_cast<const T*>(a.sino);
     hipLaunchKernelGGL(trig_kernel,
@@ -808,40 +820,47 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
                        dim3(256), 0, s, sino, a.nrow, a.nslice, a.ncol, smax);
     st = check_hip(hipGetLastError(), "slice_max_kernel launch");
     if (st != ATH_OK) return st;
-    hipLaunchKernelGGL((split_kernel<T, PL>),
-                       dim3((unsigned)((a.ncol + 127) / 128),
-                            (unsigned)a.nrow, (unsigned)groups),
-                       dim3(256), 0, s, sino, a.nrow, a.nslice, a.ncol, npair,
-                       smax, ma.scaled, spans, op);
-    st = check_hip(hipGetLastError(), "split_kernel launch");
-    if (st != ATH_OK) return st;
-    if (ma.scaled) {
-        hipLaunchKernelGGL(range_kernel, dim3((unsigned)a.nslice), dim3(256),
-                           0, s, spans, a.nrow, a.ncol, a.center, smax);
-        st = check_hip(hipGetLastError(), "range_kernel launch");
+    for (int g0 = 0; g0 < groups; g0 += part) {
+        const int n = std::min(part, groups - g0);
+        const int slice0 = g0 * kGroup;
+        hipLaunchKernelGGL((split_kernel<T, PL>),
+                           dim3((unsigned)((a.ncol + 127) / 128),
+                                (unsigned)a.nrow, (unsigned)n),
+                           dim3(256), 0, s, sino, a.nrow, a.nslice, a.ncol,
+                           npair, g0, smax, ma.scaled, spans, op);
+        st = check_hip(hipGetLastError(), "split_kernel launch");
         if (st != ATH_OK) return st;
-    }
-    ma.group0 = 0;
-    ma.group_have = groups;
-    // Pairs of groups; a last odd group by itself unless an idle one beside
-    // it is cheaper, which it is where the launch does not fill the chip
-    // twice (rounds of 256 workgroups, at the measured 0.69 against 0.88 us
-    // per angle)
-    int pairs = groups / 2;
-    if (groups & 1) {
-        const double with = rounds_of<2>(a.ncol, pairs + 1) * 0.69;
-        const double apart = rounds_of<2>(a.ncol, pairs) * 0.69 +
-                             rounds_of<1>(a.ncol, 1) * 0.88;
-        if (with < apart) ++pairs;
-    }
-    if (pairs) {
-        st = launch_matrix<PL, 2>(a, ma, 2 * pairs, s);
-        if (st != ATH_OK) return st;
-        ma.group0 = 2 * pairs;
-    }
-    if (groups > 2 * pairs) {
-        st = launch_matrix<PL, 1>(a, ma, 1, s);
-        if (st != ATH_OK) return st;
+        if (ma.scaled) {
+            hipLaunchKernelGGL(
+                range_kernel,
+                dim3((unsigned)std::min(n * kGroup, a.nslice - slice0)),
+                dim3(256), 0, s, spans, a.nrow, a.ncol, slice0, a.center,
+                smax);
+            st = check_hip(hipGetLastError(), "range_kernel launch");
+            if (st != ATH_OK) return st;
+        }
+        ma.group0 = ma.group_op = g0;
+        ma.group_have = g0 + n;
+        // Pairs of groups; a last odd group by itself unless an idle one
+        // beside it is cheaper, which it is where the launch does not fill the
+        // chip twice (rounds of 256 workgroups, at the measured 0.69 against
+        // 0.88 us per angle)
+        int pairs = n / 2;
+        if (n & 1) {
+            const double with = rounds_of<2>(a.ncol, pairs + 1) * 0.69;
+            const double apart = rounds_of<2>(a.ncol, pairs) * 0.69 +
+                                 rounds_of<1>(a.ncol, 1) * 0.88;
+            if (with < apart) ++pairs;
+        }
+        if (pairs) {
+            st = launch_matrix<PL, 2>(a, ma, 2 * pairs, s);
+            if (st != ATH_OK) return st;
+            ma.group0 += 2 * pairs;
+        }
+        if (n > 2 * pairs) {
+            st = launch_matrix<PL, 1>(a, ma, 1, s);
+            if (st != ATH_OK) return st;
+        }
     }
     // slices with non-finite or huge samples (workgroups of others leave at
     // once)
@@ -856,11 +875,13 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
 size_t back_projection_matrix_workspace(int dtype, int nrow, int nslice,
                                         int ncol) {
     const size_t groups = groups_of(nslice);
+    const size_t part =
+        part_groups(planes_of(dtype), nrow, ncol, groups_of(nslice));
     return align256(groups * kGroup * (1 + 2 * (size_t)span_count(ncol)) *
                     sizeof(unsigned)) +
            align256((size_t)nrow * sizeof(float2)) +
-           (groups * nrow * (size_t)((ncol + 1) / 2) + kTailPairs) * kGroup *
-               4 * planes_of(dtype);
+           (part * nrow * (size_t)((ncol + 1) / 2) + kTailPairs) * kGroup * 4 *
+               planes_of(dtype);
 }
 
 int back_projection_matrix(const BpArgs& a, int dtype, int acc, void* work,

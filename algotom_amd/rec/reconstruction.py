@@ -330,7 +330,12 @@ def _backproject_matrix(filt_t, angles, center, acc, edge_pad=False,
         raise ValueError("!!!Number of angles is not the same as the row "
                          "number of the sinogram!!!")
     out = torch.empty((ncol, nslice, ncol), dtype=torch.float32, device=dev)
-    work = _matrix_workspace(nrow, nslice, ncol, filt_t.dtype, dev)
+    try:
+        work = _matrix_workspace(nrow, nslice, ncol, filt_t.dtype, dev)
+    except torch.OutOfMemoryError:
+        del out
+        return _backproject_stack(filt_t, ang, center, acc, edge_pad,
+                                  mask_radius, apply_scale)
     nat.check(nat.load().ath_back_projection_matrix(
         nat.ptr(filt_t), nat.dtype_code(filt_t.dtype), nrow, nslice, ncol,
         nat.ptr(ang), float(np.float32(center)), int(bool(edge_pad)),

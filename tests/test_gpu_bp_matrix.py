@@ -113,6 +113,34 @@ def test_slice_bits_do_not_depend_on_the_tile_shape(ncol, nrow, center, edge):
     assert torch.equal(full[:, 16:], pair)
 
 
+def test_large_stacks_in_parts(monkeypatch):
+    """A stack of more than 2 GiB of split samples is summed in parts: same
+    bits, bounded workspace; without room for it the vector kernel's."""
+    import torch
+    from algotom_amd import _native as nat
+    from algotom_amd.rec import reconstruction as rec
+    nrow, nslice, ncol = 4096, 1100, 128     # 64 + 5 groups
+    size = nat.load().ath_back_projection_matrix_workspace_bytes
+    assert size(nat.ATH_F32, nrow, nslice, ncol) < (2 << 30) + (1 << 24)
+    assert size(nat.ATH_F32, nrow, 32, ncol) < (65 << 20)
+    x, ang = _case(ncol, nrow, nslice, np.pi, 2)
+    x[3, 1030, 5] = float("inf")
+    full = rec._backproject_matrix(x, ang, 63.7, 1)
+    for j0, j1 in ((0, 7), (1008, 1040), (1088, 1100)):
+        part = rec._backproject_matrix(x[:, j0:j1].contiguous(), ang, 63.7, 1)
+        assert np.array_equal(part.cpu().numpy(),
+                              full[:, j0:j1].cpu().numpy(), equal_nan=True)
+
+    def no_room(*args):
+        raise torch.OutOfMemoryError("no room")
+
+    y = x[:, :20].contiguous()
+    del x, full
+    monkeypatch.setattr(rec, "_matrix_workspace", no_room)
+    assert torch.equal(rec._backproject_matrix(y, ang, 63.7, 1),
+                       rec._backproject_stack(y, ang, 63.7, 1))
+
+
 def test_scales_and_special_samples():
     """Slices of any magnitude keep their relative error; an all-zero slice
     gives zeros; slices with inf, NaN or huge samples are exactly the vector
