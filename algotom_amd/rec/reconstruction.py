@@ -321,7 +321,9 @@ def _matrix_workspace(nrow, nslice, ncol, dtype, dev):
 
 def _backproject_matrix(filt_t, angles, center, acc, edge_pad=False,
                         mask_radius=-1.0, apply_scale=False):
-    """_backproject_stack on the matrix cores (ath_back_projection_matrix)."""
+    """_backproject_stack on the matrix cores (ath_back_projection_matrix); a
+    stack that leaves no room for the split samples (2 GiB, or 32 slices of
+    it) gets the vector kernel, which needs none."""
     import torch
     dev = filt_t.device
     nrow, nslice, ncol = filt_t.shape
@@ -353,6 +355,7 @@ _to_host = _host.to_host
 # input plus output.
 _STREAM_MIN = 256 << 20
 _CHUNK_BYTES = 384 << 20
+_GROUP_BYTES = 24 << 30
 
 
 def _streams(sinogram, out_width, out_itemsize=4):
@@ -361,15 +364,27 @@ def _streams(sinogram, out_width, out_itemsize=4):
     return nslice > 1 and nbytes >= _STREAM_MIN
 
 
-def _chunk_ranges(nslice, slice_bytes):
+def _chunk_ranges(nslice, slice_bytes, matrix_rows=0):
+    """Chunks of about _CHUNK_BYTES.  matrix_rows: the stack's angles where it
+    is summed on the matrix cores.  Their kernel always computes whole groups
+    of 16 slices, at about 16 updates per ps; a chunk's ``per`` slices move at
+    about 45 GB/s, so that up to 90 ``per`` angles the transfers take longer
+    and hide the idle part of a group (20 x 721 x 2560 from and to the host:
+    29 ms in chunks of 8, 33 in chunks of 16).  With more angles the chunks
+    are whole groups (16 x 1801 x 7192: 203 ms, 1687 in chunks of one
+    slice; 64 x 1801 x 2560: 89 ms, 142 in chunks of 8), as far as
+    _GROUP_BYTES hold one."""
     per = max(1, min(nslice, _CHUNK_BYTES // max(1, slice_bytes)))
     if per >= 8:
         per -= per % 4
+    if matrix_rows > 100 * per:
+        per = max(per - per % 16,
+                  min(16, max(1, _GROUP_BYTES // max(1, slice_bytes))))
     return [(j, min(nslice, j + per)) for j in range(0, nslice, per)]
 
 
 def _stream_numpy(sinogram, out_shape, run, apply_log, dev, allow_f64,
-                  out_dtype=np.float32):
+                  out_dtype=np.float32, matrix=False):
     """``run`` over slice chunks of a host (nrow, nslice, ncol) stack with
     overlapped transfers; returns the new (a, nslice, b) array.  With
     ``apply_log`` the values <= 0 are set to 1 on the device, and, as
@@ -382,7 +397,7 @@ def _stream_numpy(sinogram, out_shape, run, apply_log, dev, allow_f64,
     out = np.empty(out_shape, dtype=out_dtype)
     nrow, nslice, ncol = a.shape
     ranges = _chunk_ranges(nslice, 4 * nrow * ncol + out.itemsize
-                           * out_shape[0] * out_shape[2])
+                           * out_shape[0] * out_shape[2], nrow * matrix)
     flags = []
 
     def step(part):
@@ -576,9 +591,8 @@ def fbp_reconstruction(sinogram, center, angles=None, ratio=1.0,
     storage = _storage_dtype(precision)
     ang = _angles_device(angles, dev)
     # decided for the whole stack, so that a streamed one keeps its bits
-    project = (_backproject_matrix
-               if _matrix_stack(nrow, num_sino, ncol, acc, storage)
-               else _backproject_stack)
+    matrix = _matrix_stack(nrow, num_sino, ncol, acc, storage)
+    project = _backproject_matrix if matrix else _backproject_stack
 
     def run(sino_t):
         filt = _filter_stack(sino_t, pad, pad_mode, apply_log, taps, storage)
@@ -587,7 +601,8 @@ def fbp_reconstruction(sinogram, center, angles=None, ratio=1.0,
 
     if as_numpy and input_3d and _streams(sinogram, ncol):
         return _stream_numpy(sinogram, (ncol, num_sino, ncol), run,
-                             apply_log, dev, allow_f64=True)
+                             apply_log, dev, allow_f64=True,
+                             matrix=matrix)
     sino_t = _to_device(sinogram, dev).reshape(nrow, num_sino, ncol)
     if apply_log:
         _clamp_nonpositive_device(sinogram, sino_t)
@@ -839,9 +854,8 @@ def bpf_reconstruction(sinogram, center, angles=None, ratio=1.0,
         name_key = ("window", regen)
     acc = nat.ACC_F64 if (gpu and num_sino == 1) else nat.ACC_F32SEQ
     ang = _angles_device(angles, dev)
-    project = (_backproject_matrix
-               if _matrix_stack(nrow, num_sino, ncol, acc, torch.float32)
-               else _backproject_stack)
+    matrix = _matrix_stack(nrow, num_sino, ncol, acc, torch.float32)
+    project = _backproject_matrix if matrix else _backproject_stack
 
     def run(sino_t):
         if apply_log:
@@ -862,7 +876,8 @@ def bpf_reconstruction(sinogram, center, angles=None, ratio=1.0,
 
     if as_numpy and input_3d and _streams(sinogram, ncol):
         return _stream_numpy(sinogram, (ncol, num_sino, ncol), run,
-                             apply_log, dev, allow_f64=False)
+                             apply_log, dev, allow_f64=False,
+                             matrix=matrix)
     sino_t = _to_device(sinogram, dev, allow_f64=False).reshape(
         nrow, num_sino, ncol)
     if apply_log:

@@ -47,6 +47,23 @@ def test_streamed_equals_device(small_chunks, method):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("method", ["fbp", "bpf"])
+@pytest.mark.parametrize("ncol,sizes", [(256, [3] * 13 + [1]),
+                                        (512, [16, 16, 8])])
+def test_streamed_matrix_stack_equals_device(small_chunks, method, ncol,
+                                             sizes):
+    """Stacks on the matrix cores, in chunks below a group of 16 slices (few
+    angles for their size) and in whole groups."""
+    rec = small_chunks
+    fn = getattr(rec, method + "_reconstruction")
+    sino = _stack(181, 40, ncol, 5)
+    ranges = rec._chunk_ranges(40, 4 * 181 * ncol + 4 * ncol * ncol, 181)
+    assert [b - a for a, b in ranges] == sizes
+    got = fn(sino, ncol / 2 - 0.7, apply_log=True)
+    want = fn(_device(sino), ncol / 2 - 0.7, apply_log=True).cpu().numpy()
+    assert np.array_equal(got, want)
+
+
 def test_streamed_fbp_input_kinds(small_chunks, tmp_path):
     """A strided view, float64, uint16 and a memory map."""
     rec = small_chunks

@@ -29,6 +29,20 @@ def test_stack_chunks_are_eight_slices():
     assert rec._chunk_ranges(64, 4 * (1801 * 2560 + 2560 * 2560))[0] == (0, 8)
 
 
+@pytest.mark.parametrize("nslice,nrow,ncol,sizes", [
+    (40, 1801, 7192, [16, 16, 8]),           # 1 slice in _CHUNK_BYTES
+    (6, 1801, 5120, [6]),
+    (64, 1801, 2560, [16] * 4),              # 8
+    (20, 721, 2560, [8, 8, 4]),              # transfers hide the idle half
+    (128, 901, 1024, [48, 48, 32]),
+    (40, 100, 16384, [1] * 40),              # few angles
+    (9, 60000, 32768, [2, 2, 2, 2, 1])])     # no group in _GROUP_BYTES
+def test_matrix_stacks_stream_in_whole_groups(nslice, nrow, ncol, sizes):
+    ranges = rec._chunk_ranges(nslice, 4 * (nrow * ncol + ncol * ncol), nrow)
+    assert [b - a for a, b in ranges] == sizes
+    assert ranges[0][0] == 0 and ranges[-1][1] == nslice
+
+
 def test_streaming_threshold():
     small = np.zeros((10, 3, 20), np.float32)
     assert not rec._streams(small, 20)
