@@ -308,7 +308,9 @@ def _matrix_stack(nrow, nslice, ncol, acc, dtype):
     if acc == nat.ACC_F32SEQ:
         return nslice > 5
     if acc == nat.ACC_F32:
-        return (nslice > 8 and ncol >= 1000) or (nslice > 16 and ncol >= 512)
+        if ncol >= 1000:
+            return nslice > 12
+        return ncol >= 512 and nslice > (16 if ncol == 512 else 24)
     return False
 
 
@@ -364,6 +366,13 @@ def _streams(sinogram, out_width, out_itemsize=4):
     return nslice > 1 and nbytes >= _STREAM_MIN
 
 
+def _matrix_chunk(per, slice_bytes):
+    """``per`` slices as whole groups of the matrix kernel: rounded down to
+    16 slices, or up to one group as far as _GROUP_BYTES hold it."""
+    return max(per - per % 16,
+               min(16, max(per, _GROUP_BYTES // max(1, slice_bytes))))
+
+
 def _chunk_ranges(nslice, slice_bytes, matrix_rows=0):
     """Chunks of about _CHUNK_BYTES.  matrix_rows: the stack's angles where it
     is summed on the matrix cores.  Their kernel always computes whole groups
@@ -372,14 +381,12 @@ def _chunk_ranges(nslice, slice_bytes, matrix_rows=0):
     and hide the idle part of a group (20 x 721 x 2560 from and to the host:
     29 ms in chunks of 8, 33 in chunks of 16).  With more angles the chunks
     are whole groups (16 x 1801 x 7192: 203 ms, 1687 in chunks of one
-    slice; 64 x 1801 x 2560: 89 ms, 142 in chunks of 8), as far as
-    _GROUP_BYTES hold one."""
+    slice; 64 x 1801 x 2560: 89 ms, 142 in chunks of 8)."""
     per = max(1, min(nslice, _CHUNK_BYTES // max(1, slice_bytes)))
     if per >= 8:
         per -= per % 4
     if matrix_rows > 100 * per:
-        per = max(per - per % 16,
-                  min(16, max(1, _GROUP_BYTES // max(1, slice_bytes))))
+        per = _matrix_chunk(per, slice_bytes)
     return [(j, min(nslice, j + per)) for j in range(0, nslice, per)]
 
 
@@ -422,6 +429,12 @@ def _finish(out_t, as_numpy):
 
 
 _PRECISIONS = {None: None, "fp32": "fp32", "fp16": "fp16", "bf16": "bf16"}
+
+
+def _accumulation(nslice, gpu, precision):
+    if precision is not None:
+        return nat.ACC_F32
+    return nat.ACC_F64 if (gpu and nslice == 1) else nat.ACC_F32SEQ
 
 
 def _storage_dtype(precision):
@@ -558,6 +571,15 @@ def fbp_reconstruction(sinogram, center, angles=None, ratio=1.0,
         Square array(s): (ncol, ncol) for 2D input, (ncol, nslice, ncol)
         for 3D input, float32.
     """
+    return _fbp(sinogram, center, angles, ratio, ramp_win, filter_name, pad,
+                pad_mode, apply_log, gpu, precision)
+
+
+def _fbp(sinogram, center, angles=None, ratio=1.0, ramp_win=None,
+         filter_name="hann", pad=None, pad_mode="edge", apply_log=True,
+         gpu=True, precision=None, volume_slices=None):
+    """fbp_reconstruction; volume_slices: the slices of the volume that the
+    stack is a part of, which then decides whether the matrix cores sum it."""
     if precision not in _PRECISIONS:
         raise ValueError("precision must be None, 'fp32', 'fp16' or 'bf16'")
     shape = tuple(sinogram.shape)
@@ -584,14 +606,15 @@ def fbp_reconstruction(sinogram, center, angles=None, ratio=1.0,
     if pad is None:
         pad = min(int(0.15 * ncol), 150)
     taps = _window_taps(ramp_win, nrow, ncol + 2 * pad, filter_name)
-    if precision is None:
-        acc = nat.ACC_F64 if (gpu and num_sino == 1) else nat.ACC_F32SEQ
-    else:
-        acc = nat.ACC_F32
     storage = _storage_dtype(precision)
     ang = _angles_device(angles, dev)
-    # decided for the whole stack, so that a streamed one keeps its bits
-    matrix = _matrix_stack(nrow, num_sino, ncol, acc, storage)
+    # decided for the whole stack or volume, so that the bits of a streamed one
+    # do not depend on its chunks
+    whole = volume_slices or num_sino
+    acc = _accumulation(whole, gpu, precision)
+    matrix = _matrix_stack(nrow, whole, ncol, acc, storage)
+    if not matrix:
+        acc = _accumulation(num_sino, gpu, precision)
     project = _backproject_matrix if matrix else _backproject_stack
 
     def run(sino_t):

@@ -28,7 +28,9 @@ def reconstruct_volume_360(sino_360, cor, chunk=16, angles=None, ratio=1.0,
     Returns (recon, new_cor) with recon of shape (width, nslice, width),
     width = max(2*ncol - overlap, total_width).  ``angles`` are those of the
     converted 180-degree sinogram (default: the reference's
-    deg2rad(linspace(0, 180, nrow_360 // 2 + 1))).
+    deg2rad(linspace(0, 180, nrow_360 // 2 + 1))).  ``chunk``: slices at a
+    time; where the volume is summed on the matrix cores, whole groups of 16 of
+    them, and the result does not depend on it.
     """
     import torch
     dev = nat.device()
@@ -47,11 +49,15 @@ def reconstruct_volume_360(sino_360, cor, chunk=16, angles=None, ratio=1.0,
     def run(part):
         stitched, _ = conversion.convert_sinogram_360_to_180(
             part, cor, total_width=width)
-        return rec.fbp_reconstruction(stitched, new_cor, ang, ratio=ratio,
-                                      filter_name=filter_name, pad=pad,
-                                      pad_mode=pad_mode, apply_log=apply_log,
-                                      precision=precision)
+        return rec._fbp(stitched, new_cor, ang, ratio=ratio,
+                        filter_name=filter_name, pad=pad, pad_mode=pad_mode,
+                        apply_log=apply_log, precision=precision,
+                        volume_slices=nslice)
 
+    if rec._matrix_stack(n180, nslice, width,
+                         rec._accumulation(nslice, True, precision),
+                         rec._storage_dtype(precision)):
+        chunk = rec._matrix_chunk(chunk, 4 * (nrow * ncol + width * width))
     ranges = [(j0, min(nslice, j0 + chunk)) for j0 in range(0, nslice, chunk)]
     if out is not None and not rec._is_tensor(out) \
             and not rec._is_tensor(sino_360):

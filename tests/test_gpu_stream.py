@@ -117,6 +117,23 @@ def test_streamed_volume_360(tmp_path):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("precision", [None, "fp32", "fp16"])
+def test_volume_360_does_not_depend_on_its_chunks(precision):
+    """Chunks of any size, the last one of a single slice or a few, give the
+    slices of one volume the same bits (20 slices: on the matrix cores)."""
+    from algotom_amd.rec import reconstruction as rec
+    from algotom_amd.rec import volume
+    sino = _device(_stack(361, 21, 290, 6))
+    kw = dict(apply_log=True, precision=precision)
+    want, _ = volume.reconstruct_volume_360(sino, 29.5, chunk=21, **kw)
+    n180, _, width = 181, 21, want.shape[0]
+    if precision is None:
+        assert rec._matrix_stack(n180, 21, width, 1, rec._storage_dtype(None))
+    for chunk in (1, 3, 16, 20, 64):
+        got, _ = volume.reconstruct_volume_360(sino, 29.5, chunk=chunk, **kw)
+        assert np.array_equal(got.cpu().numpy(), want.cpu().numpy()), chunk
+
+
 @pytest.mark.parametrize("rows,stage", [(37, 1 << 16), (5, 1 << 12)])
 def test_stager_blocks(rows, stage):
     """Uploads and downloads split into many staging blocks, from and into
