@@ -286,23 +286,43 @@ def _matrix_stack(nrow, nslice, ncol, acc, dtype):
     (ath_back_projection_matrix) instead of the vector kernel.
 
     Float32 sums only, and only where the matrix path is both faster and no
-    further from float64: its rounding is that of one truncated product sum
-    per 4 angles, which a float32 sum after every angle exceeds from about
-    100 angles on (white noise, 181 angles: 1.9e-7 against 2.4e-7 relative,
-    1801 angles: 4.2e-7 against 7.4e-7; 37 angles: 1.6e-7 against 1.1e-7).
-    16-bit storage is closer to float64 at any number of angles.
+    further from float64.  For float32 samples that is from 128 angles on: its
+    error is below that of a float32 sum after every angle from about 100 on
+    (relative, white noise: 37 angles 1.6e-7 against 1.1e-7, 128 angles 1.8e-7
+    against 2.0e-7, 1801 angles 4.3e-7 against 7.4e-7).  16-bit storage is
+    closer to float64 at any number of angles.
 
-    Speed (361 angles, matrix against vector): a matrix workgroup always
-    computes 16 slices, the vector kernel's cost goes in steps of 4 (8 for
-    16-bit).  Per-angle sums 604 against 913 us at 6 x 1023 columns, 597
-    against 536 at 4; float32 1359 against 1387 us at 11 x 1500, 598 against
-    565 at 16 x 768, 250 against 383 at 17 x 512; float16 509 against 786 us
-    at 11 x 1023, 498 against 487 at 8."""
+    Speed, as matrix time over vector time (with the mask, 64 to 2560 columns).
+    A matrix workgroup always computes 16 slices, two groups in 32 x 32 tiles,
+    one in 64 x 32, a step of 4 angles every 2.8 to 3.5 us; the
+    vector kernel's cost goes in steps of 4 slices (8 for 16-bit).
+    * Per-angle sums, 128 and more angles: 0.55 to 0.91 at 6 slices, less at
+      more, at every width.  (5 slices 0.51 to 0.91 too: stacks of up to 5
+      keep the reference kernel's bits.)
+    * float32: 1000 columns and more 0.80 to 0.96 at 16 slices, 0.77 to 1.05
+      at 17, but 0.94 to 1.19 at 9 to 12; 512 columns 0.62 to 0.93 at 17,
+      0.86 to 1.18 at 16; 640 and 768 columns 0.96 to 1.16 at 17, 0.80 to 1.01
+      at 24, 0.59 to 0.85 at 32 (640 columns at 48 slices, three groups of
+      which two fill half a round of the chip, 1.04 to 1.19); fewer columns
+      0.94 to 1.7.
+    * 16-bit: 1000 columns and more 0.70 to 0.99 from 9 slices and 64 angles
+      on (37 angles up to 1.08, 8 angles 1.05 to 1.4); up to 512 columns 0.42
+      to 0.84 from 256 angles on, 0.56 to 0.99 at 128 angles and 9 to 24 slices
+      (32 and 48 slices 0.63 to 1.10), 64 angles up to 1.22; 640 and 768
+      columns 1.0 to 1.5 at 9 to 16 slices, 0.59 to 0.99 at 17 to 32."""
     import torch
     if ncol > 32768 or nrow > 65535 or nslice > 65535:
         return False
     if dtype in (torch.float16, torch.bfloat16):
-        return acc == nat.ACC_F32 and nslice > 8
+        if acc != nat.ACC_F32 or nslice <= 8 or nrow < 64:
+            return False
+        if ncol >= 1000:
+            return True
+        if nrow < 128:
+            return False
+        if ncol > 512:
+            return nslice > 16 and (nslice <= 32 or nrow >= 256)
+        return nslice <= 24 or nrow >= 256
     if dtype != torch.float32 or nrow < 128:
         return False
     if acc == nat.ACC_F32SEQ:

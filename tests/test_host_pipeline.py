@@ -75,3 +75,37 @@ def test_to_host_of_host_tensor():
     t = torch.arange(12, dtype=torch.float32).reshape(3, 4)
     out = _host.to_host(t)
     assert isinstance(out, np.ndarray) and np.array_equal(out, t.numpy())
+
+
+@pytest.mark.parametrize("nrow,nslice,ncol,f32seq,f32,f16", [
+    (128, 6, 64, True, False, False),
+    (127, 64, 2560, False, False, True),
+    (128, 5, 2560, False, False, False),
+    (361, 9, 640, True, False, False),       # half-filled rounds of the chip
+    (361, 17, 640, True, False, True),
+    (361, 25, 640, True, True, True),
+    (128, 48, 640, True, True, False),
+    (361, 16, 512, True, False, True),
+    (361, 17, 512, True, True, True),
+    (361, 12, 1024, True, False, True),
+    (361, 13, 1024, True, True, True),
+    (128, 24, 256, True, False, True),
+    (128, 25, 256, True, False, False),
+    (256, 48, 256, True, False, True),
+    (64, 9, 1000, False, False, True),
+    (63, 9, 1000, False, False, False),
+    (64, 9, 512, False, False, False),
+    (1801, 64, 32769, False, False, False),
+    (65536, 64, 2560, False, False, False)])
+def test_matrix_rule(nrow, nslice, ncol, f32seq, f32, f16):
+    """Where stacks go to the matrix cores: only where they measured faster
+    than the vector kernel there."""
+    import torch
+    from algotom_amd import _native as nat
+    rule = rec._matrix_stack
+    assert rule(nrow, nslice, ncol, nat.ACC_F32SEQ, torch.float32) == f32seq
+    assert rule(nrow, nslice, ncol, nat.ACC_F32, torch.float32) == f32
+    for dtype in (torch.float16, torch.bfloat16):
+        assert rule(nrow, nslice, ncol, nat.ACC_F32, dtype) == f16
+        assert not rule(nrow, nslice, ncol, nat.ACC_F32SEQ, dtype)
+    assert not rule(nrow, nslice, ncol, nat.ACC_F64, torch.float32)
