@@ -53,6 +53,10 @@ SIGNATURES = (
     ("ath_back_projection_matrix_workspace_bytes", _S, [_I, _I, _I, _I]),
     ("ath_back_projection_matrix", _I, [_P, _I, _I, _I, _I, _P, _F, _I, _I,
                                         _D, _I, _P, _P, _S, _P]),
+    ("ath_matrix_batch_plan_bytes", _S, [_I]),
+    ("ath_matrix_batch_workspace_bytes", _S, [_P, _I, _I]),
+    ("ath_matrix_batch_plan", _I, [_P, _I, _I, _I, _P, _S, _P, _S]),
+    ("ath_back_projection_matrix_batched", _I, [_P, _P, _P]),
     ("ath_back_projection_with_derivative", _I, [_P, _I, _I, _I, _P, _F,
                                                  _I, _D, _I, _P, _P, _P]),
     ("ath_back_projection_tiled", _I, [_P, _I, _I, _I, _I, _P, _F, _I, _I,

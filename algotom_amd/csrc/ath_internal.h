@@ -131,6 +131,25 @@ size_t back_projection_matrix_workspace(int dtype, int nrow, int nslice,
                                         int ncol);
 int back_projection_matrix(const BpArgs& a, int dtype, int acc, void* work,
                            hipStream_t stream);
+// many stacks at once: a plan of matrix_batch_plan_bytes(jobs), begun and
+// then given its stacks one by one, each with matrix_batch_job_bytes of
+// workspace; run from the host plan and its copy in device memory
+size_t matrix_batch_plan_bytes(int njobs);
+size_t matrix_batch_job_bytes(int dtype, int nrow, int nslice, int ncol);
+void matrix_batch_begin(void* plan, int dtype, int acc);
+int matrix_batch_add(void* plan, const BpArgs& a, void* work);
+int back_projection_matrix_batched(const void* plan, const void* plan_dev,
+                                   hipStream_t stream);
+// the slices above their threshold (BpArgs::only_above) of many stacks, whose
+// jobs in device memory lie `stride` bytes apart
+struct BpRedoJob {
+    BpArgs a;
+    unsigned begin;  // first workgroup
+};
+long long redo_tiles(int nslice, int ncol);
+int back_projection_redo(const BpRedoJob* jobs, size_t stride, int njobs,
+                         unsigned blocks, int dtype, int acc,
+                         hipStream_t stream);
 
 // ---- forward projection = adjoint of the back-projection ------------------
 // largest FFT length of the 1D ramp filter and of its adjoint

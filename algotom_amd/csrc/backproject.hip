@@ -757,6 +757,37 @@ __global__ __launch_bounds__(kThreads) void bp_tiled_kernel(
     bp_tile<MODE, SB, PY, A, Tin>(a, tx, ty, grp, sh);
 }
 
+// bp_tiled_kernel for the marked slices of many stacks; workgroups of others
+// leave at once.
+template <int MODE, int SB, int PY, int A, typename Tin>
+__global__ __launch_bounds__(kThreads) void bp_redo_kernel(
+    const char* __restrict__ jobs, size_t stride, int njobs) {
+    __shared__ BpShared<typename Mode<MODE>::Rec, SB, A,
+                        mode_span<Mode<MODE>>(kTileX, 4 * PY)> sh;
+    const auto job = [&](int i) -> const BpRedoJob& {
+        return *reinterpret_cast<const BpRedoJob*>(jobs + i * stride);
+    };
+    int lo = 0, hi = njobs - 1;  // last job with begin <= block
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (job(mid).begin <= blockIdx.x) lo = mid;
+        else hi = mid - 1;
+    }
+    const BpArgs a = job(lo).a;
+    const int tiles_x = (a.ncol + kTileX - 1) / kTileX;
+    const int tiles_y = (a.ncol + 4 * PY - 1) / (4 * PY);
+    int bid = blockIdx.x - job(lo).begin;
+    const int tx = bid % tiles_x;
+    bid /= tiles_x;
+    const int ty = bid % tiles_y;
+    const int grp = bid / tiles_y;
+    bool any = false;
+    for (int j = grp * SB; j < min(a.nslice, grp * SB + SB); ++j)
+        any = any || a.only_above[j] > a.above;
+    if (!any) return;
+    bp_tile<MODE, SB, PY, A, Tin>(a, tx, ty, grp, sh);
+}
+
 // Persistent kernel over a work list of (stack, tile) items from many stacks
 // of different widths, angle counts and centres.  Workgroups take the next
 // item from a device counter (reset by the preceding reset_counter launch)
@@ -1068,6 +1099,43 @@ int back_projection_batched(const ath_bp_job* jobs, int njobs,
         return batched_config<kAccB16, __hip_bfloat16>(
             jobs, njobs, total, sb, py, nblocks, counter, s);
     return set_error(ATH_ERR_INVALID_ARG, "back-projection: bad sinogram dtype");
+}
+
+namespace {
+
+// one configuration for every depth: the bits do not depend on it
+constexpr int kRedoSlices = 4, kRedoRows = 8;
+
+template <int MODE, typename Tin>
+int launch_redo(const BpRedoJob* jobs, size_t stride, int njobs,
+                unsigned blocks, hipStream_t s) {
+    hipLaunchKernelGGL(
+        (bp_redo_kernel<MODE, kRedoSlices, kRedoRows,
+                        angle_block<MODE, kRedoSlices, kRedoRows>(), Tin>),
+        dim3(blocks), dim3(kThreads), 0, s,
+        reinterpret_cast<const char*>(jobs), stride, njobs);
+    return check_hip(hipGetLastError(), "bp_redo_kernel launch");
+}
+
+}  // namespace
+
+long long redo_tiles(int nslice, int ncol) {
+    return (long long)((ncol + kTileX - 1) / kTileX) *
+           ((ncol + 4 * kRedoRows - 1) / (4 * kRedoRows)) *
+           ((nslice + kRedoSlices - 1) / kRedoSlices);
+}
+
+int back_projection_redo(const BpRedoJob* jobs, size_t stride, int njobs,
+                         unsigned blocks, int dtype, int acc, hipStream_t s) {
+    if (dtype == ATH_F16)
+        return launch_redo<kAccH16, __half>(jobs, stride, njobs, blocks, s);
+    if (dtype == ATH_BF16)
+        return launch_redo<kAccB16, __hip_bfloat16>(jobs, stride, njobs,
+                                                    blocks, s);
+    if (acc == ATH_ACC_F32SEQ)
+        return launch_redo<ATH_ACC_F32SEQ, float>(jobs, stride, njobs, blocks,
+                                                  s);
+    return launch_redo<ATH_ACC_F32, float>(jobs, stride, njobs, blocks, s);
 }
 
 int back_projection_naive(const BpArgs& a, int acc, hipStream_t s) {

@@ -119,16 +119,46 @@ constexpr int kTailPairs = 64;
 static_assert(kTailPairs >= Tile<1>::rows + 16, "tail");
 
 struct MatArgs {
-    const unsigned* op;     // split samples
-    const unsigned* smax;   // per slice: bits of max|s|
-    const float2* trig;     // per angle: cos, sin
+    unsigned* op;           // split samples
+    unsigned* smax;         // per slice: bits of max|s|
+    uint2* spans;           // per slice and span of columns, see split
+    float2* trig;           // per angle: cos, sin
+    size_t nop;             // entries of op (the zero tail follows)
+    double pos0;            // centre + kPosMagic
     int scaled;             // samples carry the power of two of smax
     int npair;              // column pairs per row
+    int nzero, ntail;       // words to clear from smax on, and of the tail
+    int max_rows;           // workgroups per slice that look for its maximum
     int group0, group_end;  // slice groups of the launch
     int group_op, group_have;  // slice groups that op holds
     unsigned patches_x, patches_y;
-    double pos0;            // centre + kPosMagic
 };
+
+// The kernels run one stack, whose MatJob is a launch argument, or many
+// (BATCH: jobs[0 .. njobs) in device memory, a workgroup's by its index).
+enum Stage { kClear, kMaxima, kSplit, kRange, kPairs, kSingle, kStages };
+struct MatJob {
+    BpRedoJob r;
+    MatArgs m;
+    unsigned begin[kStages];  // the job's first workgroup of a batch's launch
+};
+
+// the workgroup's job, and its number in it
+template <bool BATCH>
+__device__ __forceinline__ const MatJob& find_job(
+    const MatJob* __restrict__ jobs, int njobs, const MatJob& one, int stage,
+    unsigned& block) {
+    block = blockIdx.x;
+    if constexpr (!BATCH) return one;
+    int lo = 0, hi = njobs - 1;  // last job with begin <= block
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (jobs[mid].begin[stage] <= block) lo = mid;
+        else hi = mid - 1;
+    }
+    block -= jobs[lo].begin[stage];
+    return jobs[lo];
+}
 
 __device__ __forceinline__ double det_pos(double xc_c, double yc, double s,
                                           double cen) {
@@ -158,28 +188,35 @@ __device__ __forceinline__ float widen<__hip_bfloat16>(__hip_bfloat16 v) {
     return __bfloat162float(v);
 }
 
-__global__ void trig_kernel(const float* __restrict__ angles, int nrow,
-                            float2* __restrict__ trig,
-                            unsigned* __restrict__ zero, int nzero,
-                            unsigned* __restrict__ tail, int ntail) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nrow) {
-        const float th = -angles[i];
-        trig[i] = make_float2((float)cos((double)th), (float)sin((double)th));
+template <bool BATCH>
+__global__ __launch_bounds__(256) void clear_kernel(
+    const MatJob* __restrict__ jobs, int njobs, MatJob one) {
+    unsigned b;
+    const MatJob& job = find_job<BATCH>(jobs, njobs, one, kClear, b);
+    const MatArgs& m = job.m;
+    const int i = b * 256 + threadIdx.x;
+    if (i < job.r.a.nrow) {
+        const float th = -job.r.a.angles[i];
+        m.trig[i] =
+            make_float2((float)cos((double)th), (float)sin((double)th));
     }
-    if (i < nzero) zero[i] = 0u;
-    if (i < ntail) tail[i] = 0u;
+    if (i < m.nzero) m.smax[i] = 0u;
+    if (i < m.ntail) m.op[m.nop + i] = 0u;
 }
 
-// max|s| per slice: grid (row chunks, slices).  Integer order of the bit
+// max|s| per slice, max_rows workgroups each.  Integer order of the bit
 // patterns is the order of the magnitudes, with infinities and NaN on top.
-template <typename T>
+template <typename T, bool BATCH>
 __global__ __launch_bounds__(256) void slice_max_kernel(
-    const T* __restrict__ sino, int nrow, int nslice, int ncol,
-    unsigned* __restrict__ smax) {
-    const int j = blockIdx.y;
+    const MatJob* __restrict__ jobs, int njobs, MatJob one) {
+    unsigned b;
+    const MatJob& job = find_job<BATCH>(jobs, njobs, one, kMaxima, b);
+    const BpArgs& a = job.r.a;
+    const int nslice = a.nslice, ncol = a.ncol, step = job.m.max_rows;
+    const T* sino = static_cast<const T*>(a.sino);
+    const int j = b / step;
     unsigned m = 0u;
-    for (int r = blockIdx.x; r < nrow; r += gridDim.x) {
+    for (int r = b % step; r < a.nrow; r += step) {
         const T* row = sino + ((size_t)r * nslice + j) * ncol;
         for (int c = threadIdx.x; c < ncol; c += 256)
             m = max(m, __float_as_uint(fabsf(widen(row[c]))));
@@ -191,7 +228,7 @@ __global__ __launch_bounds__(256) void slice_max_kernel(
     __syncthreads();
     if (threadIdx.x == 0) {
         m = max(max(part[0], part[1]), max(part[2], part[3]));
-        if (m) atomicMax(&smax[j], m);
+        if (m) atomicMax(&job.m.smax[j], m);
     }
 }
 
@@ -201,16 +238,23 @@ __global__ __launch_bounds__(256) void slice_max_kernel(
 // are counted on the way for range_kernel: spans[slice][span] = (angles in
 // which the span's samples are mostly small, angles in which they are all
 // zero); ordinary slices have few of either and add nothing.
-template <typename T, int PL>
+template <typename T, int PL, bool BATCH>
 __global__ __launch_bounds__(256) void split_kernel(
-    const T* __restrict__ sino, int nrow, int nslice, int ncol, int npair,
-    int group_op, const unsigned* __restrict__ smax, int scaled, uint2* __restrict__ spans,
-    unsigned* __restrict__ op) {
+    const MatJob* __restrict__ jobs, int njobs, MatJob one) {
     constexpr int COLS = 128, SPANS = COLS / kSpanCols;
     __shared__ float tile[kGroup][COLS + 1];
     __shared__ unsigned count[SPANS][kGroup];  // not zero, large << 16
-    const int c0 = blockIdx.x * COLS, row = blockIdx.y;
-    const int g = group_op + blockIdx.z;
+    unsigned b;
+    const MatJob& job = find_job<BATCH>(jobs, njobs, one, kSplit, b);
+    const BpArgs& a = job.r.a;
+    const int nrow = a.nrow, nslice = a.nslice, ncol = a.ncol;
+    const int npair = job.m.npair, scaled = job.m.scaled;
+    const T* sino = static_cast<const T*>(a.sino);
+    const unsigned nblock = (ncol + COLS - 1) / COLS;
+    const int c0 = (int)(b % nblock) * COLS;
+    b /= nblock;
+    const int row = (int)(b % nrow);
+    const int gl = (int)(b / nrow), g = job.m.group_op + gl;
     const int tid = threadIdx.x;
     for (int e = tid; e < kGroup * COLS; e += 256) {
         const int n = e / COLS, c = c0 + e % COLS, j = g * kGroup + n;
@@ -222,11 +266,11 @@ __global__ __launch_bounds__(256) void split_kernel(
     if (tid < SPANS * kGroup) count[tid / kGroup][tid % kGroup] = 0u;
     __syncthreads();
     const int n = tid & 15, j = g * kGroup + n;
-    const unsigned bits = j < nslice ? smax[j] : 0u;
+    const unsigned bits = j < nslice ? job.m.smax[j] : 0u;
     const bool bad = bits > kMaxBits;  // redone by the vector kernel
     const int ex = scaled ? scale_exp(bits) : 0;
     unsigned* base =
-        op + (((size_t)blockIdx.z * nrow + row) * npair) * (kGroup * PL);
+        job.m.op + (((size_t)gl * nrow + row) * npair) * (kGroup * PL);
     for (int i = tid >> 4; i < COLS / 2; i += 16) {
         const int p = c0 / 2 + i;
         if (p >= npair) break;
@@ -257,7 +301,7 @@ __global__ __launch_bounds__(256) void split_kernel(
     const int sp = tid / kGroup;
     if (sp < SPANS && j < nslice && c0 + sp * kSpanCols < ncol) {
         const unsigned m = count[sp][n], some = m & 0xffffu, large = m >> 16;
-        uint2* at = spans + (size_t)j * span_count(ncol) +
+        uint2* at = job.m.spans + (size_t)j * span_count(ncol) +
                     c0 / kSpanCols + sp;
         if (some == 0u)
             atomicAdd(&at->y, 1u);
@@ -279,11 +323,15 @@ __global__ __launch_bounds__(256) void split_kernel(
 // large the rms of a pixel's samples is 2^-4 or more, and the floor's error,
 // 2^-26 sqrt(2 n / 3) for n angles, below that of a float32 sum after every
 // angle, 2^-29 n / sqrt(2), from 128 angles on.
+template <bool BATCH>
 __global__ __launch_bounds__(256) void range_kernel(
-    const uint2* __restrict__ spans, int nrow, int ncol, int slice0,
-    double center, unsigned* __restrict__ smax) {
-    const int ns = span_count(ncol), j = slice0 + blockIdx.x;
-    const uint2* sp = spans + (size_t)j * ns;
+    const MatJob* __restrict__ jobs, int njobs, MatJob one) {
+    unsigned b;
+    const MatJob& job = find_job<BATCH>(jobs, njobs, one, kRange, b);
+    const int nrow = job.r.a.nrow, ns = span_count(job.r.a.ncol);
+    const int j = job.m.group_op * kGroup + (int)b;
+    const double center = job.r.a.center;
+    const uint2* sp = job.m.spans + (size_t)j * ns;
     bool any = false;
     for (int k = threadIdx.x; k < ns; k += 256) any |= sp[k].x != 0u;
     if (!__syncthreads_or(any)) return;
@@ -298,7 +346,7 @@ __global__ __launch_bounds__(256) void range_kernel(
         }
         redo |= 2 * low > all - zero;
     }
-    if (__syncthreads_or(redo) && threadIdx.x == 0) smax[j] = kRedo;
+    if (__syncthreads_or(redo) && threadIdx.x == 0) job.m.smax[j] = kRedo;
 }
 
 __device__ __forceinline__ double clamp_pos(double f, double w1) {
@@ -331,11 +379,10 @@ struct alignas(16) Angle {
     int pad;
 };
 
+// Tile (tx, ty) of slice groups grp .. grp + SG - 1
 template <int PL, int SG>
-__global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
-                                                             MatArgs ma,
-                                                             int tiles_x,
-                                                             int tiles_y) {
+__device__ __forceinline__ void matrix_tile(const BpArgs& a, const MatArgs& ma,
+                                            int tx, int ty, int grp) {
     using TL = Tile<SG>;
     constexpr int S = SG * kGroup;
     constexpr int ROWS = TL::rows;
@@ -366,18 +413,6 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
     Angle* const angles = reinterpret_cast<Angle*>(lds + 8);
     constexpr unsigned kRecAt = kAngAt + 3 * kStep * sizeof(Angle);
 
-    // Workgroups go to the 8 XCDs in turn.  An XCD's consecutive ones take a
-    // kPatchX x kPatchY patch of tiles, whose strips of an angle overlap: one
-    // L2 then holds them for as many angles as the workgroups drift apart.
-    // Grid: groups x patches (a multiple of 8) x tiles of a patch.
-    const unsigned xcd = blockIdx.x & 7u, seq = blockIdx.x >> 3;
-    const unsigned patch = (seq / (kPatchX * kPatchY)) * 8u + xcd;
-    const unsigned in = seq % (kPatchX * kPatchY);
-    const unsigned px = patch % ma.patches_x, pr = patch / ma.patches_x;
-    const int tx = px * kPatchX + in % kPatchX;
-    const int ty = (pr % ma.patches_y) * kPatchY + in / kPatchX;
-    const int grp = ma.group0 + (pr / ma.patches_y) * SG;
-    if (tx >= tiles_x || ty >= tiles_y || grp >= ma.group_end) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n16 = lane & 15, k4 = lane >> 4;
@@ -736,29 +771,81 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(BpArgs a,
     }
 }
 
+// Workgroups go to the 8 XCDs in turn.  An XCD's consecutive ones take a
+// kPatchX x kPatchY patch of tiles, whose strips of an angle overlap: one
+// L2 then holds them for as many angles as the workgroups drift apart.
+// One stack: slice groups x patches (a multiple of 8) x tiles of a patch.  A
+// batch has no workgroups to spare for patches that hang over small images:
+// every XCD takes an eighth of a stack's tiles, four rows of them at a time.
+template <int PL, int SG, bool BATCH>
+__global__ __launch_bounds__(kThreads) void bp_matrix_kernel(
+    const MatJob* __restrict__ jobs, int njobs, MatJob one) {
+    unsigned b;
+    const MatJob& job = find_job<BATCH>(jobs, njobs, one,
+                                        SG == 2 ? kPairs : kSingle, b);
+    const BpArgs& a = job.r.a;
+    const MatArgs& ma = job.m;
+    const int tiles_x = (a.ncol + Tile<SG>::X - 1) / Tile<SG>::X;
+    const int tiles_y = (a.ncol + Tile<SG>::Y - 1) / Tile<SG>::Y;
+    int tx, ty, grp;
+    if constexpr (BATCH) {
+        // pairs from group 0 on, a last odd group
+        const unsigned tiles = tiles_x * tiles_y, groups = ma.group_have;
+        const unsigned items = SG == 2 ? tiles * (groups / 2) : tiles;
+        const unsigned c = b & 7u;  // workgroups of one XCD are 8 apart
+        const unsigned i = c * (items >> 3) + min(c, items & 7u) + (b >> 3);
+        const unsigned t = i % tiles, row4 = tiles_x * kPatchY;
+        const unsigned y0 = t / row4 * kPatchY, in = t % row4;
+        const unsigned h = min(kPatchY, tiles_y - y0);
+        tx = in / h;
+        ty = y0 + in % h;
+        grp = SG == 2 ? i / tiles * 2 : groups - 1;
+    } else {
+        const unsigned xcd = b & 7u, seq = b >> 3;
+        const unsigned patch = (seq / (kPatchX * kPatchY)) * 8u + xcd;
+        const unsigned in = seq % (kPatchX * kPatchY);
+        const unsigned px = patch % ma.patches_x, pr = patch / ma.patches_x;
+        tx = px * kPatchX + in % kPatchX;
+        ty = (pr % ma.patches_y) * kPatchY + in / kPatchX;
+        grp = ma.group0 + (pr / ma.patches_y) * SG;
+        if (tx >= tiles_x || ty >= tiles_y || grp >= ma.group_end) return;
+    }
+    matrix_tile<PL, SG>(a, ma, tx, ty, grp);
+}
+
+template <int SG> constexpr size_t matrix_lds() {
+    return (size_t)(2 * kStep * Tile<SG>::rows * SG * kGroup + 8) *
+               sizeof(uint4_t) +
+           3 * kStep * sizeof(Angle);
+}
+
+template <int PL, int SG, bool BATCH>
+int launch_kernel(const MatJob* jobs, int njobs, const MatJob& one,
+                  long long blocks, hipStream_t stream) {
+    if (blocks > 0x7fffffffLL)
+        return set_error(ATH_ERR_UNSUPPORTED, "back-projection grid too large");
+    auto kern = bp_matrix_kernel<PL, SG, BATCH>;
+    const int st = allow_dynamic_lds(reinterpret_cast<const void*>(kern),
+                                     matrix_lds<SG>());
+    if (st != ATH_OK) return st;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads),
+                       matrix_lds<SG>(), stream, jobs, njobs, one);
+    return check_hip(hipGetLastError(), "bp_matrix_kernel launch");
+}
+
 template <int PL, int SG>
-int launch_matrix(const BpArgs& a, MatArgs ma, int groups,
-                  hipStream_t stream) {
-    using TL = Tile<SG>;
-    const int tiles_x = (a.ncol + TL::X - 1) / TL::X;
-    const int tiles_y = (a.ncol + TL::Y - 1) / TL::Y;
+int launch_matrix(MatJob job, int groups, hipStream_t stream) {
+    const int ncol = job.r.a.ncol;
+    const int tiles_x = (ncol + Tile<SG>::X - 1) / Tile<SG>::X;
+    const int tiles_y = (ncol + Tile<SG>::Y - 1) / Tile<SG>::Y;
+    MatArgs& ma = job.m;
     ma.group_end = ma.group0 + groups;
     ma.patches_x = (tiles_x + kPatchX - 1) / kPatchX;
     ma.patches_y = (tiles_y + kPatchY - 1) / kPatchY;
     const long long patches =
         (long long)ma.patches_x * ma.patches_y * (groups / SG);
-    const long long blocks = (patches + 7) / 8 * 8 * (kPatchX * kPatchY);
-    if (blocks > 0x7fffffffLL)
-        return set_error(ATH_ERR_UNSUPPORTED, "back-projection grid too large");
-    auto kern = bp_matrix_kernel<PL, SG>;
-    const size_t lds =
-        (size_t)(2 * kStep * TL::rows * SG * kGroup + 8) * sizeof(uint4_t) +
-        3 * kStep * sizeof(Angle);
-    const int st = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
-    if (st != ATH_OK) return st;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), lds,
-                       stream, a, ma, tiles_x, tiles_y);
-    return check_hip(hipGetLastError(), "bp_matrix_kernel launch");
+    return launch_kernel<PL, SG, false>(
+        nullptr, 0, job, (patches + 7) / 8 * 8 * (kPatchX * kPatchY), stream);
 }
 
 // rounds of 256 workgroups that `units` slice groups (or pairs) take
@@ -781,66 +868,86 @@ int part_groups(int planes, int nrow, int ncol, int groups) {
     return (int)std::min<size_t>(groups, std::max<size_t>(n, 2));
 }
 
+// Lays a stack's job out in `work` (null: only counts) with `part` slice
+// groups of split samples; returns the bytes.
+size_t set_job(MatJob& job, const BpArgs& a, int dtype, int part, char* work) {
+    const size_t nmax = (size_t)groups_of(a.nslice) * kGroup;
+    const int planes = planes_of(dtype);
+    // maxima, then the spans' counts: cleared together
+    const size_t nzero = nmax * (1 + 2 * (size_t)span_count(a.ncol));
+    const size_t trig_at = align256(nzero * sizeof(unsigned));
+    const size_t op_at = trig_at + align256((size_t)a.nrow * sizeof(float2));
+    MatArgs& m = job.m;
+    m.smax = reinterpret_cast<unsigned*>(work);
+    m.spans = reinterpret_cast<uint2*>(work + nmax * sizeof(unsigned));
+    m.trig = reinterpret_cast<float2*>(work + trig_at);
+    m.op = reinterpret_cast<unsigned*>(work + op_at);
+    m.npair = (a.ncol + 1) / 2;
+    m.nop = (size_t)part * kGroup * a.nrow * m.npair * planes;
+    m.pos0 = a.center + kPosMagic;
+    m.scaled = dtype != ATH_F16;
+    m.nzero = (int)nzero;
+    m.ntail = kTailPairs * kGroup * planes;
+    m.max_rows = std::min(a.nrow, 128);
+    m.group0 = m.group_op = 0;
+    m.group_have = part;
+    m.group_end = 0;
+    m.patches_x = m.patches_y = 0;
+    // slices with non-finite or huge samples are the vector kernel's
+    job.r.a = a;
+    job.r.a.only_above = m.smax;
+    job.r.a.above = kMaxBits;
+    job.r.begin = 0;
+    for (unsigned& b : job.begin) b = 0;
+    return op_at + (m.nop + m.ntail) * sizeof(unsigned);
+}
+
+long long clear_blocks(const MatJob& j) {
+    return ((long long)std::max({j.r.a.nrow, j.m.nzero, j.m.ntail}) + 255) /
+           256;
+}
+long long max_blocks(const MatJob& j) {
+    return (long long)j.r.a.nslice * j.m.max_rows;
+}
+long long split_blocks(const MatJob& j, int groups) {
+    return (long long)((j.r.a.ncol + 127) / 128) * j.r.a.nrow * groups;
+}
+
+#define ATH_MATRIX_LAUNCH(KERNEL, BLOCKS, JOBS, NJOBS, ONE)                   \
+    do {                                                                      \
+        const long long n_ = (BLOCKS);                                        \
+        if (n_ > 0x7fffffffLL)                                                \
+            return set_error(ATH_ERR_UNSUPPORTED,                             \
+                             "back-projection grid too large");               \
+        if (n_ > 0) {                                                         \
+            hipLaunchKernelGGL((KERNEL), dim3((unsigned)n_), dim3(256), 0, s, \
+                               JOBS, NJOBS, ONE);                             \
+            const int st_ = check_hip(hipGetLastError(), #KERNEL " launch");  \
+            if (st_ != ATH_OK) return st_;                                    \
+        }                                                                     \
+    } while (0)
+
 template <typename T, int PL>
 int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
                hipStream_t s) {
-    const int groups = groups_of(a.nslice), npair = (a.ncol + 1) / 2;
-    MatArgs ma;
-    // maxima, then the spans' counts: cleared together
-    const size_t nmax = (size_t)groups * kGroup;
-    unsigned* smax = reinterpret_cast<unsigned*>(work);
-    uint2* spans = reinterpret_cast<uint2*>(smax + nmax);
-    const size_t nzero = nmax * (1 + 2 * (size_t)span_count(a.ncol));
-    work += align256(nzero * sizeof(unsigned));
-    float2* trig = reinterpret_cast<float2*>(work);
-    work += align256((size_t)a.nrow * sizeof(float2));
-    unsigned* op = reinterpret_cast<unsigned*>(work);
-    ma.op = op;
-    ma.smax = smax;
-    ma.trig = trig;
-    ma.scaled = dtype != ATH_F16;
-    ma.npair = npair;
-    ma.pos0 = a.center + kPosMagic;
+    const int groups = groups_of(a.nslice);
     const int part = part_groups(PL, a.nrow, a.ncol, groups);
-    const size_t nop = (size_t)part * kGroup * a.nrow * npair * PL;
-    const int ntail = kTailPairs * kGroup * PL;
-    const T* sino = static_cast<const T*>(a.sino);
-    hipLaunchKernelGGL(trig_kernel,
-                       dim3((unsigned)((std::max({(size_t)a.nrow, nzero,
-                                                  (size_t)ntail}) +
-                                        255) /
-                                       256)),
-                       dim3(256), 0, s, a.angles, a.nrow, trig, smax,
-                       (int)nzero, op + nop, ntail);
-    int st = check_hip(hipGetLastError(), "trig_kernel launch");
-    if (st != ATH_OK) return st;
-    hipLaunchKernelGGL((slice_max_kernel<T>),
-                       dim3((unsigned)std::min(a.nrow, 128),
-                            (unsigned)a.nslice),
-                       dim3(256), 0, s, sino, a.nrow, a.nslice, a.ncol, smax);
-    st = check_hip(hipGetLastError(), "slice_max_kernel launch");
-    if (st != ATH_OK) return st;
+    MatJob job;
+    set_job(job, a, dtype, part, work);
+    const MatJob* none = nullptr;
+    ATH_MATRIX_LAUNCH(clear_kernel<false>, clear_blocks(job), none, 0, job);
+    ATH_MATRIX_LAUNCH((slice_max_kernel<T, false>), max_blocks(job), none, 0,
+                      job);
     for (int g0 = 0; g0 < groups; g0 += part) {
         const int n = std::min(part, groups - g0);
-        const int slice0 = g0 * kGroup;
-        hipLaunchKernelGGL((split_kernel<T, PL>),
-                           dim3((unsigned)((a.ncol + 127) / 128),
-                                (unsigned)a.nrow, (unsigned)n),
-                           dim3(256), 0, s, sino, a.nrow, a.nslice, a.ncol,
-                           npair, g0, smax, ma.scaled, spans, op);
-        st = check_hip(hipGetLastError(), "split_kernel launch");
-        if (st != ATH_OK) return st;
-        if (ma.scaled) {
-            hipLaunchKernelGGL(
-                range_kernel,
-                dim3((unsigned)std::min(n * kGroup, a.nslice - slice0)),
-                dim3(256), 0, s, spans, a.nrow, a.ncol, slice0, a.center,
-                smax);
-            st = check_hip(hipGetLastError(), "range_kernel launch");
-            if (st != ATH_OK) return st;
-        }
-        ma.group0 = ma.group_op = g0;
-        ma.group_have = g0 + n;
+        job.m.group0 = job.m.group_op = g0;
+        job.m.group_have = g0 + n;
+        ATH_MATRIX_LAUNCH((split_kernel<T, PL, false>), split_blocks(job, n),
+                          none, 0, job);
+        if (job.m.scaled)
+            ATH_MATRIX_LAUNCH(range_kernel<false>,
+                              std::min(n * kGroup, a.nslice - g0 * kGroup),
+                              none, 0, job);
         // Pairs of groups; a last odd group by itself unless an idle one
         // beside it is cheaper, which it is where the launch does not fill the
         // chip twice (rounds of 256 workgroups, at the measured 0.69 against
@@ -853,59 +960,165 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
             if (with < apart) ++pairs;
         }
         if (pairs) {
-            st = launch_matrix<PL, 2>(a, ma, 2 * pairs, s);
+            const int st = launch_matrix<PL, 2>(job, 2 * pairs, s);
             if (st != ATH_OK) return st;
-            ma.group0 += 2 * pairs;
+            job.m.group0 += 2 * pairs;
         }
         if (n > 2 * pairs) {
-            st = launch_matrix<PL, 1>(a, ma, 1, s);
+            const int st = launch_matrix<PL, 1>(job, 1, s);
             if (st != ATH_OK) return st;
         }
     }
-    // slices with non-finite or huge samples (workgroups of others leave at
-    // once)
-    BpArgs rest = a;
-    rest.only_above = smax;
-    rest.above = kMaxBits;
-    return back_projection(rest, dtype, acc, 0, 0, s);
+    // (workgroups of other slices leave at once)
+    return back_projection(job.r.a, dtype, acc, 0, 0, s);
+}
+
+// ---- many stacks in one set of launches ------------------------------------
+// Stack by stack the small ones would leave most of the chip idle, one after
+// another.  64 stacks of 361 x 6 x 128, filter included: 15.6 ms so, 1.6 ms here
+// (the vector kernel's work list 1.7); 16 of 721 x 16 x 512 8.6 and 6.6 (15.0);
+// 8 of 901 x 12 x 1024, which fill the chip by themselves, 12.5 and 12.5 (24.7).
+struct MatPlan {
+    int njobs, dtype, acc;
+    unsigned blocks[kStages], redo_blocks;
+};
+constexpr size_t kPlanJobs = 256;
+static_assert(sizeof(MatPlan) <= kPlanJobs, "plan header");
+
+template <typename T, int PL>
+int run_batch(const MatPlan& p, const MatJob* jobs, hipStream_t s) {
+    const MatJob one{};
+    const unsigned* n = p.blocks;
+    ATH_MATRIX_LAUNCH(clear_kernel<true>, n[kClear], jobs, p.njobs, one);
+    ATH_MATRIX_LAUNCH((slice_max_kernel<T, true>), n[kMaxima], jobs, p.njobs,
+                      one);
+    ATH_MATRIX_LAUNCH((split_kernel<T, PL, true>), n[kSplit], jobs, p.njobs,
+                      one);
+    if (p.dtype != ATH_F16)
+        ATH_MATRIX_LAUNCH(range_kernel<true>, n[kRange], jobs, p.njobs, one);
+    int st = ATH_OK;
+    if (n[kPairs])
+        st = launch_kernel<PL, 2, true>(jobs, p.njobs, one, n[kPairs], s);
+    if (st == ATH_OK && n[kSingle])
+        st = launch_kernel<PL, 1, true>(jobs, p.njobs, one, n[kSingle], s);
+    if (st != ATH_OK) return st;
+    return back_projection_redo(&jobs->r, sizeof(MatJob), p.njobs,
+                                p.redo_blocks, p.dtype, p.acc, s);
+}
+#undef ATH_MATRIX_LAUNCH
+
+// what the matrix path takes
+int check_matrix(const BpArgs& a, int dtype, int acc) {
+    if (a.ncol > kMaxMatrixCols || a.nrow > 65535 || a.nslice > 65535)
+        return set_error(ATH_ERR_UNSUPPORTED,
+                         "matrix back-projection: at most 32768 columns, "
+                         "65535 angles and 65535 slices");
+    if (dtype == ATH_F32) {
+        if (acc != ATH_ACC_F32SEQ && acc != ATH_ACC_F32)
+            return set_error(ATH_ERR_INVALID_ARG,
+                             "matrix back-projection: acc must be "
+                             "ATH_ACC_F32SEQ or ATH_ACC_F32");
+        return ATH_OK;
+    }
+    if (acc != ATH_ACC_F32)
+        return set_error(ATH_ERR_UNSUPPORTED,
+                         "back-projection: float16/bfloat16 sinograms need "
+                         "acc = ATH_ACC_F32");
+    if (dtype != ATH_F16 && dtype != ATH_BF16)
+        return set_error(ATH_ERR_INVALID_ARG,
+                         "back-projection: bad sinogram dtype");
+    return ATH_OK;
 }
 
 }  // namespace
 
 size_t back_projection_matrix_workspace(int dtype, int nrow, int nslice,
                                         int ncol) {
-    const size_t groups = groups_of(nslice);
-    const size_t part =
-        part_groups(planes_of(dtype), nrow, ncol, groups_of(nslice));
-    return align256(groups * kGroup * (1 + 2 * (size_t)span_count(ncol)) *
-                    sizeof(unsigned)) +
-           align256((size_t)nrow * sizeof(float2)) +
-           (part * nrow * (size_t)((ncol + 1) / 2) + kTailPairs) * kGroup * 4 *
-               planes_of(dtype);
+    BpArgs a{};
+    a.nrow = nrow;
+    a.nslice = nslice;
+    a.ncol = ncol;
+    MatJob job;
+    return set_job(job, a, dtype,
+                   part_groups(planes_of(dtype), nrow, ncol,
+                               groups_of(nslice)),
+                   nullptr);
 }
 
 int back_projection_matrix(const BpArgs& a, int dtype, int acc, void* work,
                            hipStream_t s) {
-    if (a.ncol > kMaxMatrixCols || a.nrow > 65535 || a.nslice > 65535)
-        return set_error(ATH_ERR_UNSUPPORTED,
-                         "matrix back-projection: at most 32768 columns, "
-                         "65535 angles and 65535 slices");
+    const int st = check_matrix(a, dtype, acc);
+    if (st != ATH_OK) return st;
     char* w = static_cast<char*>(work);
-    if (dtype == ATH_F32) {
-        if (acc != ATH_ACC_F32SEQ && acc != ATH_ACC_F32)
-            return set_error(ATH_ERR_INVALID_ARG,
-                             "matrix back-projection: acc must be "
-                             "ATH_ACC_F32SEQ or ATH_ACC_F32");
-        return run_matrix<float, 2>(a, dtype, acc, w, s);
-    }
-    if (acc != ATH_ACC_F32)
-        return set_error(ATH_ERR_UNSUPPORTED,
-                         "back-projection: float16/bfloat16 sinograms need "
-                         "acc = ATH_ACC_F32");
+    if (dtype == ATH_F32) return run_matrix<float, 2>(a, dtype, acc, w, s);
     if (dtype == ATH_F16) return run_matrix<__half, 1>(a, dtype, acc, w, s);
-    if (dtype == ATH_BF16)
-        return run_matrix<__hip_bfloat16, 1>(a, dtype, acc, w, s);
-    return set_error(ATH_ERR_INVALID_ARG, "back-projection: bad sinogram dtype");
+    return run_matrix<__hip_bfloat16, 1>(a, dtype, acc, w, s);
+}
+
+size_t matrix_batch_plan_bytes(int njobs) {
+    return kPlanJobs + (size_t)njobs * sizeof(MatJob);
+}
+
+size_t matrix_batch_job_bytes(int dtype, int nrow, int nslice, int ncol) {
+    BpArgs a{};
+    a.nrow = nrow;
+    a.nslice = nslice;
+    a.ncol = ncol;
+    MatJob job;
+    return align256(set_job(job, a, dtype, groups_of(nslice), nullptr));
+}
+
+void matrix_batch_begin(void* plan, int dtype, int acc) {
+    MatPlan p{};
+    p.dtype = dtype;
+    p.acc = acc;
+    *static_cast<MatPlan*>(plan) = p;
+}
+
+int matrix_batch_add(void* plan, const BpArgs& a, void* work) {
+    MatPlan& p = *static_cast<MatPlan*>(plan);
+    const int st = check_matrix(a, p.dtype, p.acc);
+    if (st != ATH_OK) return st;
+    MatJob& j = reinterpret_cast<MatJob*>(static_cast<char*>(plan) +
+                                          kPlanJobs)[p.njobs];
+    const int groups = groups_of(a.nslice);
+    set_job(j, a, p.dtype, groups, static_cast<char*>(work));
+    j.m.max_rows = std::min(a.nrow, 32);
+    const auto tiles = [&](int x, int y) {
+        return (long long)((a.ncol + x - 1) / x) * ((a.ncol + y - 1) / y);
+    };
+    long long n[kStages];
+    n[kClear] = clear_blocks(j);
+    n[kMaxima] = max_blocks(j);
+    n[kSplit] = split_blocks(j, groups);
+    n[kRange] = a.nslice;
+    n[kPairs] = tiles(Tile<2>::X, Tile<2>::Y) * (groups / 2);
+    n[kSingle] = groups & 1 ? tiles(Tile<1>::X, Tile<1>::Y) : 0;
+    const long long redo = redo_tiles(a.nslice, a.ncol);
+    const char* large = "matrix back-projection: batch too large";
+    for (int k = 0; k < kStages; ++k)
+        if (p.blocks[k] + n[k] > 0x7fffffffLL)
+            return set_error(ATH_ERR_UNSUPPORTED, large);
+    if (p.redo_blocks + redo > 0x7fffffffLL)
+        return set_error(ATH_ERR_UNSUPPORTED, large);
+    for (int k = 0; k < kStages; ++k) {
+        j.begin[k] = p.blocks[k];
+        p.blocks[k] += (unsigned)n[k];
+    }
+    j.r.begin = p.redo_blocks;
+    p.redo_blocks += (unsigned)redo;
+    ++p.njobs;
+    return ATH_OK;
+}
+
+int back_projection_matrix_batched(const void* plan, const void* plan_dev,
+                                   hipStream_t s) {
+    const MatPlan& p = *static_cast<const MatPlan*>(plan);
+    const MatJob* jobs = reinterpret_cast<const MatJob*>(
+        static_cast<const char*>(plan_dev) + kPlanJobs);
+    if (p.dtype == ATH_F32) return run_batch<float, 2>(p, jobs, s);
+    if (p.dtype == ATH_F16) return run_batch<__half, 1>(p, jobs, s);
+    return run_batch<__hip_bfloat16, 1>(p, jobs, s);
 }
 
 }  // namespace ath

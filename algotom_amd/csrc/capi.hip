@@ -398,6 +398,73 @@ int ath_back_projection_matrix(const void* sino, int sino_dtype, int nrow,
                                   static_cast<hipStream_t>(stream));
 }
 
+size_t ath_matrix_batch_plan_bytes(int njobs) {
+    return njobs < 1 ? 0 : matrix_batch_plan_bytes(njobs);
+}
+
+size_t ath_matrix_batch_workspace_bytes(const ath_bp_job* jobs, int njobs,
+                                        int sino_dtype) {
+    if (!jobs || njobs < 1) return 0;
+    size_t sum = 0;
+    for (int i = 0; i < njobs; ++i) {
+        if (ath_back_projection_matrix_workspace_bytes(
+                sino_dtype, jobs[i].nrow, jobs[i].nslice, jobs[i].ncol) == 0)
+            return 0;
+        sum += matrix_batch_job_bytes(sino_dtype, jobs[i].nrow,
+                                      jobs[i].nslice, jobs[i].ncol);
+    }
+    return sum;
+}
+
+int ath_matrix_batch_plan(const ath_bp_job* jobs, int njobs, int sino_dtype,
+                          int acc, void* workspace, size_t workspace_bytes,
+                          void* plan, size_t plan_bytes) {
+    clear_error();
+    if (!jobs || !workspace || !plan)
+        return set_error(ATH_ERR_INVALID_ARG, "null pointer");
+    if (njobs < 1)
+        return set_error(ATH_ERR_INVALID_ARG, "need at least one job");
+    if (reinterpret_cast<size_t>(workspace) & 15)
+        return set_error(ATH_ERR_INVALID_ARG,
+                         "the workspace must be 16-byte aligned");
+    if (reinterpret_cast<size_t>(plan) & 7)
+        return set_error(ATH_ERR_INVALID_ARG,
+                         "the plan must be 8-byte aligned");
+    const size_t need =
+        ath_matrix_batch_workspace_bytes(jobs, njobs, sino_dtype);
+    if (need == 0)
+        return set_error(ATH_ERR_UNSUPPORTED,
+                         "matrix back-projection: float32, float16 or "
+                         "bfloat16 sinograms of at most 32768 columns");
+    if (workspace_bytes < need)
+        return set_error(ATH_ERR_WORKSPACE,
+                         "matrix back-projection workspace too small");
+    if (plan_bytes < matrix_batch_plan_bytes(njobs))
+        return set_error(ATH_ERR_INVALID_ARG, "plan too small");
+    matrix_batch_begin(plan, sino_dtype, acc);
+    char* work = static_cast<char*>(workspace);
+    for (int i = 0; i < njobs; ++i) {
+        const ath_bp_job& j = jobs[i];
+        BpArgs a;
+        int st = fill_bp_args(a, j.sino, j.nrow, j.nslice, j.ncol, j.angles,
+                              j.center, j.edge_pad, j.mask_radius,
+                              j.apply_scale, j.recon);
+        if (st == ATH_OK) st = matrix_batch_add(plan, a, work);
+        if (st != ATH_OK) return st;
+        work += matrix_batch_job_bytes(sino_dtype, j.nrow, j.nslice, j.ncol);
+    }
+    return ATH_OK;
+}
+
+int ath_back_projection_matrix_batched(const void* plan, const void* plan_dev,
+                                       void* stream) {
+    clear_error();
+    if (!plan || !plan_dev)
+        return set_error(ATH_ERR_INVALID_ARG, "null pointer");
+    return back_projection_matrix_batched(plan, plan_dev,
+                                          static_cast<hipStream_t>(stream));
+}
+
 int ath_back_projection_with_derivative(const float* sino, int nrow,
                                         int nslice, int ncol,
                                         const float* angles, float center,

@@ -8,18 +8,25 @@ The reference reconstructs slices one call at a time (reconstruction.py
   sinogram that shares them, one workgroup per row), then
 * one persistent back-projection launch per arithmetic over the (sinogram,
   tile) work list of its sinograms, workgroups pulling items from a device
-  counter, heaviest sinograms (most angles) first.
+  counter, heaviest sinograms (most angles) first, and
+* one set of launches for all stacks that are summed on the matrix cores.
 
 ``capture()`` records that launch sequence in a HIP graph (torch.cuda.CUDAGraph
 on ROCm) so a replay costs one graph launch.  Per sinogram the arithmetic is
 that of ``fbp_reconstruction`` with the same arguments.
 """
 
+import ctypes
+
 import numpy as np
 
 from algotom_amd import _native as nat
 from algotom_amd.rec import autotune
 from algotom_amd.rec import reconstruction as rec
+
+# Workspace of one batched launch on the matrix cores: the split samples of
+# its stacks (as many bytes as their float32 samples, in groups of 16 slices)
+_MATRIX_BYTES = 2 << 30
 
 
 class BatchFBP:
@@ -48,8 +55,8 @@ class BatchFBP:
     it: with ``precision=None`` a single sinogram with ``gpu=True`` is
     back-projected with float64 sums and the rest with float32 storage
     after every angle, so the batch runs one persistent back-projection
-    launch per arithmetic it contains, and one launch per stack that
-    fbp_reconstruction sums on the matrix cores.
+    launch per arithmetic it contains, and one set of launches for the stacks
+    that fbp_reconstruction sums on the matrix cores.
     """
 
     def __init__(self, shapes, centers, angles=None, filter_name="hann",
@@ -152,21 +159,25 @@ class BatchFBP:
                 r = min(c, ncol - c) / (0.5 * ncol)
             return float(r * (ncol // 2))
 
-        # ---- stacks that fbp_reconstruction sums on the matrix cores: a
-        # launch each, sharing one workspace
-        self.matrix_jobs = []
+        def bp_job(i):
+            nrow, nslice, ncol = self.shapes3[i]
+            return nat.BpJob(
+                self.filtered[i].data_ptr(), self.outputs[i].data_ptr(),
+                self._angles[i].data_ptr(), nrow, nslice, ncol,
+                float(np.float32(centers[i])), mask_radius(i), 1, 0, 0)
+
+        # ---- stacks that fbp_reconstruction sums on the matrix cores
         matrix = [rec._matrix_stack(*s, accs[i], store)
                   for i, s in enumerate(self.shapes3)]
-        for i in range(n):
-            if matrix[i]:
-                self.matrix_jobs.append(
-                    (i, accs[i], float(np.float32(centers[i])),
-                     mask_radius(i)))
-        self.matrix_work = None
-        if self.matrix_jobs:
-            self.matrix_work = max(
-                (rec._matrix_workspace(*self.shapes3[job[0]], store, self.dev)
-                 for job in self.matrix_jobs), key=lambda w: w.numel())
+        members = sorted((i for i in range(n) if matrix[i]),
+                         key=lambda i: -self.shapes3[i][0])
+        self.matrix_groups, self.matrix_jobs, self.matrix_work = [], [], None
+        try:
+            self._plan_matrix([(bp_job(i), accs[i]) for i in members])
+        except torch.OutOfMemoryError:
+            # no room for the split samples: the vector kernel needs none
+            self.matrix_groups, self.matrix_jobs = [], []
+            matrix = [False] * n
 
         # ---- back-projection work lists, one per arithmetic: heaviest
         # per-tile cost (most angles) first
@@ -179,11 +190,7 @@ class BatchFBP:
             order = sorted(members, key=lambda i: -self.shapes3[i][0])
             jobs = (nat.BpJob * len(order))()
             for k, i in enumerate(order):
-                nrow, nslice, ncol = self.shapes3[i]
-                jobs[k] = nat.BpJob(
-                    self.filtered[i].data_ptr(), self.outputs[i].data_ptr(),
-                    self._angles[i].data_ptr(), nrow, nslice, ncol,
-                    float(np.float32(centers[i])), mask_radius(i), 1, 0, 0)
+                jobs[k] = bp_job(i)
             sb = 1 if all(self.shapes3[i][1] == 1 for i in members) else 4
             self.bp_groups.append({
                 "acc": acc, "slice_batch": sb, "jobs": jobs,
@@ -193,6 +200,50 @@ class BatchFBP:
         self.updates = sum(s[0] * s[1] * s[2] * s[2] for s in self.shapes3)
         self._retile()
         self.graph = None
+
+    def _plan_matrix(self, members):
+        """Plans the stacks of the matrix cores, (job, acc) pairs: batched
+        launches of at most _MATRIX_BYTES of workspace each, larger stacks by
+        themselves (in parts), all after one another in one workspace."""
+        import torch
+        size = self.lib.ath_matrix_batch_workspace_bytes
+
+        def need(jobs):
+            return size(ctypes.byref(jobs), len(jobs), self.store_code)
+
+        groups, total = [], 0
+        for job, acc in members:
+            one = need((nat.BpJob * 1)(job))
+            if one > _MATRIX_BYTES:
+                self.matrix_jobs.append((job, acc))
+                continue
+            if not groups or total + one > _MATRIX_BYTES:
+                groups.append([])
+                total = 0
+            groups[-1].append((job, acc))
+            total += one
+        groups = [((nat.BpJob * len(g))(*(job for job, _ in g)), g[0][1])
+                  for g in groups]
+        most = max([need(jobs) for jobs, _ in groups]
+                   + [self._matrix_bytes(job) for job, _ in self.matrix_jobs]
+                   + [0])
+        if not most:
+            return
+        self.matrix_work = torch.empty(most, dtype=torch.uint8,
+                                       device=self.dev)
+        for jobs, acc in groups:
+            nbytes = self.lib.ath_matrix_batch_plan_bytes(len(jobs))
+            plan = np.zeros((nbytes + 7) // 8, dtype=np.uint64)
+            nat.check(self.lib.ath_matrix_batch_plan(
+                ctypes.byref(jobs), len(jobs), self.store_code, acc,
+                nat.ptr(self.matrix_work), most, plan.ctypes.data, nbytes),
+                "ath_matrix_batch_plan")
+            self.matrix_groups.append(
+                (plan, torch.from_numpy(plan.view(np.uint8)).to(self.dev)))
+
+    def _matrix_bytes(self, job):
+        return self.lib.ath_back_projection_matrix_workspace_bytes(
+            self.store_code, job.nrow, job.nslice, job.ncol)
 
     @property
     def total_tiles(self):
@@ -236,13 +287,15 @@ class BatchFBP:
                 self.store_code, g["acc"], g["slice_batch"], self.tile_rows,
                 self.nblocks, nat.ptr(g["counter"]), stream),
                 "ath_back_projection_batched")
-        for i, acc, center, radius in self.matrix_jobs:
-            nrow, nslice, ncol = self.shapes3[i]
+        for plan, plan_dev in self.matrix_groups:
+            nat.check(self.lib.ath_back_projection_matrix_batched(
+                plan.ctypes.data, nat.ptr(plan_dev), stream),
+                "ath_back_projection_matrix_batched")
+        for jb, acc in self.matrix_jobs:
             nat.check(self.lib.ath_back_projection_matrix(
-                nat.ptr(self.filtered[i]), self.store_code, nrow, nslice,
-                ncol, nat.ptr(self._angles[i]), center, 0, acc, radius, 1,
-                nat.ptr(self.outputs[i]), nat.ptr(self.matrix_work),
-                self.matrix_work.numel(), stream),
+                jb.sino, self.store_code, jb.nrow, jb.nslice, jb.ncol,
+                jb.angles, jb.center, 0, acc, jb.mask_radius, 1, jb.recon,
+                nat.ptr(self.matrix_work), self.matrix_work.numel(), stream),
                 "ath_back_projection_matrix")
 
     def capture(self):

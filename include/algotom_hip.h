@@ -197,6 +197,26 @@ int ath_back_projection_matrix(const void* sino, int sino_dtype, int nrow,
                                float* recon, void* workspace,
                                size_t workspace_bytes, void* stream);
 
+/* Many stacks of different widths, angle counts and centres on the matrix
+ * cores in one set of launches; every stack gets the bits that
+ * ath_back_projection_matrix gives it.  jobs: host array (tile_begin is
+ * ignored), in the order in which the workgroups are wanted (most angles
+ * first).  ath_matrix_batch_plan writes the plan, ath_matrix_batch_plan_bytes
+ * (njobs) bytes of host memory, 8-byte aligned; the run takes it and a copy in
+ * device memory.  workspace: ath_matrix_batch_workspace_bytes(...) of device
+ * memory (0: a job that ath_back_projection_matrix does not take either),
+ * 16-byte aligned, kept with the plan.  No allocation, no copy and no
+ * synchronisation in the run: it can be captured in a HIP graph.  No reference
+ * counterpart (as ath_back_projection_batched). */
+size_t ath_matrix_batch_plan_bytes(int njobs);
+size_t ath_matrix_batch_workspace_bytes(const ath_bp_job* jobs, int njobs,
+                                        int sino_dtype);
+int ath_matrix_batch_plan(const ath_bp_job* jobs, int njobs, int sino_dtype,
+                          int acc, void* workspace, size_t workspace_bytes,
+                          void* plan, size_t plan_bytes);
+int ath_back_projection_matrix_batched(const void* plan, const void* plan_dev,
+                                       void* stream);
+
 /* The back-projection of ath_back_projection with acc ATH_ACC_F64 into
  * recon and, in the same pass over the same positions and staged samples,
  * its derivative with respect to the rotation centre (acc ATH_ACC_DERIV)

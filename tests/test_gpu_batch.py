@@ -79,6 +79,69 @@ def test_batch_stacks_and_2d_mixed(gpu):
         assert np.array_equal(g, ref), (s.shape, s.dtype, gpu)
 
 
+def _stacks(precision, seed):
+    """Stacks of 6 to 40 slices (lone groups, pairs, both) and others that the
+    vector kernel sums, with samples that are sent back to it."""
+    rng = np.random.default_rng(seed)
+    shapes = [(131, 6, 90), (260, 17, 130), (257, 40, 65), (40, 4, 70),
+              (300, 33, 33), (181, 1, 64), (1025, 20, 97), (150, 48, 260)]
+    sinos = [rng.uniform(0.05, 1, s).astype(np.float32) for s in shapes]
+    if precision is None:
+        sinos[1][7, 9, 30] = np.inf
+        sinos[4][3, 32, 5] = 1e30
+    centers = [s[2] / 2 + rng.uniform(-3, 3) for s in shapes]
+    return sinos, centers
+
+
+@pytest.mark.parametrize("precision", [None, "fp16", "bf16"])
+@pytest.mark.parametrize("limit", [None, 5 << 19])
+def test_matrix_stacks_in_a_batch(precision, limit, monkeypatch):
+    """Stacks on the matrix cores run as one set of launches (limit: several,
+    and stacks by themselves) with fbp_reconstruction's bits, from replayed
+    graphs too."""
+    import torch
+    from algotom_amd.rec import batch, reconstruction as rec
+    if limit:
+        monkeypatch.setattr(batch, "_MATRIX_BYTES", limit)
+    sinos, centers = _stacks(precision, 5)
+    plan = batch.BatchFBP([s.shape for s in sinos], centers, apply_log=False,
+                          precision=precision)
+    assert len(plan.matrix_groups) == 1 if limit is None else (
+        len(plan.matrix_groups) > 1 and plan.matrix_jobs)
+    plan.load(sinos)
+    plan.capture()
+    for _ in range(3):
+        torch.randn(1 << 18, device="cuda").sum().item()
+        for o in plan.outputs:
+            o.fill_(7.0)
+        plan.run()
+        torch.cuda.synchronize()
+        for s, c, g in zip(sinos, centers, plan.results()):
+            ref = rec.fbp_reconstruction(s.copy(), c, apply_log=False,
+                                         precision=precision)
+            assert np.array_equal(g, ref, equal_nan=True), s.shape
+
+
+def test_matrix_stacks_without_room(monkeypatch):
+    """No room for the split samples: the vector kernel sums every stack."""
+    import torch
+    from algotom_amd.rec import batch, reconstruction as rec
+
+    def no_room(self, members):
+        raise torch.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(batch.BatchFBP, "_plan_matrix", no_room)
+    sinos, centers = _stacks(None, 6)
+    plan = batch.BatchFBP([s.shape for s in sinos], centers, apply_log=False)
+    plan.load(sinos)
+    plan.run()
+    got = plan.results()
+    monkeypatch.setattr(rec, "_matrix_stack", lambda *a: False)
+    for s, c, g in zip(sinos, centers, got):
+        ref = rec.fbp_reconstruction(s.copy(), c, apply_log=False)
+        assert np.array_equal(g, ref, equal_nan=True), s.shape
+
+
 def test_graph_replays_match_eager():
     import torch
     from algotom_amd.rec import batch
