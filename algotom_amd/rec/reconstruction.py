@@ -299,38 +299,43 @@ def _matrix_stack(nrow, nslice, ncol, acc, dtype):
     * Per-angle sums, 128 and more angles: 0.55 to 0.91 at 6 slices, less at
       more, at every width.  (5 slices 0.51 to 0.91 too: stacks of up to 5
       keep the reference kernel's bits.)
-    * float32: 1000 columns and more 0.80 to 0.96 at 16 slices, 0.77 to 1.05
-      at 17, but 0.94 to 1.19 at 9 to 12; 512 columns 0.62 to 0.93 at 17,
-      0.86 to 1.18 at 16; 640 and 768 columns 0.96 to 1.16 at 17, 0.80 to 1.01
-      at 24, 0.59 to 0.85 at 32 (640 columns at 48 slices, three groups of
-      which two fill half a round of the chip, 1.04 to 1.19); fewer columns
-      0.94 to 1.7.
-    * 16-bit: 1000 columns and more 0.70 to 0.99 from 9 slices and 64 angles
-      on (37 angles up to 1.08, 8 angles 1.05 to 1.4); up to 512 columns 0.42
+    * float32: 1000 columns and more 0.69 to 0.96 at 16 slices, 0.77 to 1.05
+      at 17; at 9 to 12 slices 0.89 to 0.99 where a group's tiles are whole
+      rounds of the 256 CUs (1024 and 2560 columns, 256 angles on), 1.06 to
+      1.19 where not (1500) and 1.03 to 1.16 at 128 angles; 512 columns 0.62
+      to 0.93 at 17 slices, 0.86 to 1.18 at 16; 640 and 768 columns 0.80 to
+      1.01 at 24, 0.59 to 0.85 at 32, 0.96 to 1.17 at 17 (at 48 slices of 640
+      columns, three groups, 0.95 to 1.19); fewer columns 0.64 to 1.8.
+    * 16-bit: 1000 columns and more 0.60 to 0.99 from 9 slices and 64 angles
+      on (37 angles up to 1.08, 8 angles 1.05 to 1.4); up to 512 columns 0.38
       to 0.84 from 256 angles on, 0.56 to 0.99 at 128 angles and 9 to 24 slices
-      (32 and 48 slices 0.63 to 1.10), 64 angles up to 1.22; 640 and 768
-      columns 1.0 to 1.5 at 9 to 16 slices, 0.59 to 0.99 at 17 to 32."""
+      (more slices 1.0 to 1.1 up to 256 columns, 0.63 to 1.04 from 384 on),
+      0.63 to 1.03 at 64 angles and 9 to 16; 640 and 768 columns 0.59 to 0.99
+      at 17 to 32 slices, 0.9 to 1.5 at 9 to 16."""
     import torch
     if ncol > 32768 or nrow > 65535 or nslice > 65535:
         return False
     if dtype in (torch.float16, torch.bfloat16):
         if acc != nat.ACC_F32 or nslice <= 8 or nrow < 64:
             return False
-        if ncol >= 1000:
+        if ncol >= 1000 or (ncol <= 512 and nrow >= 256):
             return True
-        if nrow < 128:
-            return False
         if ncol > 512:
-            return nslice > 16 and (nslice <= 32 or nrow >= 256)
-        return nslice <= 24 or nrow >= 256
+            return (nslice > 16 and nrow >= 128
+                    and (nslice <= 32 or nrow >= 256))
+        if nrow < 128:
+            return nslice <= 16
+        return nslice <= 24 or ncol >= 384
     if dtype != torch.float32 or nrow < 128:
         return False
     if acc == nat.ACC_F32SEQ:
         return nslice > 5
     if acc == nat.ACC_F32:
-        if ncol >= 1000:
-            return nslice > 12
-        return ncol >= 512 and nslice > (16 if ncol == 512 else 24)
+        if ncol < 1000:
+            return ncol >= 512 and nslice > (16 if ncol == 512 else 20)
+        tiles = -(-ncol // 64) * -(-ncol // 32)
+        whole = tiles >= 0.95 * 256 * -(-tiles // 256)
+        return nslice > 12 or (nslice > 8 and nrow >= 256 and whole)
     return False
 
 

@@ -83,18 +83,28 @@ def test_to_host_of_host_tensor():
     (128, 5, 2560, False, False, False),
     (361, 9, 640, True, False, False),       # half-filled rounds of the chip
     (361, 17, 640, True, False, True),
-    (361, 25, 640, True, True, True),
+    (361, 20, 640, True, False, True),
+    (361, 21, 640, True, True, True),
     (128, 48, 640, True, True, False),
     (361, 16, 512, True, False, True),
     (361, 17, 512, True, True, True),
-    (361, 12, 1024, True, False, True),
+    (255, 12, 1024, True, False, True),
+    (256, 9, 1024, True, True, True),
+    (361, 8, 1024, True, False, False),
+    (361, 12, 1500, True, False, True),
     (361, 13, 1024, True, True, True),
     (128, 24, 256, True, False, True),
     (128, 25, 256, True, False, False),
+    (128, 48, 384, True, False, True),
     (256, 48, 256, True, False, True),
     (64, 9, 1000, False, False, True),
     (63, 9, 1000, False, False, False),
-    (64, 9, 512, False, False, False),
+    (64, 16, 512, False, False, True),
+    (64, 17, 512, False, False, False),
+    (127, 17, 640, False, False, False),
+    (128, 17, 640, True, False, True),
+    (128, 33, 640, True, True, False),
+    (256, 33, 640, True, True, True),
     (1801, 64, 32769, False, False, False),
     (65536, 64, 2560, False, False, False)])
 def test_matrix_rule(nrow, nslice, ncol, f32seq, f32, f16):
