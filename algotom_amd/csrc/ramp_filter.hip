@@ -1112,7 +1112,7 @@ int ramp_filter_adjoint(const float* in, int nrow, int nslice, int ncol,
         return check_hip(hipGetLastError(),
                          "ramp_filter_adjoint_big_kernel launch");
     }
-    switch (maxb_for(fft_len / 2)) {
+    switch (filter_class(fft_len / 2)) {
     case 1: return launch_adjoint<1>(in, nrow, nslice, ncol, pad, pad_mode,
                                      plan, fft_len, nwin, out, s);
     case kRegs1024:

@@ -304,3 +304,35 @@ def test_filter_rows_in_registers_many(ncol):
     adj = adj.view(rep, 5, ncol)[:, [0, 1, 2, 4]]
     assert torch.isfinite(adj).all()
     assert torch.equal(adj, adj[:1].expand_as(adj))
+
+
+# the transpose's rows in registers: the shortest and longest row (ncol + 2 pad
+# just above and at a power of two) of M = 1024, 2048 and 4096, and its
+# neighbours that stay in LDS (512 and 8192)
+@pytest.mark.parametrize("mode", ["edge", "reflect", "symmetric", "wrap",
+                                  "constant"])
+@pytest.mark.parametrize("ncol,pad", [
+    (358, 77), (359, 77), (724, 150), (513, 0), (725, 150), (1748, 150),
+    (1749, 150), (3796, 150), (3797, 150)])
+def test_filter_adjoint_identity(ncol, pad, mode):
+    """<F x, y> = <x, F^T y> with F x in float64; the transpose's float32
+    outputs are off by half an ulp each (2^-24 relative), its sums in float64
+    by far less."""
+    import torch
+    from algotom_amd import _native as nat
+    from algotom_amd.rec import autograd
+    nrow = 3
+    x = _rows(nrow, 2, ncol, ncol, positive=False)
+    y = _rows(nrow, 2, ncol, ncol + 1, positive=False)
+    geom = autograd.FBPGeometry(nrow, ncol, np.linspace(0.0, 3.0, nrow),
+                                pad=pad, pad_mode=mode)
+    fx = _gpu_filter(x, pad, mode, False, geom.taps, torch.float64)
+    fty = geom.filter_adjoint(torch.from_numpy(y).to(nat.device()))
+    fty = fty.cpu().numpy().astype(np.float64)
+    for j in range(2):
+        for i in range(nrow):
+            left = np.dot(fx[i, j], y[i, j].astype(np.float64))
+            terms = x[i, j].astype(np.float64) * fty[i, j]
+            tol = (2.0 ** -24 * np.abs(terms).sum()
+                   + 1e-12 * np.abs(fx[i, j] * y[i, j]).sum())
+            assert abs(left - terms.sum()) <= tol, (i, j)
