@@ -495,9 +495,9 @@ __device__ __forceinline__ void angle_setup(const BpArgs& a, Sh& sh, int sl,
 // every thread of the workgroup; starts and ends with all LDS consumed.
 //
 // A tile outside the mask (18 % of a 2560-wide image's 64 x 32 tiles) is
-// v * 0: zero unless a sum is infinite or NaN.  It only looks through the
-// samples its angles could reach, and sums them as any other tile where one
-// is not below 2^100: one 1801 x 2560 sinogram 4.44 -> 3.93 ms,
+// v * 0: zero (here always +0) unless a sum is infinite or NaN, times the scale
+// (NaN with a single angle).  It only looks through the samples its angles could
+// reach, and sums them as any other tile where one is not below 2^100: one 1801 x 2560 sinogram 4.44 -> 3.93 ms,
 // the 24-sinogram batch 19.6 -> 16.6 ms, a centre search 11.2 -> 9.85 ms.
 template <int MODE, int SB, int PY, int A, typename Tin>
 __device__ __forceinline__ void bp_tile(
@@ -556,8 +556,9 @@ __device__ __forceinline__ void bp_tile(
                     if (a.only_above && a.only_above[j0 + js] <= a.above)
                         continue;
                     const size_t o = ((size_t)y * S + j0 + js) * C + x;
-                    a.recon[o] = 0.0f;
-                    if constexpr (M::kTwoOut) a.recon2[o] = 0.0f;
+                    a.recon[o] = finalize(a, 0.0f, x, y);
+                    if constexpr (M::kTwoOut)
+                        a.recon2[o] = finalize(a, 0.0f, x, y);
                 }
             }
             return;

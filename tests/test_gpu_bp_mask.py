@@ -50,3 +50,17 @@ def test_masked_tiles_with_derivative():
     outside = torch.from_numpy(xx ** 2 + yy ** 2 > 50 ** 2).cuda()
     assert not out.permute(1, 0, 2)[:, outside].any()
     assert not der.permute(1, 0, 2)[:, outside].any()
+
+
+def test_masked_tiles_of_a_single_angle():
+    """One angle in a batch: the scale divides by nrow - 1 = 0, so a pixel
+    outside the mask is 0 / 0 in a skipped tile as in a summed one."""
+    from algotom_amd.rec import batch
+    rng = np.random.default_rng(3)
+    sino = rng.uniform(0.5, 1.0, (1, 300)).astype(np.float32)
+    plan = batch.BatchFBP([sino.shape], [149.5], ratio=0.5)
+    plan.load([sino])
+    plan.run()
+    got = plan.results()[0]
+    yy, xx = np.mgrid[:300, :300] - 150
+    assert np.isnan(got[xx ** 2 + yy ** 2 > 75 ** 2]).all()
