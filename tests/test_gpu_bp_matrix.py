@@ -58,6 +58,37 @@ def test_error_against_float64_sums(case, dtype):
     assert err <= bound
 
 
+@pytest.mark.parametrize("data", ["noise", "positive", "filtered"])
+@pytest.mark.parametrize("ncol,nrow,nslice,center", [
+    (64, 128, 6, 31.2),                 # the rule's smallest
+    (131, 181, 17, 70.0),               # a pair
+    (1025, 128, 33, 512.37),            # a pair and a lone group
+    (700, 400, 9, 3.0),                 # half of the pixels' angles in range
+    (300, 400, 6, -20.5), (300, 400, 6, 313.0),     # outside the detector
+    (513, 901, 6, 250.4)])
+def test_error_below_float32_sums(ncol, nrow, nslice, center, data):
+    """What sends float32 stacks of 128 and more angles to the matrix cores:
+    their error against float64 sums is no larger than that of a float32 sum
+    after every angle (no allowance).  Noise, projections of a disc with edge
+    padding, and the same filtered."""
+    import torch
+    from algotom_amd.rec import reconstruction as rec
+    x, ang = _case(ncol, nrow, nslice, np.pi, 4)
+    edge = data == "positive"
+    if data != "noise":
+        u = torch.linspace(-1, 1, ncol, device="cuda")
+        x = ((2.0 * (1 - u * u).sqrt() + 0.02 * x).abs() + 1e-3).contiguous()
+    if data == "filtered":
+        pad = min(int(0.15 * ncol), 150)
+        taps = rec._window_taps(None, nrow, ncol + 2 * pad, "hann")
+        x = rec._filter_stack(x, pad, "edge", False, taps, torch.float32)
+    ref = rec._backproject_stack(x, ang, center, 0, edge)
+    err = [_rel(rec._backproject_stack(x, ang, center, 1, edge), ref),
+           _rel(rec._backproject_matrix(x, ang, center, 1, edge), ref)]
+    print("float32 sums %.3g, matrix %.3g" % tuple(err))
+    assert err[1] <= err[0]
+
+
 def test_slice_bits_do_not_depend_on_the_stack():
     """A slice in either group of a pair, in a padded group or beside other
     slices keeps its bits, and so do mask and scale (zero outside the circle).
