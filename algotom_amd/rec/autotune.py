@@ -3,7 +3,8 @@
 A configuration is (slice_batch, tile_rows): slices per workgroup and image
 rows per 64-column tile.  Every configuration computes the same bits (the
 per-pixel arithmetic and angle order do not depend on tiling), so tuning
-only changes speed.
+only changes speed.  Stacks that fbp_reconstruction and bpf_reconstruction
+sum on the matrix cores have fixed tiles and take no configuration.
 
 Lookup order for a key (arch, kernel, mode, dtype, width bucket, stack
 bucket): the in-process table, the user cache (``$ALGOTOM_AMD_TUNE_CACHE`` or

@@ -44,7 +44,7 @@ class BatchFBP:
     filter_name, pad, pad_mode, apply_log, ratio, gpu :
         As in fbp_reconstruction, shared by the batch.
     precision : {None, "fp32", "fp16", "bf16"}
-        None keeps the reference arithmetic.
+        As in fbp_reconstruction.
     tile_rows : int or None
         Back-projection tile height; None takes the tuned value.
     dtypes : list of numpy dtypes or None

@@ -20,8 +20,8 @@ every compute entry raises ``RuntimeError``.
   every angle, but not its bits (``back_projection_gpu_chunk`` keeps them).
 * ``block`` and ``ncore`` are accepted and ignored: tiles are fixed by the
   kernel and there is no CPU worker pool.
-* keyword-only ``precision`` (not in the reference): ``None`` keeps the
-  reference arithmetic; ``"fp32"`` interpolates and accumulates in float32
+* keyword-only ``precision`` (not in the reference): ``None`` is the
+  arithmetic above; ``"fp32"`` interpolates and accumulates in float32
   (float64 detector positions); ``"fp16"`` / ``"bf16"`` also store the
   filtered sinogram in 16 bits.
 """
@@ -312,9 +312,9 @@ def _matrix_stack(nrow, nslice, ncol, acc, dtype):
       (more slices 1.0 to 1.1 up to 256 columns, 0.63 to 1.04 from 384 on),
       0.63 to 1.03 at 64 angles and 9 to 16; 640 and 768 columns 0.59 to 0.99
       at 17 to 32 slices, 0.9 to 1.5 at 9 to 16."""
-    import torch
-    if ncol > 32768 or nrow > 65535 or nslice > 65535:
+    if nslice <= 5 or ncol > 32768 or nrow > 65535 or nslice > 65535:
         return False
+    import torch
     if dtype in (torch.float16, torch.bfloat16):
         if acc != nat.ACC_F32 or nslice <= 8 or nrow < 64:
             return False
@@ -329,7 +329,7 @@ def _matrix_stack(nrow, nslice, ncol, acc, dtype):
     if dtype != torch.float32 or nrow < 128:
         return False
     if acc == nat.ACC_F32SEQ:
-        return nslice > 5
+        return True
     if acc == nat.ACC_F32:
         if ncol < 1000:
             return ncol >= 512 and nslice > (16 if ncol == 512 else 20)
@@ -588,7 +588,8 @@ def fbp_reconstruction(sinogram, center, angles=None, ratio=1.0,
     ncore : int or None
         Accepted for compatibility; ignored.
     precision : {None, "fp32", "fp16", "bf16"}, keyword only
-        None keeps the reference arithmetic.
+        None: the reference arithmetic that ``gpu`` selects, except for larger
+        stacks (see the module docstring).
 
     Returns
     -------
@@ -638,7 +639,7 @@ def _fbp(sinogram, center, angles=None, ratio=1.0, ramp_win=None,
     whole = volume_slices or num_sino
     acc = _accumulation(whole, gpu, precision)
     matrix = _matrix_stack(nrow, whole, ncol, acc, storage)
-    if not matrix:
+    if not matrix and whole != num_sino:
         acc = _accumulation(num_sino, gpu, precision)
     project = _backproject_matrix if matrix else _backproject_stack
 

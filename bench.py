@@ -12,7 +12,7 @@ U = 64 * 2560^2 * 1801 = 7.554e11 updates per step.
 
 roofline (bp_matrix_kernel, the dominant one): its products run on the matrix
 cores and their operands are built by the VALU, whose issue is the bound; its
-HBM traffic is 14 % of peak.
+HBM traffic is 13 % of peak.
 achieved = the kernel's VALU instructions per launch (SQ_INSTS_VALU, which
 counts the matrix instructions too, from the
 committed rocprofv3 counters of this kernel and workload,
@@ -923,7 +923,7 @@ def main():
         "config": {"workload": "fbp_stack_64x1801x2560", "nslice": NSLICE,
                    "nrow": NROW, "ncol": NCOL, "center": CENTER,
                    "apply_log": True, "filter": "hann", "pad": pad,
-                   "precision": args.precision or "reference",
+                   "precision": args.precision or "default",
                    "parallelism": "single-gpu"},
         "roofline": roof,
         "cpu_baseline": base,
