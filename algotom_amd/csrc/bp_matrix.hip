@@ -172,8 +172,8 @@ __device__ __forceinline__ int scale_exp(unsigned bits) {
     return 14 - ilogbf(__uint_as_float(bits));
 }
 
-// a scaled sample that is large for range_kernel
-constexpr float kLarge = 0.25f;
+// scaled samples that are large or huge for range_kernel
+constexpr float kLarge = 0.25f, kHuge = 8.0f;
 __host__ __device__ inline int span_count(int ncol) {
     return (ncol + kSpanCols - 1) / kSpanCols;
 }
@@ -236,14 +236,16 @@ __global__ __launch_bounds__(256) void slice_max_kernel(
 // block handles 128 columns of one angle's 16 slices through LDS, so both
 // the reads (columns) and the writes (slices) are contiguous.  Scaled samples
 // are counted on the way for range_kernel: spans[slice][span] = (angles in
-// which the span's samples are mostly small, angles in which they are all
-// zero); ordinary slices have few of either and add nothing.
+// which few of the span's samples are kLarge, those in which few are kHuge <<
+// 16, angles in which all are zero); ordinary slices have few of them and add
+// next to nothing.
 template <typename T, int PL, bool BATCH>
 __global__ __launch_bounds__(256) void split_kernel(
     const MatJob* __restrict__ jobs, int njobs, MatJob one) {
     constexpr int COLS = 128, SPANS = COLS / kSpanCols;
     __shared__ float tile[kGroup][COLS + 1];
-    __shared__ unsigned count[SPANS][kGroup];  // not zero, large << 16
+    // not zero, large << 8, huge << 16 (32 at most each)
+    __shared__ unsigned count[SPANS][kGroup];
     unsigned b;
     const MatJob& job = find_job<BATCH>(jobs, njobs, one, kSplit, b);
     const BpArgs& a = job.r.a;
@@ -279,9 +281,12 @@ __global__ __launch_bounds__(256) void split_kernel(
         s0 = ldexpf(s0, ex);
         s1 = ldexpf(s1, ex);
         if (scaled) {
-            const unsigned m = (s0 != 0.0f) + (s1 != 0.0f) +
-                               ((fabsf(s0) >= kLarge) << 16) +
-                               ((fabsf(s1) >= kLarge) << 16);
+            const auto rank = [](float v) {
+                const float u = fabsf(v);
+                return (unsigned)(u != 0.0f) + ((unsigned)(u >= kLarge) << 8) +
+                       ((unsigned)(u >= kHuge) << 16);
+            };
+            const unsigned m = rank(s0) + rank(s1);
             if (m) atomicAdd(&count[i / (kSpanCols / 2)][n], m);
         }
         const half2_t h = {(_Float16)s0, (_Float16)s1};
@@ -300,13 +305,14 @@ __global__ __launch_bounds__(256) void split_kernel(
     __syncthreads();
     const int sp = tid / kGroup;
     if (sp < SPANS && j < nslice && c0 + sp * kSpanCols < ncol) {
-        const unsigned m = count[sp][n], some = m & 0xffffu, large = m >> 16;
+        const unsigned m = count[sp][n];
+        const unsigned some = m & 255u, large = m >> 8 & 255u, huge = m >> 16;
         uint2* at = job.m.spans + (size_t)j * span_count(ncol) +
                     c0 / kSpanCols + sp;
         if (some == 0u)
             atomicAdd(&at->y, 1u);
-        else if (8u * large < some)
-            atomicAdd(&at->x, 1u);
+        else if (8u * huge < some)
+            atomicAdd(&at->x, 0x10000u + (8u * large < some ? 1u : 0u));
     }
 }
 
@@ -315,14 +321,17 @@ __global__ __launch_bounds__(256) void split_kernel(
 // sample of less than 2^-16 of it has 24 bits no more.  That is nothing to a
 // pixel that also sees larger ones (the sum's own rounding is coarser), but a
 // pixel whose samples are all small, beside a few that are huge (a hot pixel
-// or column), would lose its value.  A pixel at a distance d from the axis sees
-// the columns within d of the centre, so a slice is redone if for any d, in
-// steps of a span of 32 columns, more than half of the (span, angle) pairs in
-// there that are not all zero have fewer than one sample in 8 of kLarge =
-// 2^-2 or more (the maximum is scaled to 2^14 .. 2^15).  With half of them
-// large the rms of a pixel's samples is 2^-4 or more, and the floor's error,
-// 2^-26 sqrt(2 n / 3) for n angles, below that of a float32 sum after every
-// angle, 2^-29 n / sqrt(2), from 128 angles on.
+// or column), would lose its value.  The floor's error of a pixel, 2^-26
+// sqrt(2 n / 3) for n angles, stays below that of a float32 sum after every
+// angle, r 2^-25 n / sqrt(2), from 128 angles on if the rms of its samples is r
+// >= 2^-4 (with the maximum scaled to 2^14 .. 2^15).  A pixel at a distance d
+// from the axis sees the columns within d of the centre, so a slice stays if
+// for every d, in steps of a span of 32 columns, of the (span, angle) pairs in
+// there that are not all zero
+//   * half have one sample in 8 of kLarge = 2^-2 or more (r >= 2^-4), or
+//   * one in 16 has one sample in 8 of kHuge = 2^3 or more: an object in air
+//     whose edges fade out, which every pixel sees from 2 / (16 pi) of
+//     the angles at least (r >= 2^-1).
 template <bool BATCH>
 __global__ __launch_bounds__(256) void range_kernel(
     const MatJob* __restrict__ jobs, int njobs, MatJob one) {
@@ -333,18 +342,18 @@ __global__ __launch_bounds__(256) void range_kernel(
     const double center = job.r.a.center;
     const uint2* sp = job.m.spans + (size_t)j * ns;
     bool any = false;
-    for (int k = threadIdx.x; k < ns; k += 256) any |= sp[k].x != 0u;
+    for (int k = threadIdx.x; k < ns; k += 256) any |= (sp[k].x & 0xffffu) != 0u;
     if (!__syncthreads_or(any)) return;
     const int mid = (int)fmin(fmax(center / kSpanCols, 0.0), ns - 1.0);
     bool redo = false;
     for (int d = threadIdx.x; d < ns; d += 256) {
-        unsigned long long low = 0, zero = 0, all = 0;
+        unsigned long long low = 0, faint = 0, some = 0;
         for (int k = max(mid - d, 0); k <= min(mid + d, ns - 1); ++k) {
-            low += sp[k].x;
-            zero += sp[k].y;
-            all += (unsigned)nrow;
+            low += sp[k].x & 0xffffu;
+            faint += sp[k].x >> 16;
+            some += (unsigned)nrow - sp[k].y;
         }
-        redo |= 2 * low > all - zero;
+        redo |= 2 * low > some && 16 * (some - faint) < some;
     }
     if (__syncthreads_or(redo) && threadIdx.x == 0) job.m.smax[j] = kRedo;
 }

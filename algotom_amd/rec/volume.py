@@ -54,10 +54,12 @@ def reconstruct_volume_360(sino_360, cor, chunk=16, angles=None, ratio=1.0,
                         apply_log=apply_log, precision=precision,
                         volume_slices=nslice)
 
-    if rec._matrix_stack(n180, nslice, width,
-                         rec._accumulation(nslice, True, precision),
-                         rec._storage_dtype(precision)):
+    # (a chunk that range() refuses, or that leaves nothing to do, stays so)
+    if len(range(0, nslice, chunk)) and rec._matrix_stack(
+            n180, nslice, width, rec._accumulation(nslice, True, precision),
+            rec._storage_dtype(precision)):
         chunk = rec._matrix_chunk(chunk, 4 * (nrow * ncol + width * width))
+
     ranges = [(j0, min(nslice, j0 + chunk)) for j0 in range(0, nslice, chunk)]
     if out is not None and not rec._is_tensor(out) \
             and not rec._is_tensor(sino_360):

@@ -182,10 +182,10 @@ int ath_back_projection(const void* sino, int sino_dtype, int nrow,
  * on its error against float64 is below that of ATH_ACC_F32SEQ.  A slice's
  * result does not depend on the other slices of the stack.  sino_dtype: ATH_F32
  * (acc ATH_ACC_F32SEQ or ATH_ACC_F32), ATH_F16 or ATH_BF16 (acc ATH_ACC_F32).
- * A slice with a non-finite or > 2^100 sample, or (not ATH_F16) one where the
- * samples within some distance of the centre's column mostly lie below 2^-16
- * of the slice's largest, is computed with acc exactly as ath_back_projection
- * does.  workspace: device memory of at least
+ * A slice with a non-finite or > 2^100 sample, or (not ATH_F16) one where
+ * nearly all samples within some distance of the centre's column lie below
+ * 2^-12 of the slice's largest and most of them below 2^-16, is computed with
+ * acc exactly as ath_back_projection does.  workspace: device memory of at least
  * ath_back_projection_matrix_workspace_bytes(...) (0: unsupported), 16-byte
  * aligned; ATH_ERR_WORKSPACE when too small. */
 size_t ath_back_projection_matrix_workspace_bytes(int sino_dtype, int nrow,

@@ -240,7 +240,8 @@ def test_ordinary_samples_beside_huge_ones(kind, dtype):
 
 
 @pytest.mark.parametrize("nrow", [128, 400])
-@pytest.mark.parametrize("data", ["noise", "2 orders of columns", "tails"])
+@pytest.mark.parametrize("data", ["noise", "2 orders of columns", "tails",
+                                  "object in air"])
 def test_small_samples_that_are_kept(nrow, data):
     """Slices with a large range that stay on the matrix cores: the error in
     every ring of pixels is at most that of a float32 sum after every angle
@@ -254,8 +255,10 @@ def test_small_samples_that_are_kept(nrow, data):
         x[5, :, 3] = 2.0 ** 13      # an outlier within the range
     elif data == "2 orders of columns":
         x = x * torch.where(col.abs() < 40, 1.0, 100.0)
-    else:                           # a narrow object's filtered tails
+    elif data == "tails":           # a narrow object's filtered tails
         x = x * torch.exp2(-(col.abs() / 6))
+    else:                           # a blurred one, air down to 2^-32 of it
+        x = x.abs() * torch.exp2(-((col.abs() - 12).clamp(min=0) / 2))
     x = x.contiguous()
     ref = rec._backproject_stack(x, ang, cen, 0, True)
     seq = rec._backproject_stack(x, ang, cen, 1, True)

@@ -132,6 +132,8 @@ def test_volume_360_does_not_depend_on_its_chunks(precision):
     for chunk in (1, 3, 16, 20, 64):
         got, _ = volume.reconstruct_volume_360(sino, 29.5, chunk=chunk, **kw)
         assert np.array_equal(got.cpu().numpy(), want.cpu().numpy()), chunk
+    with pytest.raises(ValueError):
+        volume.reconstruct_volume_360(sino, 29.5, chunk=0, **kw)
 
 
 @pytest.mark.parametrize("rows,stage", [(37, 1 << 16), (5, 1 << 12)])
