@@ -464,12 +464,11 @@ __device__ __forceinline__ void matrix_tile(const BpArgs& a, const MatArgs& ma,
         const double yb = to_scalar((double)yw + 1.5 - ic);
 
         auto trig = [&](int a0) { return ma.trig[min(a0 + k4, N - 1)]; };
-        // the tile's centre
-        const double xm = to_scalar((double)x0 + 0.5 * (TL::X - 1) - ic);
-        const double ym = (double)y0 + 0.5 * (TL::Y - 1) - ic;
         // lanes 0, 16, 32, 48 of one wave: the angles of the step at a0
         auto geometry = [&](int a0, float2 tf, unsigned slot) {
             const double2 t = make_double2((double)tf.x, (double)tf.y);
+            const double xm = (double)x0 + 0.5 * (TL::X - 1) - ic;
+            const double ym = (double)y0 + 0.5 * (TL::Y - 1) - ic;
             const double fm = det_pos(xm * t.x, ym, t.y, cen);
             const double ext = fma(0.5 * (TL::Y - 1), fabs(t.y),
                                    0.5 * (TL::X - 1) * fabs(t.x));
@@ -692,13 +691,18 @@ __device__ __forceinline__ void matrix_tile(const BpArgs& a, const MatArgs& ma,
                 // or more past L, so the clamps change none)
                 const double q_end = kWinMagic - (w1 - l + 0.5 * kSlack);
                 const bool valid = g->valid;
+                // (16 bits: opaque, so that the columns' coordinates are not
+                // kept in registers across the angle loop; in float32 the
+                // copies would spill)
+                double xo = xl, yo = yl;
+                if constexpr (PL == 1) asm volatile("" : "+v"(xo), "+v"(yo));
 #pragma unroll
                 for (int i = 0; i < BX; ++i) {
                     const double m = (double)(xw - xg + 4 * i);
                     const double q = fmin(fmax(fma(-m, c, bn), q_end),
                                           kWinMagic - 0.5 * kSlack);
                     e[i] = (unsigned)__double2loint(q) >> 25;
-                    const double f = det_pos((xl + m) * c, yl, s, cen);
+                    const double f = det_pos((xo + m) * c, yo, s, cen);
                     const bool in = f >= 0.0 && f <= w1;
                     const double edge = clamp_pos(f, w1) - l + kPosMagic;
                     p[i] = (unsigned)__double2loint(in ? fma(m, c, fr) : edge);
