@@ -252,11 +252,13 @@ __global__ __launch_bounds__(256) void split_kernel(
     const int nrow = a.nrow, nslice = a.nslice, ncol = a.ncol;
     const int npair = job.m.npair, scaled = job.m.scaled;
     const T* sino = static_cast<const T*>(a.sino);
+    // one stack: grid.y is the row (its workgroups can be more than 2^24)
     const unsigned nblock = (ncol + COLS - 1) / COLS;
     const int c0 = (int)(b % nblock) * COLS;
     b /= nblock;
-    const int row = (int)(b % nrow);
-    const int gl = (int)(b / nrow), g = job.m.group_op + gl;
+    const int row = BATCH ? (int)(b % nrow) : (int)blockIdx.y;
+    const int gl = BATCH ? (int)(b / nrow) : (int)b;
+    const int g = job.m.group_op + gl;
     const int tid = threadIdx.x;
     for (int e = tid; e < kGroup * COLS; e += 256) {
         const int n = e / COLS, c = c0 + e % COLS, j = g * kGroup + n;
@@ -826,6 +828,9 @@ __global__ __launch_bounds__(kThreads) void bp_matrix_kernel(
     matrix_tile<PL, SG>(a, ma, tx, ty, grp);
 }
 
+// workgroups of 256 threads in a grid's x: its work items are a 32-bit number
+constexpr long long kMaxBlocks = (1LL << 24) - 1;
+
 template <int SG> constexpr size_t matrix_lds() {
     return (size_t)(2 * kStep * Tile<SG>::rows * SG * kGroup + 8) *
                sizeof(uint4_t) +
@@ -835,7 +840,7 @@ template <int SG> constexpr size_t matrix_lds() {
 template <int PL, int SG, bool BATCH>
 int launch_kernel(const MatJob* jobs, int njobs, const MatJob& one,
                   long long blocks, hipStream_t stream) {
-    if (blocks > 0x7fffffffLL)
+    if (blocks > kMaxBlocks / 4)
         return set_error(ATH_ERR_UNSUPPORTED, "back-projection grid too large");
     auto kern = bp_matrix_kernel<PL, SG, BATCH>;
     const int st = allow_dynamic_lds(reinterpret_cast<const void*>(kern),
@@ -915,6 +920,7 @@ size_t set_job(MatJob& job, const BpArgs& a, int dtype, int part, char* work) {
     return op_at + (m.nop + m.ntail) * sizeof(unsigned);
 }
 
+int split_block_columns(const MatJob& j) { return (j.r.a.ncol + 127) / 128; }
 long long clear_blocks(const MatJob& j) {
     return ((long long)std::max({j.r.a.nrow, j.m.nzero, j.m.ntail}) + 255) /
            256;
@@ -923,18 +929,18 @@ long long max_blocks(const MatJob& j) {
     return (long long)j.r.a.nslice * j.m.max_rows;
 }
 long long split_blocks(const MatJob& j, int groups) {
-    return (long long)((j.r.a.ncol + 127) / 128) * j.r.a.nrow * groups;
+    return (long long)split_block_columns(j) * j.r.a.nrow * groups;
 }
 
-#define ATH_MATRIX_LAUNCH(KERNEL, BLOCKS, JOBS, NJOBS, ONE)                   \
+#define ATH_MATRIX_LAUNCH(KERNEL, BLOCKS, ROWS, JOBS, NJOBS, ONE)             \
     do {                                                                      \
         const long long n_ = (BLOCKS);                                        \
-        if (n_ > 0x7fffffffLL)                                                \
+        if (n_ > kMaxBlocks)                                                  \
             return set_error(ATH_ERR_UNSUPPORTED,                             \
                              "back-projection grid too large");               \
         if (n_ > 0) {                                                         \
-            hipLaunchKernelGGL((KERNEL), dim3((unsigned)n_), dim3(256), 0, s, \
-                               JOBS, NJOBS, ONE);                             \
+            hipLaunchKernelGGL((KERNEL), dim3((unsigned)n_, ROWS), dim3(256), \
+                               0, s, JOBS, NJOBS, ONE);                       \
             const int st_ = check_hip(hipGetLastError(), #KERNEL " launch");  \
             if (st_ != ATH_OK) return st_;                                    \
         }                                                                     \
@@ -948,19 +954,20 @@ int run_matrix(const BpArgs& a, int dtype, int acc, char* work,
     MatJob job;
     set_job(job, a, dtype, part, work);
     const MatJob* none = nullptr;
-    ATH_MATRIX_LAUNCH(clear_kernel<false>, clear_blocks(job), none, 0, job);
-    ATH_MATRIX_LAUNCH((slice_max_kernel<T, false>), max_blocks(job), none, 0,
-                      job);
+    ATH_MATRIX_LAUNCH(clear_kernel<false>, clear_blocks(job), 1, none, 0, job);
+    ATH_MATRIX_LAUNCH((slice_max_kernel<T, false>), max_blocks(job), 1, none,
+                      0, job);
     for (int g0 = 0; g0 < groups; g0 += part) {
         const int n = std::min(part, groups - g0);
         job.m.group0 = job.m.group_op = g0;
         job.m.group_have = g0 + n;
-        ATH_MATRIX_LAUNCH((split_kernel<T, PL, false>), split_blocks(job, n),
+        ATH_MATRIX_LAUNCH((split_kernel<T, PL, false>),
+                          (long long)split_block_columns(job) * n, a.nrow,
                           none, 0, job);
         if (job.m.scaled)
             ATH_MATRIX_LAUNCH(range_kernel<false>,
                               std::min(n * kGroup, a.nslice - g0 * kGroup),
-                              none, 0, job);
+                              1, none, 0, job);
         // Pairs of groups; a last odd group by itself unless an idle one
         // beside it is cheaper, which it is where the launch does not fill the
         // chip twice (rounds of 256 workgroups, at the measured 0.69 against
@@ -1002,13 +1009,14 @@ template <typename T, int PL>
 int run_batch(const MatPlan& p, const MatJob* jobs, hipStream_t s) {
     const MatJob one{};
     const unsigned* n = p.blocks;
-    ATH_MATRIX_LAUNCH(clear_kernel<true>, n[kClear], jobs, p.njobs, one);
-    ATH_MATRIX_LAUNCH((slice_max_kernel<T, true>), n[kMaxima], jobs, p.njobs,
-                      one);
-    ATH_MATRIX_LAUNCH((split_kernel<T, PL, true>), n[kSplit], jobs, p.njobs,
+    ATH_MATRIX_LAUNCH(clear_kernel<true>, n[kClear], 1, jobs, p.njobs, one);
+    ATH_MATRIX_LAUNCH((slice_max_kernel<T, true>), n[kMaxima], 1, jobs,
+                      p.njobs, one);
+    ATH_MATRIX_LAUNCH((split_kernel<T, PL, true>), n[kSplit], 1, jobs, p.njobs,
                       one);
     if (p.dtype != ATH_F16)
-        ATH_MATRIX_LAUNCH(range_kernel<true>, n[kRange], jobs, p.njobs, one);
+        ATH_MATRIX_LAUNCH(range_kernel<true>, n[kRange], 1, jobs, p.njobs,
+                          one);
     int st = ATH_OK;
     if (n[kPairs])
         st = launch_kernel<PL, 2, true>(jobs, p.njobs, one, n[kPairs], s);
@@ -1110,9 +1118,10 @@ int matrix_batch_add(void* plan, const BpArgs& a, void* work) {
     const long long redo = redo_tiles(a.nslice, a.ncol);
     const char* large = "matrix back-projection: batch too large";
     for (int k = 0; k < kStages; ++k)
-        if (p.blocks[k] + n[k] > 0x7fffffffLL)
+        if (p.blocks[k] + n[k] >
+            (k == kPairs || k == kSingle ? kMaxBlocks / 4 : kMaxBlocks))
             return set_error(ATH_ERR_UNSUPPORTED, large);
-    if (p.redo_blocks + redo > 0x7fffffffLL)
+    if (p.redo_blocks + redo > kMaxBlocks)
         return set_error(ATH_ERR_UNSUPPORTED, large);
     for (int k = 0; k < kStages; ++k) {
         j.begin[k] = p.blocks[k];

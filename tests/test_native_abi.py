@@ -119,6 +119,43 @@ def test_invalid_filter_arguments():
     assert st == nat.ATH_ERR_INVALID_ARG  # nwin neither 1 nor nrow
 
 
+def test_matrix_batch_plan_sizes_and_refusals():
+    # host work only: the plan is written without a device
+    lib = nat.load()
+    jobs = (nat.BpJob * 3)(*[
+        nat.BpJob(16, 16, 16, nrow, nslice, ncol, ncol / 2.0, -1.0, 1, 0, 0)
+        for nrow, nslice, ncol in ((131, 6, 90), (260, 17, 130), (200, 33, 65))])
+    ref = ctypes.byref(jobs)
+    work = lib.ath_matrix_batch_workspace_bytes(ref, 3, nat.ATH_F32)
+    one = [lib.ath_back_projection_matrix_workspace_bytes(
+        nat.ATH_F32, j.nrow, j.nslice, j.ncol) for j in jobs]
+    assert sum(one) <= work <= sum(one) + 3 * 256
+    size = lib.ath_matrix_batch_plan_bytes(3)
+    plan = np.zeros(size // 8 + 1, dtype=np.uint64)
+
+    def make(jobs_=ref, n=3, dtype=nat.ATH_F32, acc=nat.ACC_F32SEQ, at=256,
+             nwork=work, to=plan.ctypes.data, nplan=size):
+        return lib.ath_matrix_batch_plan(jobs_, n, dtype, acc, at, nwork, to,
+                                         nplan)
+
+    assert make() == nat.ATH_OK
+    assert make(dtype=nat.ATH_F16, acc=nat.ACC_F32) == nat.ATH_OK
+    assert make(nwork=work - 1) == nat.ATH_ERR_WORKSPACE
+    assert make(dtype=nat.ATH_F64) == nat.ATH_ERR_UNSUPPORTED
+    assert make(dtype=nat.ATH_F16) == nat.ATH_ERR_UNSUPPORTED
+    for bad in (dict(jobs_=None), dict(n=0), dict(at=None), dict(at=264),
+                dict(to=None), dict(nplan=size - 1), dict(acc=nat.ACC_F64)):
+        assert make(**bad) == nat.ATH_ERR_INVALID_ARG, bad
+    jobs[1].nrow = 1                    # the scale needs two angles
+    assert make() == nat.ATH_ERR_INVALID_ARG
+    jobs[1].nrow, jobs[2].ncol = 260, 32769
+    assert lib.ath_matrix_batch_workspace_bytes(ref, 3, nat.ATH_F32) == 0
+    assert make() == nat.ATH_ERR_UNSUPPORTED
+    assert lib.ath_matrix_batch_plan_bytes(0) == 0
+    assert lib.ath_back_projection_matrix_batched(
+        None, None, None) == nat.ATH_ERR_INVALID_ARG
+
+
 def test_forward_projection_ws_rejects_small_workspace():
     # the size check comes before any device work
     lib = nat.load()
