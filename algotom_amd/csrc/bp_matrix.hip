@@ -42,7 +42,7 @@
 //
 // Measured (64 x 1801 x 2560, with the mask): float32 42 ms against 181 ms
 // for ATH_ACC_F32SEQ (17.9 against 4.2 updates per ps), float16 31
-// against 75 ms; 16 slices 15.8 against 46 ms.  What bounds it is VALU issue,
+// against 75 ms; 16 slices 14.9 against 46 ms.  What bounds it is VALU issue,
 // 41 instructions per block and four angles of 32 slices (76 % busy with the
 // matrix unit 41 %; simple 32-bit instructions take 1.2 ns per wave here,
 // permutes, shift-adds and float64 2.0, a matrix instruction 7.4 of which it
